@@ -1900,12 +1900,36 @@ int lpa_cglp_csr_get(lpa_engine *e, uint64_t *row, uint32_t *col, uint64_t *m) {
 struct lpa_mlp {
     int device = 0;
     hipStream_t stream = nullptr;
-    DevBuf<float> params, grad, m1, m2, loss;
+    // parameters, first and second moments (MLP_STRIDE floats each), double
+    // buffered: a training step reads state[cur] and writes the other one
+    DevBuf<float> state[2], part[2], grad;
+    DevBuf<double> loss;
+    int cur = 0;
     int t = 0;
     ~lpa_mlp() {
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
+
+// Workgroups (and partials) of a step over n samples: 64 samples each, up to
+// a limit, beyond which a workgroup takes more.  In training every workgroup
+// reads all partials of the batch before (5.8 KB each), so their number is
+// kept at 64; a single gradient spreads over the device.
+constexpr uint32_t MLP_PARTS_TRAIN = 64, MLP_PARTS_MAX = 256;
+static uint32_t mlp_parts(uint64_t n, uint32_t most) {
+    const uint64_t per = MLP_WAVES * MLP_TILE;
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + per - 1) / per, most));
+}
+
+// k_mlp_step over the model's state; with an update pending (np > 0) the
+// other state buffer becomes the current one.
+static void launch_mlp_step(lpa_mlp *m, const float *part_in, uint32_t np, const AdamArgs &adam, double *loss,
+                            const float *x, const float *target, const uint8_t *mask, const uint32_t *idx, uint64_t n,
+                            float scale, float *part_out, uint32_t parts) {
+    hipLaunchKernelGGL(k_mlp_step, dim3(parts), dim3(64 * MLP_WAVES), 0, m->stream, m->state[m->cur].p,
+                       m->state[m->cur ^ 1].p, part_in, np, adam, loss, x, target, mask, idx, n, scale, part_out);
+    if (np) m->cur ^= 1;
+}
 
 static int family_of(int kind) {
     switch (kind) {
@@ -2054,13 +2078,12 @@ int lpa_mlp_create(int device, uint64_t seed, lpa_mlp **out) {
             for (int i = 0; i < MLP_H * MLP_IN; i++) p[MLP_W1 + i] = (float)(normal() * std::sqrt(2.0 / MLP_IN));
             for (int i = 0; i < MLP_H * MLP_H; i++) p[MLP_W2 + i] = (float)(normal() * std::sqrt(2.0 / MLP_H));
             for (int i = 0; i < MLP_OUT * MLP_H; i++) p[MLP_W3 + i] = (float)(normal() * std::sqrt(2.0 / MLP_H));
-            m->params.upload(p.data(), MLP_NPARAM, m->stream);
-            m->grad.alloc(MLP_NPARAM);
-            m->m1.alloc(MLP_NPARAM);
-            m->m2.alloc(MLP_NPARAM);
-            m->loss.alloc(1);
-            HIPCHK(hipMemsetAsync(m->m1.p, 0, MLP_NPARAM * 4, m->stream));
-            HIPCHK(hipMemsetAsync(m->m2.p, 0, MLP_NPARAM * 4, m->stream));
+            p.resize(3 * MLP_STRIDE, 0.0f);   // zero moments
+            for (int i = 0; i < 2; i++) {
+                m->state[i].upload(p.data(), p.size(), m->stream);
+                m->part[i].alloc((uint64_t)MLP_PARTS_MAX * MLP_STRIDE);
+            }
+            m->grad.alloc(MLP_STRIDE);
             HIPCHK(hipStreamSynchronize(m->stream));
         } catch (...) {
             delete m;
@@ -2082,7 +2105,7 @@ int lpa_mlp_get_params(lpa_mlp *m, float *params) {
     return guard([&] {
         if (!m || !params) throw Fail(LPA_ERR_ARG, "null argument");
         HIPCHK(hipSetDevice(m->device));
-        HIPCHK(hipMemcpy(params, m->params.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(params, m->state[m->cur].p, MLP_NPARAM * 4, hipMemcpyDeviceToHost));
     });
 }
 
@@ -2090,10 +2113,10 @@ int lpa_mlp_set_params(lpa_mlp *m, const float *params) {
     return guard([&] {
         if (!m || !params) throw Fail(LPA_ERR_ARG, "null argument");
         HIPCHK(hipSetDevice(m->device));
-        HIPCHK(hipMemcpy(m->params.p, params, MLP_NPARAM * 4, hipMemcpyHostToDevice));
+        float h[3 * MLP_STRIDE] = {};   // zero moments
+        std::memcpy(h, params, MLP_NPARAM * 4);
+        HIPCHK(hipMemcpy(m->state[m->cur].p, h, sizeof h, hipMemcpyHostToDevice));
         m->t = 0;
-        HIPCHK(hipMemset(m->m1.p, 0, MLP_NPARAM * 4));
-        HIPCHK(hipMemset(m->m2.p, 0, MLP_NPARAM * 4));
     });
 }
 
@@ -2106,7 +2129,7 @@ int lpa_mlp_forward(lpa_mlp *m, const float *x, uint64_t n, float *y) {
         dx.upload(x, n * MLP_IN, m->stream);
         dy.alloc(n * MLP_OUT);
         hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream,
-                           m->params.p, dx.p, dy.p, n);
+                           m->state[m->cur].p, dx.p, dy.p, n);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(y, dy.p, n * MLP_OUT * 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));
@@ -2123,13 +2146,12 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
         dx.upload(x, n * MLP_IN, m->stream);
         dt.upload(target, n * MLP_OUT, m->stream);
         dm.upload(mask, n * MLP_OUT, m->stream);
-        hipLaunchKernelGGL(k_zero_f32, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->grad.p, MLP_NPARAM);
-        hipLaunchKernelGGL(k_zero_f32, dim3(1), dim3(64), 0, m->stream, m->loss.p, 1);
-        hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, m->params.p,
-                           dx.p, dt.p, dm.p, (const uint32_t *)nullptr, n, 1.0f / (float)n, m->grad.p, m->loss.p);
+        const uint32_t np = mlp_parts(n, MLP_PARTS_MAX);
+        launch_mlp_step(m, nullptr, 0, AdamArgs{}, nullptr, dx.p, dt.p, dm.p, nullptr, n, 1.0f / (float)n, m->part[0].p, np);
+        hipLaunchKernelGGL(k_mlp_sum, dim3((MLP_STRIDE / 4 + 63) / 64), dim3(64), 0, m->stream, m->part[0].p, np, m->grad.p);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(grad, m->grad.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipMemcpyAsync(loss, m->loss.p, 4, hipMemcpyDeviceToHost, m->stream));
+        HIPCHK(hipMemcpyAsync(loss, m->grad.p + MLP_NPARAM, 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));
     });
 }
@@ -2151,30 +2173,42 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
         std::iota(idx.begin(), idx.end(), 0u);
         uint64_t s = seed;
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+        m->loss.alloc(epochs);
+        HIPCHK(hipMemsetAsync(m->loss.p, 0, (uint64_t)epochs * sizeof(double), m->stream));
+        // a batch's update is applied by the next step (the last one's by a
+        // step without samples); np partials of it are pending
+        uint32_t np = 0;
+        AdamArgs adam{lr, b1, b2, eps, 0, 0};
+        double *pending_loss = nullptr;
+        int pb = 0;
+        uint64_t nb = 0;
         for (int ep = 0; ep < epochs; ep++) {
             for (uint64_t i = n - 1; i > 0; i--) std::swap(idx[i], idx[splitmix64(s) % (i + 1)]);
             HIPCHK(hipMemcpyAsync(didx.p, idx.data(), n * 4, hipMemcpyHostToDevice, m->stream));
-            hipLaunchKernelGGL(k_zero_f32, dim3(1), dim3(64), 0, m->stream, m->loss.p, 1);
-            int nb = 0;
+            // idx is shuffled again while this epoch's steps run
+            HIPCHK(hipStreamSynchronize(m->stream));
+            nb = 0;
             for (uint64_t b0 = 0; b0 < n; b0 += (uint64_t)batch, nb++) {
                 const uint64_t bn = std::min<uint64_t>(batch, n - b0);
-                hipLaunchKernelGGL(k_zero_f32, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->grad.p,
-                                   MLP_NPARAM);
-                hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)((bn + 255) / 256)), dim3(256), 0, m->stream,
-                                   m->params.p, dx.p, dt.p, dm.p, didx.p + b0, bn, 1.0f / (float)bn, m->grad.p,
-                                   m->loss.p);
+                const uint32_t parts = mlp_parts(bn, MLP_PARTS_TRAIN);
+                launch_mlp_step(m, m->part[pb].p, np, adam, pending_loss, dx.p, dt.p, dm.p, didx.p + b0, bn,
+                                1.0f / (float)bn, m->part[pb ^ 1].p, parts);
                 m->t++;
-                const float c1 = (float)(1.0 / (1.0 - std::pow((double)b1, m->t)));
-                const float c2 = (float)(1.0 / (1.0 - std::pow((double)b2, m->t)));
-                hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->params.p,
-                                   m->grad.p, m->m1.p, m->m2.p, lr, b1, b2, eps, c1, c2);
+                adam.c1 = (float)(1.0 / (1.0 - std::pow((double)b1, m->t)));
+                adam.c2 = (float)(1.0 / (1.0 - std::pow((double)b2, m->t)));
+                np = parts;
+                pending_loss = m->loss.p + ep;
+                pb ^= 1;
             }
             HIPCHK(hipGetLastError());
-            float l = 0;
-            HIPCHK(hipMemcpyAsync(&l, m->loss.p, 4, hipMemcpyDeviceToHost, m->stream));
-            HIPCHK(hipStreamSynchronize(m->stream));
-            if (loss_per_epoch) loss_per_epoch[ep] = l / (float)nb;
         }
+        launch_mlp_step(m, m->part[pb].p, np, adam, pending_loss, dx.p, dt.p, dm.p, nullptr, 0, 0.0f, nullptr, 1);
+        HIPCHK(hipGetLastError());
+        std::vector<double> l(epochs);
+        HIPCHK(hipMemcpyAsync(l.data(), m->loss.p, l.size() * sizeof(double), hipMemcpyDeviceToHost, m->stream));
+        HIPCHK(hipStreamSynchronize(m->stream));
+        if (loss_per_epoch)
+            for (int ep = 0; ep < epochs; ep++) loss_per_epoch[ep] = (float)(l[ep] / (double)nb);
     });
 }
 
