@@ -1,10 +1,10 @@
 // encode_long.hpp -- CGR records of long rows, encoded by a whole workgroup.
 //
-// k_encode_len / k_encode_write give a record to one lane, which walks its
-// row several times; a hub of millions of ids keeps that lane busy for
-// seconds while the rest of the device idles.  Rows longer than LONG_ROW
-// are left to the kernels here, one 1024-lane workgroup per row, which
-// produce the same bits in data-parallel phases:
+// A wave that encodes a row (encode_wave.hpp) streams over it 64 ids at a
+// time; a hub of millions of ids would keep it busy long after the rest of
+// the device is done.  Rows longer than LONG_ROW are left to the kernels
+// here, one 1024-lane workgroup per row, which produce the same bits in
+// data-parallel phases:
 //
 //  1. runs: id i opens a maximal run of consecutive ids when adj[i-1] + 1 !=
 //     adj[i]; along a sorted row adj[j] - j never decreases, so the run ends
@@ -33,7 +33,7 @@ namespace lpa {
 
 namespace enc {
 
-constexpr uint32_t LONG_ROW = 1u << 16;   // rows longer than this take the workgroup kernels
+constexpr uint32_t LONG_ROW = 1u << 13;   // rows longer than this take the workgroup kernels
 constexpr uint32_t LONG_LANES = 1024;
 
 // Last index j >= s of the run of consecutive ids containing adj[s] (adj

@@ -27,6 +27,7 @@
 #include "bfs_relabel.hpp"
 #include "encode_kernels.hpp"
 #include "encode_long.hpp"
+#include "encode_wave.hpp"
 #include "heavy_kernels.hpp"
 #include "mlp_kernels.hpp"
 #include "lp_kernels.hpp"
@@ -705,7 +706,7 @@ static void finish_graph(lpa_engine *e) {
     e->counter.alloc(1);
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
     if (n_c)
-        hipLaunchKernelGGL(k_scan_records, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, e->stream, e->words0.p,
+        hipLaunchKernelGGL(k_scan_records, dim3((unsigned)((n_c * SCAN_G + 255) / 256)), dim3(256), 0, e->stream, e->words0.p,
                            e->offs0.p, e->vid0.p, n_c, (uint32_t)e->n, ddeg.p, e->feat0.p, e->meta0.p, e->counter.p);
     HIPCHK(hipGetLastError());
     unsigned long long bad = 0;
@@ -717,6 +718,26 @@ static void finish_graph(lpa_engine *e) {
     e->m_c = 0;
     for (uint32_t d : e->deg_c) e->m_c += d;
     e->have_graph = true;
+}
+
+// The encoder's two passes over rows of at most long_min ids (longer ones
+// take a workgroup each, encode_long.hpp): a lane per short row, a wave per
+// longer one.
+static void launch_encode_len(hipStream_t s, const uint64_t *row, const uint32_t *col, const uint32_t *vid,
+                              uint64_t n_c, uint64_t n, uint64_t *len, unsigned long long *err, uint32_t long_min) {
+    if (n_c == 0) return;
+    hipLaunchKernelGGL(k_encode_len, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, s, row, col, vid, n_c,
+                       (uint32_t)n, len, err, enc::LANE_ROW);
+    hipLaunchKernelGGL(k_encode_wave_len, dim3((unsigned)((n_c + enc::ENC_WAVES - 1) / enc::ENC_WAVES)),
+                       dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, n_c, (uint32_t)n, len, err, long_min);
+}
+static void launch_encode_write(hipStream_t s, const uint64_t *row, const uint32_t *col, const uint32_t *vid,
+                                uint64_t n_c, const uint64_t *offs, uint64_t *words, uint32_t long_min) {
+    if (n_c == 0) return;
+    hipLaunchKernelGGL(k_encode_write, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, s, row, col, vid, n_c, offs,
+                       words, enc::LANE_ROW);
+    hipLaunchKernelGGL(k_encode_wave_write, dim3((unsigned)((n_c + enc::ENC_WAVES - 1) / enc::ENC_WAVES)),
+                       dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, n_c, offs, words, long_min);
 }
 
 // ------------------------------------------------------------------ C ABI
@@ -909,9 +930,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         e->offs0.alloc(n_c + 1);
         e->counter.alloc(1);
         hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
-        if (n_c)
-            hipLaunchKernelGGL(k_encode_len, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, e->stream, drow.p,
-                               dcol.p, e->vid0.p, n_c, (uint32_t)n, len.p, e->counter.p, enc::LONG_ROW);
+        launch_encode_len(e->stream, drow.p, dcol.p, e->vid0.p, n_c, n, len.p, e->counter.p, enc::LONG_ROW);
         // rows longer than LONG_ROW: one workgroup each, with scratch of
         // d + 1 entries per row for every per-entry array (44 bytes each),
         // in groups of rows whose scratch stays within 2^28 entries
@@ -979,9 +998,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         e->words0.alloc(n64);
         hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((n64 + 255) / 256)), dim3(256), 0, e->stream,
                            (unsigned long long *)e->words0.p, n64, 0ull);
-        if (n_c)
-            hipLaunchKernelGGL(k_encode_write, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, e->stream, drow.p,
-                               dcol.p, e->vid0.p, n_c, e->offs0.p, e->words0.p, enc::LONG_ROW);
+        launch_encode_write(e->stream, drow.p, dcol.p, e->vid0.p, n_c, e->offs0.p, e->words0.p, enc::LONG_ROW);
         for (const auto &G : lgroups) {
             // one group: its scratch is still in place; several: each is
             // measured again before it is written (the same lengths result)
@@ -1018,8 +1035,7 @@ int lpa_encode_csr_device(lpa_engine *e, uint64_t n, uint64_t n_c, const uint64_
             return;
         }
         // record lengths into offsets[0..n_c), then an in-place exclusive scan
-        hipLaunchKernelGGL(k_encode_len, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, e->stream, row, col, vid,
-                           n_c, (uint32_t)n, offsets, (unsigned long long *)scr, UINT32_MAX);
+        launch_encode_len(e->stream, row, col, vid, n_c, n, offsets, (unsigned long long *)scr, UINT32_MAX);
         const uint64_t nb = (n_c + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK;
         hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(256), 0, e->stream, offsets, n_c, scr + 1);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, e->stream, scr + 1, nb);
@@ -1041,8 +1057,7 @@ int lpa_encode_csr_device(lpa_engine *e, uint64_t n, uint64_t n_c, const uint64_
         if (nw)
             hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, e->stream,
                                (unsigned long long *)words, nw, 0ull);
-        hipLaunchKernelGGL(k_encode_write, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, e->stream, row, col, vid,
-                           n_c, offsets, words, UINT32_MAX);
+        launch_encode_write(e->stream, row, col, vid, n_c, offsets, words, UINT32_MAX);
         HIPCHK(hipGetLastError());
         e->sync();
         *nbits = total;
