@@ -98,6 +98,93 @@ struct BitReader {
     }
 };
 
+// Reader over a range of the stream staged as 32-bit words in LDS (stream
+// order, MSB first; word k of the range at w[k + 2], so that every position
+// has a word before it).  q = bit position in the range + 63: with s = (q & 31)
+// + 1 bits of w[q >> 5] consumed, the 32 bits at the position are one funnel
+// shift of two words, for any alignment.  Nearly every code is at most 32
+// bits long (gamma below 2^16 - 1, zeta_3 below 2^24 - 1) and costs a dozen
+// 32-bit instructions and one LDS read; longer ones take a third word.
+// BitReader's 64-bit shifts and its shifting of six words cost several times
+// that.  R-MAT 20, K = 1, settled steps: group kernels of 16 / 64 / 256 lanes
+// 28.5 / 56.6 / 44.9 -> 22.4 / 48.1 / 40.7 us per launch; R-MAT 19 decoded to
+// CSR with coalesced stores besides: 316 -> 160 us per step.
+// CHECK: words from index `lim` on are not staged and are read from the
+// stream itself (64-bit words W from index `base`).
+template <bool CHECK> struct WinReader {
+    const uint32_t *w;
+    uint32_t q;
+    uint32_t lim;
+    const uint64_t *__restrict__ W;
+    uint64_t base;
+
+    LPA_HD __forceinline__ void set(uint64_t bit) { q = (uint32_t)(bit - (base << 6)) + 63; }
+    LPA_HD __forceinline__ uint32_t stream_word(uint32_t k) const {
+        const uint64_t x = W[base + ((k - 2) >> 1)];
+        return (k & 1) ? (uint32_t)x : (uint32_t)(x >> 32);
+    }
+    static LPA_HD __forceinline__ uint32_t funnel(uint32_t a, uint32_t b, uint32_t q) {
+#ifdef __HIP_DEVICE_COMPILE__
+        return __builtin_amdgcn_alignbit(a, b, ~q);   // by the low 5 bits of ~q
+#else
+        return (uint32_t)((((uint64_t)a << 32) | b) >> (~q & 31));
+#endif
+    }
+    LPA_HD __forceinline__ uint32_t window() const {
+        const uint32_t k = q >> 5;
+        uint32_t a, b;
+        if (!CHECK || k + 1 < lim) {
+            a = w[k];
+            b = w[k + 1];
+        } else {
+            a = stream_word(k);
+            b = stream_word(k + 1);
+        }
+        return funnel(a, b, q);
+    }
+    // 64 bits at the position, `hi` its first 32
+    LPA_HD __forceinline__ uint64_t window64(uint32_t hi) const {
+        const uint32_t k = q >> 5;
+        uint32_t b, c;
+        if (!CHECK || k + 2 < lim) {
+            b = w[k + 1];
+            c = w[k + 2];
+        } else {
+            b = stream_word(k + 1);
+            c = stream_word(k + 2);
+        }
+        return ((uint64_t)hi << 32) | funnel(b, c, q);
+    }
+    LPA_HD __forceinline__ uint32_t gamma() {
+        const uint32_t hi = window();
+        if (hi >> 16) {
+            const uint32_t L = (uint32_t)__builtin_clz(hi), y = hi >> (31 - 2 * L);
+            q += 2 * L + 1;
+            return y - 1;
+        }
+        const uint64_t x = window64(hi);
+        const uint32_t L = (uint32_t)__builtin_clzll(x | 1ull), len = 2 * L + 1;
+        q += len;
+        return (uint32_t)((x >> (64 - len)) - 1);
+    }
+    LPA_HD __forceinline__ uint32_t zeta() {
+        const uint32_t hi = window();
+        if (hi >> 24) {
+            const uint32_t h = (uint32_t)__builtin_clz(hi);
+            const uint32_t y = (hi << (h + 1)) >> (29 - 3 * h);
+            q += 4 * h + 4;
+            return y - 1;
+        }
+        const uint64_t x = window64(hi);
+        const uint32_t h = (uint32_t)__builtin_clzll(x | 1ull), body = 3 * (h + 1);
+        q += 4 * (h + 1);
+        return (uint32_t)(((x << (h + 1)) >> (64 - body)) - 1);
+    }
+};
+
+// Stream word pair as staged: the 32 bits that come first at the lower index.
+LPA_HD __forceinline__ uint64_t staged_pair(uint64_t x) { return (x >> 32) | (x << 32); }
+
 // decode_first_num (graph_utils.cuh:34-37)
 LPA_HD __forceinline__ uint32_t from_nat(uint32_t v, uint32_t x) {
     return (x & 1) ? v - (x >> 1) - 1 : v + (x >> 1);
@@ -105,8 +192,8 @@ LPA_HD __forceinline__ uint32_t from_nat(uint32_t v, uint32_t x) {
 
 // Decodes the interval segment the reader stands at (vertex v); calls
 // emit_run(left, len) for every interval; leaves the reader after it.
-template <class F>
-LPA_HD __forceinline__ void read_interval_segment(BitReader &r, uint32_t v, F &&emit_run) {
+template <class R, class F>
+LPA_HD __forceinline__ void read_interval_segment(R &r, uint32_t v, F &&emit_run) {
     const uint32_t c = r.gamma();
     uint32_t stop = 0;
     for (uint32_t t = 0; t < c; t++) {
@@ -117,15 +204,23 @@ LPA_HD __forceinline__ void read_interval_segment(BitReader &r, uint32_t v, F &&
     }
 }
 
-// Decodes the residual segment the reader stands at; emit(u) per neighbour.
-template <class F>
-LPA_HD __forceinline__ void read_residual_segment(BitReader &r, uint32_t v, F &&emit) {
-    const uint32_t c = r.gamma();
-    uint32_t cur = 0;
-    for (uint32_t t = 0; t < c; t++) {
-        cur = (t == 0) ? from_nat(v, r.zeta()) : cur + r.zeta() + 1;
+// Decodes the c ids of a residual segment (the reader stands after its count).
+template <class R, class F>
+LPA_HD __forceinline__ void read_residual_ids(R &r, uint32_t v, uint32_t c, F &&emit) {
+    if (c == 0) return;
+    uint32_t cur = from_nat(v, r.zeta());
+    emit(cur);
+    for (uint32_t t = 1; t < c; t++) {
+        cur += r.zeta() + 1;
         emit(cur);
     }
+}
+
+// Decodes the residual segment the reader stands at; emit(u) per neighbour.
+template <class R, class F>
+LPA_HD __forceinline__ void read_residual_segment(R &r, uint32_t v, F &&emit) {
+    const uint32_t c = r.gamma();
+    read_residual_ids(r, v, c, emit);
 }
 
 // Interval segment at bit q; returns the bit just after it.
@@ -155,6 +250,25 @@ LPA_HD __forceinline__ uint32_t block_header(const uint64_t *__restrict__ W, uin
     uint32_t s = r.gamma() + 1;
     *base = r.pos;
     return s;
+}
+
+// Serial decode of a whole staged record (the reader stands at its start):
+// emit(u) per neighbour, in encoded order.
+template <class R, class F>
+LPA_HD __forceinline__ void read_record(R &r, uint32_t v, F &&emit) {
+    uint32_t ns = r.gamma() + 1, base = r.q;
+    for (uint32_t j = 0; j < ns; j++) {
+        r.q = base + SEG_BITS * j;
+        read_interval_segment(r, v, [&](uint32_t l, uint32_t len) {
+            for (uint32_t x = 0; x < len; x++) emit(l + x);
+        });
+    }
+    ns = r.gamma() + 1;
+    base = r.q;
+    for (uint32_t j = 0; j < ns; j++) {
+        r.q = base + SEG_BITS * j;
+        read_residual_segment(r, v, emit);
+    }
 }
 
 // Serial decode of a whole record by one lane with one reader: emit(u) per

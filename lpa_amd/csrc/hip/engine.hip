@@ -327,7 +327,7 @@ struct lpa_engine {
 
     void launch_bin(const Bin &b, StepArgs a, bool as_csr);
     HeavyArgs heavy_args(const HeavySet &hs, const StepArgs &a, bool as_csr) const;
-    void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1);
+    void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, bool to_csr = false);
     void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool decode = true);
     template <class F> void for_each_batch(F &&fn);
     void step_host_stream();
@@ -489,12 +489,15 @@ HeavyArgs lpa_engine::heavy_args(const HeavySet &hs, const StepArgs &a, bool as_
     return h;
 }
 
-// Decode tasks [t0, t1) of a heavy set (compressed part) into its lists.
-void lpa_engine::launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1) {
+// Decode tasks [t0, t1) of a heavy set (compressed part) into its lists, or
+// into their rows of the decoded CSR.
+void lpa_engine::launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, bool to_csr) {
     if (t1 <= t0) return;
     const HeavyArgs h = heavy_args(hs, a, false);
-    if (hs.cms) hipLaunchKernelGGL(k_heavy_decode<1>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0);
-    else hipLaunchKernelGGL(k_heavy_decode<0>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0);
+    const uint64_t *row = to_csr ? crow.p : nullptr;
+    uint32_t *col = to_csr ? ccol.p : nullptr;
+    if (hs.cms) hipLaunchKernelGGL(k_heavy_decode<1>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0, row, col);
+    else hipLaunchKernelGGL(k_heavy_decode<0>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0, row, col);
 }
 
 // A heavy set's step: decode its records into the lists (unless `decode` is
@@ -785,6 +788,9 @@ int lpa_engine_create(int device, lpa_engine **out) {
                                        (const void *)k_heavy_local<0, 1, 8>, (const void *)k_heavy_local<0, HEAVY_KB_MAX, 8>,
                                        (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>,
                                        (const void *)k_heavy_local<1, 1, 4>, (const void *)k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>};
+            for (const void *f : {(const void *)k_decode_csr_group<16>, (const void *)k_decode_csr_group<64>,
+                                  (const void *)k_decode_csr_group<BLOCK>})
+                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
             for (const void *f : heavy_fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
             (void)hipGetLastError();
         } catch (...) {
@@ -1255,6 +1261,7 @@ static void build_heavy(lpa_engine *e) {
                         t.j0 = j0;
                         t.ni = hm[i].y;
                         t.ns = segs;
+                        t.h = i;
                         tk.push_back(t);
                         owner.push_back(i);
                         hs->task_pos.push_back(q);
@@ -1760,28 +1767,64 @@ int lpa_set_graph_mode(lpa_engine *e, int on) {
 }
 
 // CGLP's first kernel over stream positions [p0, p1): decode every
-// compressed record there into its CSR row.
-static void decode_range(lpa_engine *e, const uint64_t *words, uint32_t p0, uint32_t p1) {
+// compressed record there into its CSR row.  Heavy records run as decode
+// tasks, task[j] of heavy set j.
+static void decode_range(lpa_engine *e, const uint64_t *words, uint32_t p0, uint32_t p1,
+                         const std::vector<std::pair<uint32_t, uint32_t>> &tasks) {
     for (const Bin &b : e->bins) {
-        if (b.csr || b.kind == LPA_BIN_SKIP) continue;
+        if (b.csr) continue;
         const uint32_t lo = std::max(b.begin, p0), hi = std::min(b.end, p1);
         if (lo >= hi) continue;
-        const uint32_t count = hi - lo;
-        if (b.maxdeg <= 256)
-            hipLaunchKernelGGL(k_decode_csr, dim3((count + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, e->stream, words,
-                               e->offs.p, e->vid.p, e->crow.p, e->ccol.p, lo, hi);
-        else
-            hipLaunchKernelGGL(k_decode_csr_group, dim3(std::min<uint32_t>(count, 4096)), dim3(BLOCK), 0, e->stream,
-                               words, e->offs.p, e->vid.p, e->crow.p, e->ccol.p, lo, hi);
+        const uint32_t count = hi - lo, logT = (uint32_t)b.param;
+        switch (b.kind) {
+        case LPA_BIN_LANE: {
+            const dim3 g((count + BLOCK - 1) / BLOCK);
+            auto lane = [&](auto fn) {
+                hipLaunchKernelGGL(fn, g, dim3(BLOCK), 0, e->stream, words, e->offs.p, e->vid.p, e->crow.p, e->ccol.p, lo, hi);
+            };
+            switch (b.param) {
+            case 4: lane(k_decode_csr<4>); break;
+            case 8: lane(k_decode_csr<8>); break;
+            case 16: lane(k_decode_csr<16>); break;
+            case 32: lane(k_decode_csr<32>); break;
+            default: lane(k_decode_csr<64>); break;
+            }
+            break;
+        }
+        case LPA_BIN_WAVE:
+        case LPA_BIN_BLOCK: {
+            const int ng = b.kind == LPA_BIN_BLOCK ? 1 : wave_groups(logT);
+            const dim3 g((count + ng - 1) / ng);
+            auto group = [&](auto fn) {
+                hipLaunchKernelGGL(fn, g, dim3(BLOCK), group_lds(ng, logT), e->stream, words, e->offs.p, e->vid.p,
+                                   e->meta.p, e->crow.p, e->ccol.p, lo, hi, logT);
+            };
+            if (ng == 1) group(k_decode_csr_group<BLOCK>);
+            else if (ng == 4) group(k_decode_csr_group<64>);
+            else group(k_decode_csr_group<16>);
+            break;
+        }
+        default: break;   // degree 0; heavy records follow
+        }
+    }
+    for (size_t j = 0; j < e->heavy.size(); j++) {
+        if (e->heavy[j]->csr_part) continue;
+        StepArgs a = e->base_args(false);
+        a.words = words;
+        e->launch_heavy_decode(*e->heavy[j], a, tasks[j].first, tasks[j].second, true);
     }
 }
 
 // Decodes the whole compressed part to the CSR (batch by batch when the
 // stream is host-resident).
 static void decode_all(lpa_engine *e) {
-    if (e->host_stream)
-        e->for_each_batch([&](const StreamBatch &sb, const uint64_t *w) { decode_range(e, w, sb.p0, sb.p1); });
-    else decode_range(e, e->words.p, 0, (uint32_t)e->n_c);
+    if (e->host_stream) {
+        e->for_each_batch([&](const StreamBatch &sb, const uint64_t *w) { decode_range(e, w, sb.p0, sb.p1, sb.tasks); });
+    } else {
+        std::vector<std::pair<uint32_t, uint32_t>> all;
+        for (auto &hs : e->heavy) all.push_back({0u, hs->ntasks});
+        decode_range(e, e->words.p, 0, (uint32_t)e->n_c, all);
+    }
     HIPCHK(hipGetLastError());
 }
 

@@ -128,7 +128,7 @@ struct DecodeTask {
     uint64_t ibase, rbase;   // absolute bit of interval segment 0 / residual segment 0
     uint64_t out;            // first list slot of the task's ids
     uint32_t v, j0, ni, ns;  // vertex, first segment, #interval segments, #segments
-    uint32_t count, pad;     // ids the task writes
+    uint32_t count, h;       // ids the task writes; index of its heavy vertex
 };
 constexpr uint32_t DECODE_STAGE = 8192;
 
@@ -157,61 +157,83 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_task_count(StepArgs a, DecodeTa
     if (threadIdx.x == 0) tasks[t].count = total;
 }
 
-// One workgroup per task: each lane decodes its segment, claiming output
-// slots with one LDS atomic per run (runs of LONG_RUN or more ids are
-// written by the whole workgroup) or per residual segment; the task's ids
-// are assembled in LDS and stored to the list with coalesced stores, or
-// written in place when they exceed the staging buffer.
+// One workgroup per task: the words of its segments (one range of interval
+// segments, one of residual segments) are staged in LDS, then each lane
+// decodes its segment, claiming output slots with one LDS atomic per run
+// (runs of LONG_RUN or more ids are written by the whole workgroup) or per
+// residual segment; the task's ids are assembled in LDS and stored to the list
+// with coalesced stores, or written in place when they exceed the staging
+// buffer.  With crow the ids go to the heavy vertex's row of the decoded CSR
+// ccol instead.
 // CMS: the heavy set's mode (names the launch in profiles; same code)
+constexpr uint32_t TASK_WORDS = BLOCK * SEG_BITS / 64;   // 64-bit words of a task's segments
+constexpr uint32_t TASK_AHEAD = 8;   // words staged from the last segment's first (the stream is
+                                     // padded by as many): most of a merged last segment
 template <int CMS>
 __global__ void __launch_bounds__(BLOCK) k_heavy_decode(HeavyArgs h, const DecodeTask *__restrict__ tasks,
-                                                        uint32_t ntasks) {
+                                                        uint32_t ntasks, const uint64_t *__restrict__ crow,
+                                                        uint32_t *__restrict__ ccol) {
     __shared__ GroupShared<BLOCK> sh;
     __shared__ uint32_t stage[DECODE_STAGE];
+    __shared__ uint64_t sw[TASK_WORDS + 2 * (TASK_AHEAD + 1)];
     const uint32_t t = blockIdx.x;
     if (t >= ntasks || h.csr) return;
     const uint64_t t0 = h.s.rec ? cycles() : 0;
     const DecodeTask T = tasks[t];
+    const uint64_t *__restrict__ W = h.s.words;
     if (threadIdx.x == 0) {
         sh.cnt = 0;
         sh.qn = 0;
     }
+    // segments [j0, j1) of the record; those below ni are interval segments
+    const uint32_t j1 = T.ns - T.j0 < (uint32_t)BLOCK ? T.ns : T.j0 + BLOCK;
+    const uint32_t i1 = j1 < T.ni ? j1 : T.ni, r0 = T.j0 < T.ni ? T.ni : T.j0;
+    // words of segments [a, b) of the block at bit `at`, behind one dummy word
+    auto stage_range = [&](uint64_t at, uint32_t a, uint32_t b, uint64_t *to, uint64_t &base) -> uint32_t {
+        base = (at + (uint64_t)SEG_BITS * a) >> 6;
+        if (b <= a) return 0;
+        const uint32_t nw = (uint32_t)(((at + (uint64_t)SEG_BITS * (b - 1)) >> 6) - base) + TASK_AHEAD;
+        for (uint32_t i = threadIdx.x; i < nw; i += BLOCK) to[i + 1] = staged_pair(W[base + i]);
+        return nw + 1;
+    };
+    uint64_t ib, rb;
+    const uint32_t iw = stage_range(T.ibase, T.j0, i1, sw, ib);
+    const uint32_t rw = stage_range(T.rbase, r0 - T.ni, j1 > r0 ? j1 - T.ni : r0 - T.ni, sw + iw, rb);
     __syncthreads();
-    uint32_t *out = h.list + T.out;
     const bool staged = T.count <= DECODE_STAGE;
-    uint32_t *dst = staged ? stage : out;
+    uint32_t *out = crow ? ccol + crow[h.pos[T.h]] + (T.out - h.loff[T.h]) : h.list + T.out;
     const uint32_t j = T.j0 + threadIdx.x;
-    if (j < T.ns) {
-        BitReader r;
-        if (task_segment(h.s, T, j, r)) {
-            read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
-                const uint32_t o = atomicAdd(&sh.cnt, len);
-                if (len >= LONG_RUN) {
-                    const uint32_t q = atomicAdd(&sh.qn, 1u);
-                    if (q < (uint32_t)GroupShared<BLOCK>::QCAP) {
-                        sh.qleft[q] = l;
-                        sh.qlen[q] = len;
-                        sh.qpos[q] = o;
-                        return;
-                    }
-                }
-                for (uint32_t x = 0; x < len; x++) dst[o + x] = l + x;
-            });
-        } else {
-            BitReader peek = r;   // the segment's count claims its slots
-            uint32_t o = atomicAdd(&sh.cnt, peek.gamma());
-            read_residual_segment(r, T.v, [&](uint32_t u) { dst[o++] = u; });
+    auto decode = [&](uint32_t *dst) {
+        if (j < j1) {
+            WinReader<true> r{};
+            r.W = W;
+            if (j < T.ni) {
+                r.w = reinterpret_cast<const uint32_t *>(sw);
+                r.lim = 2 * iw;
+                r.base = ib;
+                r.set(T.ibase + (uint64_t)SEG_BITS * j);
+                read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
+                    put_run<BLOCK>(&sh, dst, atomicAdd(&sh.cnt, len), l, len);
+                });
+            } else {
+                r.w = reinterpret_cast<const uint32_t *>(sw + iw);
+                r.lim = 2 * rw;
+                r.base = rb;
+                r.set(T.rbase + (uint64_t)SEG_BITS * (j - T.ni));
+                const uint32_t c = r.gamma();   // claims the segment's slots
+                uint32_t o = atomicAdd(&sh.cnt, c);
+                read_residual_ids(r, T.v, c, [&](uint32_t u) { dst[o++] = u; });
+            }
         }
-    }
-    __syncthreads();
-    const uint32_t nq = sh.qn < (uint32_t)GroupShared<BLOCK>::QCAP ? sh.qn : (uint32_t)GroupShared<BLOCK>::QCAP;
-    for (uint32_t q = 0; q < nq; q++) {
-        const uint32_t l = sh.qleft[q], len = sh.qlen[q], qo = sh.qpos[q];
-        for (uint32_t x = threadIdx.x; x < len; x += BLOCK) dst[qo + x] = l + x;
-    }
-    if (staged) {
+        __syncthreads();
+        write_long_runs<BLOCK>(&sh, threadIdx.x, dst);
+    };
+    if (staged) {   // two instances: LDS stores in one, global stores in the other
+        decode(stage);
         __syncthreads();
         for (uint32_t x = threadIdx.x; x < T.count; x += BLOCK) out[x] = stage[x];
+    } else {
+        decode(out);
     }
     if (h.s.rec && threadIdx.x == 0) atomicAdd(&h.s.rec[T.v], (cycles() - t0) * BLOCK);
 }

@@ -164,6 +164,24 @@ __device__ __forceinline__ void load_row(const StepArgs &a, uint32_t u, uint32_t
     }
 }
 
+// 64-bit stream words a workgroup of the lane kernels stages: its 256 records
+// lie back to back in the stream (about 60 bits each at N = 4, 400 at N =
+// 32).  A longer range is read in place.
+template <int N> constexpr uint32_t lane_stage_words() { return N <= 4 ? 512 : N <= 8 ? 768 : N <= 16 ? 1152 : 2048; }
+
+// Stages the words of records [first, first + cnt) of the stream in sw (one
+// dummy word before them), with coalesced loads; false when they do not fit.
+// The same in every lane; the caller synchronises before reading.
+template <uint32_t CAP>
+__device__ __forceinline__ bool stage_records(const uint64_t *__restrict__ words, const uint64_t *__restrict__ offs,
+                                              uint32_t first, uint32_t cnt, uint64_t *sw, uint64_t &base) {
+    base = offs[first] >> 6;
+    const uint64_t nw = ((offs[first + cnt] + 63) >> 6) - base;
+    if (nw > CAP) return false;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)nw; i += BLOCK) sw[i + 1] = staged_pair(words[base + i]);
+    return true;
+}
+
 // One lane per vertex decodes the record into LDS (CSR=false) or looks up
 // its CSR row (CSR=true); then the block's (vertex, label vector) pairs are
 // dealt out to the lanes with the vector index fastest, so the lanes that
@@ -180,10 +198,19 @@ __global__ void __launch_bounds__(BLOCK) k_lane(StepArgs a) {
     __shared__ uint32_t rows[STAGE ? N * BLOCK : 1];
     __shared__ uint32_t sv[BLOCK], sd[BLOCK];
     __shared__ uint64_t sbase[CSR ? BLOCK : 1];
+    constexpr uint32_t SW = lane_stage_words<N>();
+    __shared__ uint64_t sw[CSR ? 1 : SW + 3];   // a dummy before, look-ahead after
     const uint32_t first = a.begin + xcd_tile(blockIdx.x, gridDim.x, a.xcds) * BLOCK;
     const uint32_t p = first + threadIdx.x;
     const uint32_t nact = a.end - first < (uint32_t)BLOCK ? a.end - first : (uint32_t)BLOCK;
     const uint64_t t0 = a.rec ? cycles() : 0;
+    WinReader<false> r{};
+    bool staged = false;
+    if (!CSR) {
+        r.w = reinterpret_cast<const uint32_t *>(sw);
+        staged = stage_records<SW>(a.words, a.offs, first, nact, sw, r.base);
+        __syncthreads();
+    }
     const uint64_t b0 = STAGE ? a.row[first] : 0;
     if (p < a.end) {
         uint32_t d = 0;
@@ -194,10 +221,16 @@ __global__ void __launch_bounds__(BLOCK) k_lane(StepArgs a) {
         } else {
             const uint32_t v = a.vid[p];
             sv[threadIdx.x] = v;
-            decode_record(a.words, a.offs[p], v, [&](uint32_t u) {
+            auto put = [&](uint32_t u) {
                 if (d < N) list[d][threadIdx.x] = u;
                 d++;
-            });
+            };
+            if (staged) {
+                r.set(a.offs[p]);
+                read_record(r, v, put);
+            } else {
+                decode_record(a.words, a.offs[p], v, put);
+            }
         }
         sd[threadIdx.x] = d;
         if (a.rec) atomicAdd(&a.rec[sv[threadIdx.x]], cycles() - t0);
@@ -360,7 +393,6 @@ constexpr uint32_t LONG_RUN = 16;
 
 template <int G> struct GroupShared {
     static constexpr int QCAP = G == BLOCK ? 512 : G == 64 ? 64 : G == 32 ? 32 : 16;
-    uint64_t res_start;
     uint32_t cnt;                 // ids written to the list so far
     uint32_t qn;
     uint32_t qleft[QCAP];
@@ -368,58 +400,99 @@ template <int G> struct GroupShared {
     uint32_t qpos[QCAP];
 };
 
-// Phase A: the G lanes of a group decode the record at position p into
-// `list` (order irrelevant to the mode).  Segments (256-bit units) go one
-// per lane: the interval block first, then the residual block, which starts
-// where the last interval segment ends.  Each run claims its slots with one
-// LDS atomic, each residual segment with one atomic for its whole count;
-// runs of LONG_RUN or more ids are written by all lanes together so a hub
-// whose neighbours form one long run is not written by a single lane.
-// Returns the degree (valid in every lane of the group).
+// The record of position p staged in `stage` (cap 64-bit words) by its group,
+// or read in place when it does not fit.  A record of d ids takes less than
+// 64 d + 256 bits when its segments are as full as the encoder makes them.
+// fn(at) runs with at(bit) = a reader at that bit of the stream.
+template <int G, class F>
+__device__ __forceinline__ void with_record(const uint64_t *__restrict__ words, uint64_t start, uint64_t stop,
+                                            uint32_t gl, uint64_t *stage, uint32_t cap, F &&fn) {
+    const uint64_t base = start >> 6, nw = ((stop + 63) >> 6) - base;
+    if (nw + 3 <= cap) {   // a dummy word before, look-ahead after
+        for (uint32_t i = gl; i < (uint32_t)nw; i += G) stage[i + 1] = staged_pair(words[base + i]);
+        group_sync<G>();
+        fn([&](uint64_t bit) {
+            WinReader<false> r{};
+            r.w = reinterpret_cast<const uint32_t *>(stage);
+            r.base = base;
+            r.set(bit);
+            return r;
+        });
+    } else {
+        group_sync<G>();
+        fn([&](uint64_t bit) {
+            BitReader r;
+            r.seek(words, bit);
+            return r;
+        });
+    }
+}
+
+// Runs of LONG_RUN or more ids queued by the lanes, written by the group.
 template <int G>
-__device__ __forceinline__ uint32_t group_decode(const StepArgs &a, uint32_t p, uint32_t v, uint32_t gl,
-                                                 GroupShared<G> *sh, uint32_t *list) {
-    if (gl == 0) {
-        sh->cnt = 0;
-        sh->qn = 0;
-    }
-    group_sync<G>();
-    // segment j of the record (intervals first, then residuals) is at a
-    // position known from the metadata: every lane seeks its own segment
-    const uint64_t start = a.offs[p];
-    const uint4 m = a.meta[p];
-    const uint32_t ni = m.y, ns = m.y + m.w;
-    auto emit_run = [&](uint32_t l, uint32_t len) {
-        const uint32_t o = atomicAdd(&sh->cnt, len);
-        if (len >= LONG_RUN) {
-            const uint32_t q = atomicAdd(&sh->qn, 1u);
-            if (q < (uint32_t)GroupShared<G>::QCAP) {
-                sh->qleft[q] = l;
-                sh->qlen[q] = len;
-                sh->qpos[q] = o;
-                return;
-            }
-        }
-        for (uint32_t x = 0; x < len; x++) list[o + x] = l + x;
-    };
-    for (uint32_t j = gl; j < ns; j += G) {
-        BitReader r;
-        if (j < ni) {
-            r.seek(a.words, start + m.x + (uint64_t)SEG_BITS * j);
-            read_interval_segment(r, v, emit_run);
-        } else {
-            r.seek(a.words, start + m.z + (uint64_t)SEG_BITS * (j - ni));
-            BitReader peek = r;   // the segment's count claims its list slots
-            uint32_t o = atomicAdd(&sh->cnt, peek.gamma());
-            read_residual_segment(r, v, [&](uint32_t u) { list[o++] = u; });
-        }
-    }
-    group_sync<G>();
+__device__ __forceinline__ void write_long_runs(const GroupShared<G> *sh, uint32_t gl, uint32_t *list) {
     const uint32_t nq = sh->qn < (uint32_t)GroupShared<G>::QCAP ? sh->qn : (uint32_t)GroupShared<G>::QCAP;
     for (uint32_t q = 0; q < nq; q++) {
         const uint32_t l = sh->qleft[q], len = sh->qlen[q], o = sh->qpos[q];
         for (uint32_t x = gl; x < len; x += G) list[o + x] = l + x;
     }
+}
+
+// Ids l .. l + len - 1 at list[o ..): queued for the group when the run is
+// long and the queue has room.
+template <int G>
+__device__ __forceinline__ void put_run(GroupShared<G> *sh, uint32_t *list, uint32_t o, uint32_t l, uint32_t len) {
+    if (len >= LONG_RUN) {
+        const uint32_t q = atomicAdd(&sh->qn, 1u);
+        if (q < (uint32_t)GroupShared<G>::QCAP) {
+            sh->qleft[q] = l;
+            sh->qlen[q] = len;
+            sh->qpos[q] = o;
+            return;
+        }
+    }
+    for (uint32_t x = 0; x < len; x++) list[o + x] = l + x;
+}
+
+// Phase A: the G lanes of a group decode the record at position p into
+// `list` (order irrelevant to the mode).  The record's words are staged in
+// `stage` first (the memory of the group's table, which is not in use yet).
+// Segments (256-bit units) go one per lane: the interval block first, then
+// the residual block, which starts where the last interval segment ends.
+// Each run claims its slots with one LDS atomic, each residual segment with
+// one atomic for its whole count; runs of LONG_RUN or more ids are written by
+// all lanes together so a hub whose neighbours form one long run is not
+// written by a single lane.  Returns the degree (valid in every lane of the
+// group).
+template <int G>
+__device__ __forceinline__ uint32_t group_decode(const StepArgs &a, uint32_t p, uint32_t v, uint32_t gl,
+                                                 GroupShared<G> *sh, uint32_t *list, uint64_t *stage, uint32_t cap) {
+    if (gl == 0) {
+        sh->cnt = 0;
+        sh->qn = 0;
+    }
+    // segment j of the record (intervals first, then residuals) is at a
+    // position known from the metadata: every lane seeks its own segment
+    const uint64_t start = a.offs[p];
+    const uint4 m = a.meta[p];
+    const uint32_t ni = m.y, ns = m.y + m.w;
+    with_record<G>(a.words, start, a.offs[p + 1], gl, stage, cap, [&](auto &&at) {
+        for (uint32_t j = gl; j < ns; j += G) {
+            if (j < ni) {
+                auto r = at(start + m.x + (uint64_t)SEG_BITS * j);
+                read_interval_segment(r, v, [&](uint32_t l, uint32_t len) {
+                    put_run<G>(sh, list, atomicAdd(&sh->cnt, len), l, len);
+                });
+            } else {
+                auto r = at(start + m.z + (uint64_t)SEG_BITS * (j - ni));
+                const uint32_t c = r.gamma();   // claims the segment's list slots
+                uint32_t o = atomicAdd(&sh->cnt, c);
+                read_residual_ids(r, v, c, [&](uint32_t u) { list[o++] = u; });
+            }
+        }
+    });
+    group_sync<G>();
+    write_long_runs<G>(sh, gl, list);
     if (G == BLOCK) __threadfence_block();
     group_sync<G>();
     return sh->cnt;
@@ -635,7 +708,7 @@ __global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint
                 d = (uint32_t)(a.row[p + 1] - a.row[p]);
             }
         } else if (live) {
-            d = group_decode<G>(a, p, v, gl, sh, list);
+            d = group_decode<G>(a, p, v, gl, sh, list, tab, T);
         }
         for (uint32_t k0 = 0; k0 < a.K; k0 += KB) {
             const uint32_t kb = a.K - k0 < (uint32_t)KB ? a.K - k0 : (uint32_t)KB;
@@ -694,79 +767,127 @@ __global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint
 
 // --------------------------------------------------------- CGLP kernel 1
 
-// Decode the records of positions [begin,end) into CSR rows crow[p]..crow[p+1]
-// (rows follow the device layout; one lane per record; the two-kernel
-// method's decode step).
+// Decode the records of positions [begin,end), of at most N ids each, into
+// CSR rows crow[p]..crow[p+1] (rows follow the device layout, so a
+// workgroup's 256 rows are one range of ccol); one lane per record, ids
+// assembled in LDS and stored with coalesced stores.
+template <int N>
 __global__ void __launch_bounds__(BLOCK) k_decode_csr(const uint64_t *__restrict__ words,
                                                       const uint64_t *__restrict__ offs,
                                                       const uint32_t *__restrict__ vid,
                                                       const uint64_t *__restrict__ crow,
                                                       uint32_t *__restrict__ ccol, uint32_t begin, uint32_t end) {
-    const uint32_t p = begin + blockIdx.x * BLOCK + threadIdx.x;
-    if (p >= end) return;
-    const uint32_t v = vid[p];
-    uint64_t o = crow[p];
-    decode_record(words, offs[p], v, [&](uint32_t u) { ccol[o++] = u; });
+    constexpr uint32_t SW = lane_stage_words<N>();
+    __shared__ uint64_t sw[SW + 3];
+    __shared__ uint32_t out[N * BLOCK];
+    const uint32_t first = begin + blockIdx.x * BLOCK, p = first + threadIdx.x;
+    const uint32_t cnt = end - first < (uint32_t)BLOCK ? end - first : (uint32_t)BLOCK;
+    WinReader<false> r{};
+    r.w = reinterpret_cast<const uint32_t *>(sw);
+    const bool staged = stage_records<SW>(words, offs, first, cnt, sw, r.base);
+    const uint64_t o0 = crow[first];
+    __syncthreads();
+    if (p < end) {
+        const uint32_t v = vid[p];
+        uint32_t o = (uint32_t)(crow[p] - o0);
+        auto put = [&](uint32_t u) { out[o++] = u; };
+        if (staged) {
+            r.set(offs[p]);
+            read_record(r, v, put);
+        } else {
+            decode_record(words, offs[p], v, put);
+        }
+    }
+    __syncthreads();
+    const uint32_t tot = (uint32_t)(crow[first + cnt] - o0);
+    for (uint32_t x = threadIdx.x; x < tot; x += BLOCK) ccol[o0 + x] = out[x];
 }
 
-// Same for long records: a workgroup per record, one lane per segment;
-// output slots are claimed with an LDS cursor, and intervals of LONG_RUN or
-// more ids are written by all lanes together.
+// Exclusive sum of x over the group's lanes (every lane calls it), and the
+// total; xs: LDS for one word per wave when G > 64.
+template <int G>
+__device__ __forceinline__ uint32_t group_scan(uint32_t x, uint32_t *xs, uint32_t &total) {
+    constexpr int W = G < 64 ? G : 64;
+    const uint32_t wl = threadIdx.x & (W - 1);
+    uint32_t inc = x;
+#pragma unroll
+    for (int o = 1; o < W; o <<= 1) {
+        const uint32_t y = __shfl_up(inc, o, W);
+        if (wl >= (uint32_t)o) inc += y;
+    }
+    total = __shfl(inc, W - 1, W);
+    if (G <= 64) return inc - x;
+    __syncthreads();   // the last use of xs is over
+    if (wl == 0) xs[threadIdx.x >> 6] = total;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+    for (uint32_t w = 0; w < G / 64; w++) {
+        if (w < threadIdx.x >> 6) before += xs[w];
+        total += xs[w];
+    }
+    return before + inc - x;
+}
+
+// Same for longer records: G lanes per record, one lane per segment; the
+// ids' places follow from the segments' counts, so the rows keep the encoded
+// order; assembled in LDS, stored with coalesced stores.  Dynamic LDS per
+// group as in k_group.
+template <int G>
 __global__ void __launch_bounds__(BLOCK) k_decode_csr_group(const uint64_t *__restrict__ words,
                                                             const uint64_t *__restrict__ offs,
                                                             const uint32_t *__restrict__ vid,
+                                                            const uint4 *__restrict__ meta,
                                                             const uint64_t *__restrict__ crow,
                                                             uint32_t *__restrict__ ccol, uint32_t begin,
-                                                            uint32_t end) {
-    constexpr int QCAP = 512;
-    __shared__ uint64_t res_start;
-    __shared__ unsigned long long cursor;
-    __shared__ uint32_t qn;
-    __shared__ uint32_t qleft[QCAP], qlen[QCAP];
-    __shared__ uint64_t qout[QCAP];
-    for (uint32_t p = begin + blockIdx.x; p < end; p += gridDim.x) {
-        const uint32_t v = vid[p];
-        if (threadIdx.x == 0) {
-            cursor = crow[p];
-            qn = 0;
+                                                            uint32_t end, uint32_t logT) {
+    constexpr int NG = BLOCK / G;
+    extern __shared__ uint64_t lds[];
+    __shared__ GroupShared<G> gsh[NG];
+    __shared__ uint32_t xs[BLOCK / 64];
+    const uint32_t gid = threadIdx.x / G, gl = threadIdx.x % G, T = 1u << logT;
+    uint64_t *stage = lds + (uint64_t)gid * (T + T / 4);
+    uint32_t *list = (uint32_t *)(stage + T);
+    GroupShared<G> *sh = &gsh[gid];
+    const uint32_t p = begin + blockIdx.x * NG + gid;
+    if (p >= end) return;   // whole groups; a workgroup of one group is never empty
+    const uint32_t v = vid[p];
+    const uint64_t start = offs[p], o0 = crow[p];
+    const uint32_t d = (uint32_t)(crow[p + 1] - o0);
+    const uint4 m = meta[p];
+    if (gl == 0) sh->qn = 0;
+    with_record<G>(words, start, offs[p + 1], gl, stage, T, [&](auto &&at) {
+        uint32_t done = 0, total;
+        for (uint32_t j0 = 0; j0 < m.y; j0 += G) {
+            const uint32_t j = j0 + gl;
+            uint32_t c = 0;
+            if (j < m.y) {
+                auto r = at(start + m.x + (uint64_t)SEG_BITS * j);
+                read_interval_segment(r, v, [&](uint32_t, uint32_t len) { c += len; });
+            }
+            uint32_t o = done + group_scan<G>(c, xs, total);
+            done += total;
+            if (c) {
+                auto r = at(start + m.x + (uint64_t)SEG_BITS * j);
+                read_interval_segment(r, v, [&](uint32_t l, uint32_t len) {
+                    put_run<G>(sh, list, o, l, len);
+                    o += len;
+                });
+            }
         }
-        __syncthreads();
-        uint64_t base;
-        const uint32_t ni = block_header(words, offs[p], &base);
-        uint64_t my_end = 0;
-        for (uint32_t j = threadIdx.x; j < ni; j += BLOCK) {
-            uint64_t e = decode_interval_segment(words, base + (uint64_t)SEG_BITS * j, v,
-                                                 [&](uint32_t l, uint32_t len) {
-                                                     uint64_t o = atomicAdd(&cursor, (unsigned long long)len);
-                                                     if (len >= LONG_RUN) {
-                                                         uint32_t q = atomicAdd(&qn, 1u);
-                                                         if (q < QCAP) {
-                                                             qleft[q] = l;
-                                                             qlen[q] = len;
-                                                             qout[q] = o;
-                                                             return;
-                                                         }
-                                                     }
-                                                     for (uint32_t x = 0; x < len; x++) ccol[o + x] = l + x;
-                                                 });
-            if (j == ni - 1) my_end = e;
+        for (uint32_t j0 = 0; j0 < m.w; j0 += G) {
+            const uint32_t j = j0 + gl;
+            auto r = at(start + m.z + (uint64_t)SEG_BITS * (j < m.w ? j : 0));
+            const uint32_t c = j < m.w ? r.gamma() : 0;
+            uint32_t o = done + group_scan<G>(c, xs, total);
+            done += total;
+            read_residual_ids(r, v, c, [&](uint32_t u) { list[o++] = u; });
         }
-        if (threadIdx.x == ((ni - 1) & (BLOCK - 1))) res_start = my_end;
-        __syncthreads();
-        const uint32_t nq = qn < (uint32_t)QCAP ? qn : (uint32_t)QCAP;
-        for (uint32_t q = 0; q < nq; q++)
-            for (uint32_t x = threadIdx.x; x < qlen[q]; x += BLOCK) ccol[qout[q] + x] = qleft[q] + x;
-        const uint32_t nr = block_header(words, res_start, &base);
-        for (uint32_t j = threadIdx.x; j < nr; j += BLOCK) {
-            const uint64_t q = base + (uint64_t)SEG_BITS * j;
-            BitReader r;
-            r.seek(words, q);
-            const uint32_t c = r.gamma();
-            uint64_t o = atomicAdd(&cursor, (unsigned long long)c);
-            decode_residual_segment(words, q, v, [&](uint32_t u) { ccol[o++] = u; });
-        }
-        __syncthreads();
-    }
+    });
+    group_sync<G>();
+    write_long_runs<G>(sh, gl, list);
+    group_sync<G>();
+    for (uint32_t x = gl; x < d; x += G) ccol[o0 + x] = list[x];
 }
 
 }  // namespace lpa

@@ -64,6 +64,37 @@ int64_t dc_decode_segments(const uint64_t *words, uint64_t pos, uint32_t v, uint
     return (int64_t)d;
 }
 
+// The window reader over the record staged as the kernels stage it, all of
+// it (check 0), or only its first `have` 64-bit words with the rest read from
+// the stream (check 1).
+int64_t dc_decode_record_window(const uint64_t *words, uint64_t pos, uint64_t stop, uint32_t v, uint32_t *out,
+                                uint64_t cap, int check, uint64_t have) {
+    const uint64_t base = pos >> 6, nw = ((stop + 63) >> 6) - base;
+    std::vector<uint64_t> st(nw + 3, 0xAAAAAAAAAAAAAAAAull);   // dummy and look-ahead: any value
+    const uint64_t k = check ? (have < nw ? have : nw) : nw;
+    for (uint64_t i = 0; i < k; i++) st[i + 1] = lpa::staged_pair(words[base + i]);
+    uint64_t d = 0;
+    auto put = [&](uint32_t u) {
+        if (d < cap) out[d] = u;
+        d++;
+    };
+    auto run = [&](auto r) {
+        r.w = reinterpret_cast<const uint32_t *>(st.data());
+        r.base = base;
+        r.set(pos);
+        lpa::read_record(r, v, put);
+    };
+    if (check) {
+        lpa::WinReader<true> r{};
+        r.lim = (uint32_t)(2 * (k + 1));
+        r.W = words;
+        run(r);
+    } else {
+        run(lpa::WinReader<false>{});
+    }
+    return (int64_t)d;
+}
+
 // Bits of vertex v's record (sorted adjacency adj[0..d)), as the device
 // encoder measures it.
 uint64_t dc_encode_bits(uint32_t v, const uint32_t *adj, uint32_t d) {
