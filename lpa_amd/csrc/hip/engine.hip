@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "bfs_relabel.hpp"
+#include "bins.hpp"
 #include "encode_kernels.hpp"
 #include "encode_long.hpp"
 #include "encode_wave.hpp"
@@ -156,14 +157,6 @@ constexpr uint64_t DEFAULT_BATCH_BYTES = 1ull << 30;
 
 // XCDs of an MI355X (gfx950): workgroups are dealt to them round robin
 constexpr uint32_t XCDS = 8;
-
-struct Bin {
-    int kind;          // LPA_BIN_*
-    int param;         // LANE: network size N; WAVE/BLOCK: log2 table slots
-    bool csr;          // small-vertex CSR part
-    uint32_t begin, end;
-    uint32_t maxdeg;
-};
 
 inline uint32_t ceil_log2(uint64_t x) {
     uint32_t l = 0;
@@ -325,7 +318,6 @@ struct lpa_engine {
         return a;
     }
 
-    void launch_bin(const Bin &b, StepArgs a, bool as_csr);
     HeavyArgs heavy_args(const HeavySet &hs, const StepArgs &a, bool as_csr) const;
     void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, bool to_csr = false);
     void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool decode = true);
@@ -337,102 +329,6 @@ struct lpa_engine {
 };
 
 // ---------------------------------------------------------------- launches
-
-template <bool CSR> static void launch_lane(int N, StepArgs a, uint32_t count, hipStream_t s) {
-    dim3 grid((count + BLOCK - 1) / BLOCK);
-    switch (N) {
-    case 4: hipLaunchKernelGGL((k_lane<4, CSR>), grid, dim3(BLOCK), 0, s, a); break;
-    case 8: hipLaunchKernelGGL((k_lane<8, CSR>), grid, dim3(BLOCK), 0, s, a); break;
-    case 16: hipLaunchKernelGGL((k_lane<16, CSR>), grid, dim3(BLOCK), 0, s, a); break;
-    case 32: hipLaunchKernelGGL((k_lane<32, CSR>), grid, dim3(BLOCK), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_lane<64, CSR>), grid, dim3(BLOCK), 0, s, a); break;
-    }
-}
-
-// LDS bytes of the WAVE / BLOCK kernels' per-group table (2^logT slots) and
-// neighbour list (2^logT / 2 ids), for NG groups per workgroup.
-static size_t group_lds(int ng, uint32_t logT) { return (size_t)ng * 10ull * (1ull << logT); }
-static int wave_groups(uint32_t logT, uint32_t quarter_max = 128) {
-    return (1u << (logT - 1)) <= quarter_max ? 16 : 4;
-}
-
-// label vectors staged per row gather by the group kernels: 8 from K = 5
-// (one gather per neighbour and step at K = 8; with one aggregated match
-// round the kernels stay fast enough at the lower occupancy that even label
-// rows held by the 256 MB last-level cache gain from it), else K rounded
-// down to 4 / 2 / 1.
-static int group_kb(uint32_t K, uint64_t n) {
-    (void)n;
-    return K >= 5 ? 8 : K >= 3 ? 4 : K == 2 ? 2 : 1;
-}
-
-// instance of the group kernel for a batch size and staged ids per lane
-template <int G, bool CSR> static const void *group_fn(int kb, uint32_t ipl) {
-    switch (kb) {
-    case 1: return (const void *)k_group<G, CSR, 1, 8>;
-    case 2: return (const void *)k_group<G, CSR, 2, 8>;
-    case 4:
-        return ipl <= 2 ? (const void *)k_group<G, CSR, 4, 2>
-             : ipl <= 4 ? (const void *)k_group<G, CSR, 4, 4> : (const void *)k_group<G, CSR, 4, 8>;
-    default:
-        return ipl <= 2 ? (const void *)k_group<G, CSR, 8, 2>
-             : ipl <= 4 ? (const void *)k_group<G, CSR, 8, 4> : (const void *)k_group<G, CSR, 8, 8>;
-    }
-}
-
-template <int G>
-static void launch_group(bool as_csr, uint32_t K, uint64_t n, dim3 grid, size_t lds, hipStream_t s,
-                         const StepArgs &a, uint32_t logT, uint32_t cap) {
-    const uint32_t ipl = (cap + G - 1) / G;
-    // quarter-wave and wave groups hold few labels per lane: all 8 vectors
-    // of a batch fit their registers, and one gather per row wins
-    const int kb = G <= 64 && K >= 5 ? 8 : group_kb(K, n);
-    const void *fn = as_csr ? group_fn<G, true>(kb, ipl) : group_fn<G, false>(kb, ipl);
-    StepArgs args = a;
-    void *params[] = {&args, &logT, &cap};
-    (void)hipLaunchKernel(fn, grid, dim3(BLOCK), params, lds, s);
-}
-
-template <int G> static void allow_group_lds(int dyn) {
-    for (int kb : {1, 2, 4, 8})
-        for (uint32_t ipl : {2u, 4u, 8u})
-            for (const void *f : {group_fn<G, false>(kb, ipl), group_fn<G, true>(kb, ipl)})
-                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
-}
-
-void lpa_engine::launch_bin(const Bin &b, StepArgs a, bool as_csr) {
-    a.begin = b.begin;
-    a.end = b.end;
-    const uint32_t count = b.end - b.begin;
-    if (count == 0) return;
-    switch (b.kind) {
-    case LPA_BIN_LANE:
-        if (as_csr) launch_lane<true>(b.param, a, count, stream);
-        else launch_lane<false>(b.param, a, count, stream);
-        break;
-    case LPA_BIN_WAVE: {
-        // a quarter wave per vertex up to degree 128, a whole wave above
-        const uint32_t logT = (uint32_t)b.param, cap = 1u << (logT - 1);
-        int ng = wave_groups(logT, sched_used.quarter_max ? sched_used.quarter_max : 128);
-        // with 8 vectors per staged gather, lists of 65..128 ids take half
-        // waves (4 ids per lane) rather than quarter waves (8 per lane):
-        // half the staged registers, twice the waves resident
-        if (ng == 16 && cap > 64 && K >= 5) ng = 8;
-        const size_t lds = group_lds(ng, logT);
-        dim3 grid((count + ng - 1) / ng);
-        if (ng == 16) launch_group<16>(as_csr, K, n, grid, lds, stream, a, logT, cap);
-        else if (ng == 8) launch_group<32>(as_csr, K, n, grid, lds, stream, a, logT, cap);
-        else launch_group<64>(as_csr, K, n, grid, lds, stream, a, logT, cap);
-        break;
-    }
-    case LPA_BIN_BLOCK: {
-        const uint32_t logT = (uint32_t)b.param, cap = 1u << (logT - 1);
-        launch_group<BLOCK>(as_csr, K, n, dim3(count), group_lds(1, logT), stream, a, logT, cap);
-        break;
-    }
-    default: break;   // CMS and GLOBAL bins run through launch_heavy
-    }
-}
 
 // One-workgroup CMS kernel: label vectors per pass and its LDS bytes.  One
 // vector keeps 32-bit cells; several take 16-bit cells, two vectors to a
@@ -581,12 +477,13 @@ void lpa_engine::step(bool cglp, hipEvent_t *launch_events) {
     }
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)1, 0ull);
     StepArgs a = base_args(cglp);
-    for (size_t i = 0; i < bins.size(); i++) {
+    if (!launch_events) launch_bins(bins, a, cglp, sched_used.quarter_max, stream);
+    for (size_t i = 0; launch_events && i < bins.size(); i++) {
         const Bin &b = bins[i];
         if (b.kind == LPA_BIN_SKIP || b.kind == LPA_BIN_CMS || b.kind == LPA_BIN_GLOBAL || b.end == b.begin) continue;
-        if (launch_events) HIPCHK(hipEventRecord(launch_events[2 * i], stream));
-        launch_bin(b, a, b.csr || cglp);
-        if (launch_events) HIPCHK(hipEventRecord(launch_events[2 * i + 1], stream));
+        HIPCHK(hipEventRecord(launch_events[2 * i], stream));
+        launch_bin(b, a, b.csr || cglp, sched_used.quarter_max, stream);
+        HIPCHK(hipEventRecord(launch_events[2 * i + 1], stream));
     }
     run_heavy(cglp, launch_events);
     HIPCHK(hipGetLastError());
@@ -642,13 +539,15 @@ void lpa_engine::step_host_stream() {
             Bin c = b;
             c.begin = std::max(b.begin, sb.p0);
             c.end = std::min(b.end, sb.p1);
-            if (c.begin < c.end) launch_bin(c, ab, false);
+            if (c.begin < c.end) launch_bin(c, ab, false, sched_used.quarter_max, stream);
         }
         for (size_t j = 0; j < heavy.size(); j++)
             if (!heavy[j]->csr_part) launch_heavy_decode(*heavy[j], ab, sb.tasks[j].first, sb.tasks[j].second);
     });
+    std::vector<Bin> small;
     for (const Bin &b : bins)
-        if (b.csr && b.kind != LPA_BIN_SKIP && b.kind != LPA_BIN_CMS && b.kind != LPA_BIN_GLOBAL) launch_bin(b, a, true);
+        if (b.csr) small.push_back(b);
+    launch_bins(small, a, true, sched_used.quarter_max, stream);
     for (auto &hp : heavy) launch_heavy(*hp, a, hp->csr_part, false);
     HIPCHK(hipGetLastError());
 }
@@ -669,7 +568,7 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
             const Bin &b = bins[i];
             if (b.kind == LPA_BIN_SKIP || b.kind == LPA_BIN_CMS || b.kind == LPA_BIN_GLOBAL || b.end == b.begin) continue;
             HIPCHK(hipEventRecord(ev[2 * i], stream));
-            launch_bin(b, a, b.csr);
+            launch_bin(b, a, b.csr, sched_used.quarter_max, stream);
             HIPCHK(hipEventRecord(ev[2 * i + 1], stream));
             used[i] = 1;
         }
@@ -778,19 +677,13 @@ int lpa_engine_create(int device, lpa_engine **out) {
             e->counter.alloc(1);
             HIPCHK(hipHostMalloc((void **)&e->h_counter, sizeof(unsigned long long), hipHostMallocDefault));
             const int dyn = (int)(e->lds_max - 20480);
-            allow_group_lds<16>(dyn);
-            allow_group_lds<32>(dyn);
-            allow_group_lds<64>(dyn);
-            allow_group_lds<BLOCK>(dyn);
+            bins_allow_lds(dyn);
             const void *heavy_fns[] = {(const void *)k_heavy_chunks<0, 1>, (const void *)k_heavy_chunks<0, HEAVY_KB_MAX>,
                                        (const void *)k_heavy_chunks<1, 1>, (const void *)k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>,
                                        (const void *)k_heavy_local<0, 1, 4>, (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4>,
                                        (const void *)k_heavy_local<0, 1, 8>, (const void *)k_heavy_local<0, HEAVY_KB_MAX, 8>,
                                        (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>,
                                        (const void *)k_heavy_local<1, 1, 4>, (const void *)k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>};
-            for (const void *f : {(const void *)k_decode_csr_group<16>, (const void *)k_decode_csr_group<64>,
-                                  (const void *)k_decode_csr_group<BLOCK>})
-                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
             for (const void *f : heavy_fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
             (void)hipGetLastError();
         } catch (...) {
@@ -1784,42 +1677,14 @@ int lpa_set_graph_mode(lpa_engine *e, int on) {
 // tasks, task[j] of heavy set j.
 static void decode_range(lpa_engine *e, const uint64_t *words, uint32_t p0, uint32_t p1,
                          const std::vector<std::pair<uint32_t, uint32_t>> &tasks) {
-    for (const Bin &b : e->bins) {
+    std::vector<Bin> mine;
+    for (Bin b : e->bins) {
         if (b.csr) continue;
-        const uint32_t lo = std::max(b.begin, p0), hi = std::min(b.end, p1);
-        if (lo >= hi) continue;
-        const uint32_t count = hi - lo, logT = (uint32_t)b.param;
-        switch (b.kind) {
-        case LPA_BIN_LANE: {
-            const dim3 g((count + BLOCK - 1) / BLOCK);
-            auto lane = [&](auto fn) {
-                hipLaunchKernelGGL(fn, g, dim3(BLOCK), 0, e->stream, words, e->offs.p, e->vid.p, e->crow.p, e->ccol.p, lo, hi);
-            };
-            switch (b.param) {
-            case 4: lane(k_decode_csr<4>); break;
-            case 8: lane(k_decode_csr<8>); break;
-            case 16: lane(k_decode_csr<16>); break;
-            case 32: lane(k_decode_csr<32>); break;
-            default: lane(k_decode_csr<64>); break;
-            }
-            break;
-        }
-        case LPA_BIN_WAVE:
-        case LPA_BIN_BLOCK: {
-            const int ng = b.kind == LPA_BIN_BLOCK ? 1 : wave_groups(logT);
-            const dim3 g((count + ng - 1) / ng);
-            auto group = [&](auto fn) {
-                hipLaunchKernelGGL(fn, g, dim3(BLOCK), group_lds(ng, logT), e->stream, words, e->offs.p, e->vid.p,
-                                   e->meta.p, e->crow.p, e->ccol.p, lo, hi, logT);
-            };
-            if (ng == 1) group(k_decode_csr_group<BLOCK>);
-            else if (ng == 4) group(k_decode_csr_group<64>);
-            else group(k_decode_csr_group<16>);
-            break;
-        }
-        default: break;   // degree 0; heavy records follow
-        }
+        b.begin = std::max(b.begin, p0);
+        b.end = std::min(b.end, p1);
+        if (b.begin < b.end) mine.push_back(b);
     }
+    launch_decode_bins(mine, DecodeArgs{words, e->offs.p, e->vid.p, e->meta.p, e->crow.p, e->ccol.p}, e->stream);
     for (size_t j = 0; j < e->heavy.size(); j++) {
         if (e->heavy[j]->csr_part) continue;
         StepArgs a = e->base_args(false);
@@ -1902,13 +1767,10 @@ static void cglp_step(lpa_engine *e) {
 // CSR): CGLP's second kernel, and on its own the uncompressed comparator.
 static void csr_lp(lpa_engine *e) {
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
-    StepArgs a = e->base_args(false);
-    StepArgs ac = e->base_args(true);
-    for (const Bin &b : e->bins) {
-        if (b.kind == LPA_BIN_SKIP || b.kind == LPA_BIN_CMS || b.kind == LPA_BIN_GLOBAL) continue;
-        if (b.csr) e->launch_bin(b, a, true);
-        else e->launch_bin(b, ac, true);
-    }
+    std::vector<Bin> part[2];
+    for (const Bin &b : e->bins) part[b.csr].push_back(b);
+    launch_bins(part[0], e->base_args(true), true, e->sched_used.quarter_max, e->stream);
+    launch_bins(part[1], e->base_args(false), true, e->sched_used.quarter_max, e->stream);
     e->run_heavy(true, nullptr);
     HIPCHK(hipGetLastError());
 }

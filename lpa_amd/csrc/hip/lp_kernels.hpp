@@ -188,19 +188,32 @@ __device__ __forceinline__ bool stage_records(const uint64_t *__restrict__ words
 // gather neighbour u's labels for consecutive vectors read consecutive
 // words of u's label row in one access.  Each lane sorts its pair's labels
 // with a bitonic network and takes the longest run.
-template <int N, bool CSR>
-__global__ void __launch_bounds__(BLOCK) k_lane(StepArgs a) {
+template <int N, bool CSR> struct LaneShared {
     // CSR rows follow the layout back to back, so the block's rows are one
     // range of nbr: the workgroup copies it to LDS with coalesced loads
     // instead of every lane walking its own row (N <= 32: at most 32 KB)
-    constexpr bool STAGE = CSR && N <= 32;
-    __shared__ uint32_t list[CSR ? 1 : N][BLOCK];
-    __shared__ uint32_t rows[STAGE ? N * BLOCK : 1];
-    __shared__ uint32_t sv[BLOCK], sd[BLOCK];
-    __shared__ uint64_t sbase[CSR ? BLOCK : 1];
-    constexpr uint32_t SW = lane_stage_words<N>();
-    __shared__ uint64_t sw[CSR ? 1 : SW + 3];   // a dummy before, look-ahead after
-    const uint32_t first = a.begin + xcd_tile(blockIdx.x, gridDim.x, a.xcds) * BLOCK;
+    static constexpr bool STAGE = CSR && N <= 32;
+    static constexpr uint32_t SW = lane_stage_words<N>();
+    uint64_t sw[CSR ? 1 : SW + 3];   // staged stream words: a dummy before, look-ahead after
+    uint64_t sbase[CSR ? BLOCK : 1];
+    uint32_t list[CSR ? 1 : N][BLOCK];
+    uint32_t rows[STAGE ? N * BLOCK : 1];
+    uint32_t sv[BLOCK], sd[BLOCK];
+};
+
+// One workgroup of the lane family: tile `tile` (256 vertices) of the bin
+// [a.begin, a.end).
+template <int N, bool CSR>
+__device__ __forceinline__ void lane_tile(const StepArgs &a, uint32_t tile, LaneShared<N, CSR> &sh) {
+    constexpr bool STAGE = LaneShared<N, CSR>::STAGE;
+    constexpr uint32_t SW = LaneShared<N, CSR>::SW;
+    auto &list = sh.list;
+    auto &rows = sh.rows;
+    auto &sv = sh.sv;
+    auto &sd = sh.sd;
+    auto &sbase = sh.sbase;
+    auto &sw = sh.sw;
+    const uint32_t first = a.begin + tile * BLOCK;
     const uint32_t p = first + threadIdx.x;
     const uint32_t nact = a.end - first < (uint32_t)BLOCK ? a.end - first : (uint32_t)BLOCK;
     const uint64_t t0 = a.rec ? cycles() : 0;
@@ -313,6 +326,11 @@ __global__ void __launch_bounds__(BLOCK) k_lane(StepArgs a) {
         }
     }
     flush_changes(nch, a.changed);
+}
+
+template <int N, bool CSR> __global__ void __launch_bounds__(BLOCK) k_lane(StepArgs a) {
+    __shared__ LaneShared<N, CSR> sh;
+    lane_tile<N, CSR>(a, xcd_tile(blockIdx.x, gridDim.x, a.xcds), sh);
 }
 
 // ------------------------------------------------------------ group kernels
@@ -680,21 +698,28 @@ __device__ __forceinline__ void count_staged(const StepArgs &a, const uint32_t *
 // staged in registers, IPL neighbours per lane (the launch picks the
 // smallest IPL with IPL * G >= listcap, so the staged labels, IPL * KB
 // registers, cost no more occupancy than the bin needs).
+template <int G, int KB> struct GroupStatic {
+    uint64_t red[BLOCK / 64];
+    uint32_t xw[G > 64 ? KB * (G / 64) : 1], xs[KB];
+    GroupShared<G> gsh[BLOCK / G];
+};
+
+// Workgroup `tile` of `tiles` over the bin [a.begin, a.end).
 template <int G, bool CSR, int KB, int IPL>
-__global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint32_t listcap) {
+__device__ __forceinline__ void group_tile(const StepArgs &a, uint32_t logT, uint32_t listcap, uint32_t tile,
+                                           uint32_t tiles, uint64_t *lds, GroupStatic<G, KB> &st) {
     constexpr int NG = BLOCK / G;
-    extern __shared__ uint64_t lds[];
-    __shared__ uint64_t red[BLOCK / 64];
-    __shared__ uint32_t xw[G > 64 ? KB * (G / 64) : 1], xs[KB];
-    __shared__ GroupShared<G> gsh[NG];
+    auto &red = st.red;
+    auto &xw = st.xw;
+    auto &xs = st.xs;
     const uint32_t gid = threadIdx.x / G, gl = threadIdx.x % G;
     const uint32_t T = 1u << logT;
     uint64_t *tab = lds + (uint64_t)gid * (T + (listcap + 1) / 2);
     uint32_t *list = (uint32_t *)(tab + T);
-    GroupShared<G> *sh = &gsh[gid];
-    const uint32_t stride = gridDim.x * NG;
+    GroupShared<G> *sh = &st.gsh[gid];
+    const uint32_t stride = tiles * NG;
     uint32_t nch = 0;
-    for (uint32_t p0 = a.begin + xcd_tile(blockIdx.x, gridDim.x, a.xcds) * NG; p0 < a.end; p0 += stride) {
+    for (uint32_t p0 = a.begin + tile * NG; p0 < a.end; p0 += stride) {
         // all groups of a wave (or workgroup) run the same trip count
         const uint32_t p = p0 + gid;
         const bool live = p < a.end;
@@ -765,42 +790,119 @@ __global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint
     flush_changes(nch, a.changed);
 }
 
+template <int G, bool CSR, int KB, int IPL>
+__global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint32_t listcap) {
+    extern __shared__ uint64_t lds[];
+    __shared__ GroupStatic<G, KB> st;
+    group_tile<G, CSR, KB, IPL>(a, logT, listcap, xcd_tile(blockIdx.x, gridDim.x, a.xcds), gridDim.x, lds, st);
+}
+
+// --------------------------------------------------------- several bins at once
+
+// Bins of one step that share a launch (k_bins).
+// BC_LANE64 only decodes to a CSR here.
+enum BinCode : uint32_t { BC_LANE4, BC_LANE8, BC_LANE16, BC_LANE32, BC_LANE64, BC_G16, BC_G32, BC_G64, BC_G256 };
+struct BinTable {
+    static constexpr uint32_t MAX = 12;
+    struct Entry {
+        uint32_t first;        // first workgroup of the bin
+        uint32_t begin, end;   // its positions
+        uint32_t code;         // BinCode
+        uint32_t csr, logT;
+    } e[MAX];
+    uint32_t n;
+};
+
+// Staged ids per lane of a merged bin: those of the separate launch when
+// their number changes the registers (several vectors), else 8.
+template <int G, bool CSR, int KB>
+__device__ __forceinline__ void group_bin(const StepArgs &a, const BinTable::Entry &e, uint32_t tile, uint32_t tiles,
+                                          uint64_t *lds) {
+    auto &st = *reinterpret_cast<GroupStatic<G, KB> *>(lds);
+    uint64_t *dyn = lds + (sizeof(GroupStatic<G, KB>) + 7) / 8;
+    const uint32_t cap = 1u << (e.logT - 1), ipl = (cap + G - 1) / G;
+    if (KB >= 4 && G != 32 && ipl <= 2) group_tile<G, CSR, KB, (KB >= 4 ? 2 : 8)>(a, e.logT, cap, tile, tiles, dyn, st);
+    else if (KB >= 4 && (G == 32 || ipl <= 4)) group_tile<G, CSR, KB, (KB >= 4 ? 4 : 8)>(a, e.logT, cap, tile, tiles, dyn, st);
+    else group_tile<G, CSR, KB, 8>(a, e.logT, cap, tile, tiles, dyn, st);
+}
+
+template <int KB, bool CSR>
+__device__ __forceinline__ void one_bin(const StepArgs &a, const BinTable::Entry &e, uint32_t tile, uint32_t tiles,
+                                        uint64_t *lds) {
+    switch (e.code) {
+    case BC_LANE4: lane_tile<4, CSR>(a, tile, *reinterpret_cast<LaneShared<4, CSR> *>(lds)); break;
+    case BC_LANE8: lane_tile<8, CSR>(a, tile, *reinterpret_cast<LaneShared<8, CSR> *>(lds)); break;
+    case BC_LANE16: lane_tile<16, CSR>(a, tile, *reinterpret_cast<LaneShared<16, CSR> *>(lds)); break;
+    case BC_LANE32: lane_tile<32, CSR>(a, tile, *reinterpret_cast<LaneShared<32, CSR> *>(lds)); break;
+    case BC_G16: group_bin<16, CSR, KB>(a, e, tile, tiles, lds); break;
+    case BC_G32:
+        if (KB == 8) group_bin<32, CSR, KB>(a, e, tile, tiles, lds);
+        break;
+    case BC_G64: group_bin<64, CSR, KB>(a, e, tile, tiles, lds); break;
+    default: group_bin<BLOCK, CSR, KB>(a, e, tile, tiles, lds); break;
+    }
+}
+
+// The workgroups of several bins in one launch, each doing what its bin's own
+// kernel would.  A launch costs 5.5 us in a stream whatever it does, and a
+// bin of few workgroups leaves most of the device idle until its last one is
+// done; registers and LDS are those of the most demanding bin, so bins that
+// fill the device by themselves keep their own launch.
+template <int KB> __global__ void __launch_bounds__(BLOCK) k_bins(StepArgs a, BinTable t) {
+    extern __shared__ uint64_t lds[];
+    uint32_t i = 0;
+    while (i + 1 < t.n && blockIdx.x >= t.e[i + 1].first) i++;
+    const BinTable::Entry e = t.e[i];
+    const uint32_t tiles = (i + 1 < t.n ? t.e[i + 1].first : gridDim.x) - e.first;
+    a.begin = e.begin;
+    a.end = e.end;
+    if (e.csr) one_bin<KB, true>(a, e, blockIdx.x - e.first, tiles, lds);
+    else one_bin<KB, false>(a, e, blockIdx.x - e.first, tiles, lds);
+}
+
 // --------------------------------------------------------- CGLP kernel 1
 
 // Decode the records of positions [begin,end), of at most N ids each, into
 // CSR rows crow[p]..crow[p+1] (rows follow the device layout, so a
 // workgroup's 256 rows are one range of ccol); one lane per record, ids
 // assembled in LDS and stored with coalesced stores.
+struct DecodeArgs {
+    const uint64_t *__restrict__ words;
+    const uint64_t *__restrict__ offs;
+    const uint32_t *__restrict__ vid;
+    const uint4 *__restrict__ meta;
+    const uint64_t *__restrict__ crow;
+    uint32_t *__restrict__ ccol;
+};
+template <int N> struct LaneDecodeShared {
+    uint64_t sw[lane_stage_words<N>() + 3];
+    uint32_t out[N * BLOCK];
+};
 template <int N>
-__global__ void __launch_bounds__(BLOCK) k_decode_csr(const uint64_t *__restrict__ words,
-                                                      const uint64_t *__restrict__ offs,
-                                                      const uint32_t *__restrict__ vid,
-                                                      const uint64_t *__restrict__ crow,
-                                                      uint32_t *__restrict__ ccol, uint32_t begin, uint32_t end) {
+__device__ __forceinline__ void lane_decode_tile(const DecodeArgs &a, uint32_t begin, uint32_t end, uint32_t tile,
+                                                 LaneDecodeShared<N> &sh) {
     constexpr uint32_t SW = lane_stage_words<N>();
-    __shared__ uint64_t sw[SW + 3];
-    __shared__ uint32_t out[N * BLOCK];
-    const uint32_t first = begin + blockIdx.x * BLOCK, p = first + threadIdx.x;
+    const uint32_t first = begin + tile * BLOCK, p = first + threadIdx.x;
     const uint32_t cnt = end - first < (uint32_t)BLOCK ? end - first : (uint32_t)BLOCK;
     WinReader<false> r{};
-    r.w = reinterpret_cast<const uint32_t *>(sw);
-    const bool staged = stage_records<SW>(words, offs, first, cnt, sw, r.base);
-    const uint64_t o0 = crow[first];
+    r.w = reinterpret_cast<const uint32_t *>(sh.sw);
+    const bool staged = stage_records<SW>(a.words, a.offs, first, cnt, sh.sw, r.base);
+    const uint64_t o0 = a.crow[first];
     __syncthreads();
     if (p < end) {
-        const uint32_t v = vid[p];
-        uint32_t o = (uint32_t)(crow[p] - o0);
-        auto put = [&](uint32_t u) { out[o++] = u; };
+        const uint32_t v = a.vid[p];
+        uint32_t o = (uint32_t)(a.crow[p] - o0);
+        auto put = [&](uint32_t u) { sh.out[o++] = u; };
         if (staged) {
-            r.set(offs[p]);
+            r.set(a.offs[p]);
             read_record(r, v, put);
         } else {
-            decode_record(words, offs[p], v, put);
+            decode_record(a.words, a.offs[p], v, put);
         }
     }
     __syncthreads();
-    const uint32_t tot = (uint32_t)(crow[first + cnt] - o0);
-    for (uint32_t x = threadIdx.x; x < tot; x += BLOCK) ccol[o0 + x] = out[x];
+    const uint32_t tot = (uint32_t)(a.crow[first + cnt] - o0);
+    for (uint32_t x = threadIdx.x; x < tot; x += BLOCK) a.ccol[o0 + x] = sh.out[x];
 }
 
 // Exclusive sum of x over the group's lanes (every lane calls it), and the
@@ -833,30 +935,27 @@ __device__ __forceinline__ uint32_t group_scan(uint32_t x, uint32_t *xs, uint32_
 // ids' places follow from the segments' counts, so the rows keep the encoded
 // order; assembled in LDS, stored with coalesced stores.  Dynamic LDS per
 // group as in k_group.
+template <int G> struct GroupDecodeStatic {
+    GroupShared<G> gsh[BLOCK / G];
+    uint32_t xs[BLOCK / 64];
+};
 template <int G>
-__global__ void __launch_bounds__(BLOCK) k_decode_csr_group(const uint64_t *__restrict__ words,
-                                                            const uint64_t *__restrict__ offs,
-                                                            const uint32_t *__restrict__ vid,
-                                                            const uint4 *__restrict__ meta,
-                                                            const uint64_t *__restrict__ crow,
-                                                            uint32_t *__restrict__ ccol, uint32_t begin,
-                                                            uint32_t end, uint32_t logT) {
+__device__ __forceinline__ void group_decode_tile(const DecodeArgs &a, uint32_t begin, uint32_t end, uint32_t logT,
+                                                  uint32_t tile, uint64_t *lds, GroupDecodeStatic<G> &st) {
     constexpr int NG = BLOCK / G;
-    extern __shared__ uint64_t lds[];
-    __shared__ GroupShared<G> gsh[NG];
-    __shared__ uint32_t xs[BLOCK / 64];
+    uint32_t *xs = st.xs;
     const uint32_t gid = threadIdx.x / G, gl = threadIdx.x % G, T = 1u << logT;
     uint64_t *stage = lds + (uint64_t)gid * (T + T / 4);
     uint32_t *list = (uint32_t *)(stage + T);
-    GroupShared<G> *sh = &gsh[gid];
-    const uint32_t p = begin + blockIdx.x * NG + gid;
+    GroupShared<G> *sh = &st.gsh[gid];
+    const uint32_t p = begin + tile * NG + gid;
     if (p >= end) return;   // whole groups; a workgroup of one group is never empty
-    const uint32_t v = vid[p];
-    const uint64_t start = offs[p], o0 = crow[p];
-    const uint32_t d = (uint32_t)(crow[p + 1] - o0);
-    const uint4 m = meta[p];
+    const uint32_t v = a.vid[p];
+    const uint64_t start = a.offs[p], o0 = a.crow[p];
+    const uint32_t d = (uint32_t)(a.crow[p + 1] - o0);
+    const uint4 m = a.meta[p];
     if (gl == 0) sh->qn = 0;
-    with_record<G>(words, start, offs[p + 1], gl, stage, T, [&](auto &&at) {
+    with_record<G>(a.words, start, a.offs[p + 1], gl, stage, T, [&](auto &&at) {
         uint32_t done = 0, total;
         for (uint32_t j0 = 0; j0 < m.y; j0 += G) {
             const uint32_t j = j0 + gl;
@@ -887,7 +986,25 @@ __global__ void __launch_bounds__(BLOCK) k_decode_csr_group(const uint64_t *__re
     group_sync<G>();
     write_long_runs<G>(sh, gl, list);
     group_sync<G>();
-    for (uint32_t x = gl; x < d; x += G) ccol[o0 + x] = list[x];
+    for (uint32_t x = gl; x < d; x += G) a.ccol[o0 + x] = list[x];
+}
+
+// Workgroup `tile` of a bin's records.
+__device__ __forceinline__ void decode_bin(const DecodeArgs &a, const BinTable::Entry &e, uint32_t tile, uint64_t *lds) {
+    auto lane = [&](auto *sh) { lane_decode_tile(a, e.begin, e.end, tile, *sh); };
+    auto group = [&](auto *st) {
+        group_decode_tile(a, e.begin, e.end, e.logT, tile, lds + (sizeof(*st) + 7) / 8, *st);
+    };
+    switch (e.code) {
+    case BC_LANE4: lane(reinterpret_cast<LaneDecodeShared<4> *>(lds)); break;
+    case BC_LANE8: lane(reinterpret_cast<LaneDecodeShared<8> *>(lds)); break;
+    case BC_LANE16: lane(reinterpret_cast<LaneDecodeShared<16> *>(lds)); break;
+    case BC_LANE32: lane(reinterpret_cast<LaneDecodeShared<32> *>(lds)); break;
+    case BC_LANE64: lane(reinterpret_cast<LaneDecodeShared<64> *>(lds)); break;
+    case BC_G16: group(reinterpret_cast<GroupDecodeStatic<16> *>(lds)); break;
+    case BC_G64: group(reinterpret_cast<GroupDecodeStatic<64> *>(lds)); break;
+    default: group(reinterpret_cast<GroupDecodeStatic<BLOCK> *>(lds)); break;
+    }
 }
 
 }  // namespace lpa
