@@ -1151,6 +1151,7 @@ static void build_heavy(lpa_engine *e) {
                         DecodeTask t{};
                         t.ibase = start + hm[i].x;
                         t.rbase = start + hm[i].z;
+                        t.end = e->h_loffs[q + 1];
                         t.v = e->h_vertices[e->order_c[q]];
                         t.j0 = j0;
                         t.ni = hm[i].y;

@@ -126,6 +126,7 @@ __device__ __forceinline__ uint32_t heavy_deg(const HeavyArgs &h, uint32_t i) {
 // the order of a list is irrelevant to the counts).
 struct DecodeTask {
     uint64_t ibase, rbase;   // absolute bit of interval segment 0 / residual segment 0
+    uint64_t end;            // bit after the record
     uint64_t out;            // first list slot of the task's ids
     uint32_t v, j0, ni, ns;  // vertex, first segment, #interval segments, #segments
     uint32_t count, h;       // ids the task writes; index of its heavy vertex
@@ -164,71 +165,75 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_task_count(StepArgs a, DecodeTa
 // residual segment; the task's ids are assembled in LDS and stored to the list
 // with coalesced stores, or written in place when they exceed the staging
 // buffer.  With crow the ids go to the heavy vertex's row of the decoded CSR
-// ccol instead.
+// ccol instead.  Bound by the longest lane: a dense residual segment holds
+// about 60 codes, the merged last one up to twice that.  Per step: R-MAT 20 104 -> 71
+// us (both heavy sets), a copying graph's 60 hubs 152 -> 53 us, R-MAT 12 32 ->
+// 26 us, against words read in place, long runs written one after another
+// and the claims turned into loops over the lanes.
 // CMS: the heavy set's mode (names the launch in profiles; same code)
-constexpr uint32_t TASK_WORDS = BLOCK * SEG_BITS / 64;   // 64-bit words of a task's segments
-constexpr uint32_t TASK_AHEAD = 8;   // words staged from the last segment's first (the stream is
-                                     // padded by as many): most of a merged last segment
+constexpr uint32_t TASK_WORDS = BLOCK * SEG_BITS / 64 + 32;   // 64-bit words staged: a task's segments, the
+                                                              // merged last ones' tails, dummies and look-ahead
 template <int CMS>
 __global__ void __launch_bounds__(BLOCK) k_heavy_decode(HeavyArgs h, const DecodeTask *__restrict__ tasks,
                                                         uint32_t ntasks, const uint64_t *__restrict__ crow,
                                                         uint32_t *__restrict__ ccol) {
     __shared__ GroupShared<BLOCK> sh;
     __shared__ uint32_t stage[DECODE_STAGE];
-    __shared__ uint64_t sw[TASK_WORDS + 2 * (TASK_AHEAD + 1)];
+    __shared__ uint64_t sw[TASK_WORDS];
     const uint32_t t = blockIdx.x;
     if (t >= ntasks || h.csr) return;
     const uint64_t t0 = h.s.rec ? cycles() : 0;
     const DecodeTask T = tasks[t];
     const uint64_t *__restrict__ W = h.s.words;
-    if (threadIdx.x == 0) {
-        sh.cnt = 0;
-        sh.qn = 0;
-    }
-    // segments [j0, j1) of the record; those below ni are interval segments
+    if (threadIdx.x == 0) clear_runs(&sh);
+    // segments [j0, j1) of the record; those below ni are interval segments.
+    // Each block's share is one range of words: up to the next segment, or
+    // to the block's end behind its last segment.
     const uint32_t j1 = T.ns - T.j0 < (uint32_t)BLOCK ? T.ns : T.j0 + BLOCK;
     const uint32_t i1 = j1 < T.ni ? j1 : T.ni, r0 = T.j0 < T.ni ? T.ni : T.j0;
-    // words of segments [a, b) of the block at bit `at`, behind one dummy word
-    auto stage_range = [&](uint64_t at, uint32_t a, uint32_t b, uint64_t *to, uint64_t &base) -> uint32_t {
-        base = (at + (uint64_t)SEG_BITS * a) >> 6;
-        if (b <= a) return 0;
-        const uint32_t nw = (uint32_t)(((at + (uint64_t)SEG_BITS * (b - 1)) >> 6) - base) + TASK_AHEAD;
-        for (uint32_t i = threadIdx.x; i < nw; i += BLOCK) to[i + 1] = staged_pair(W[base + i]);
-        return nw + 1;
-    };
-    uint64_t ib, rb;
-    const uint32_t iw = stage_range(T.ibase, T.j0, i1, sw, ib);
-    const uint32_t rw = stage_range(T.rbase, r0 - T.ni, j1 > r0 ? j1 - T.ni : r0 - T.ni, sw + iw, rb);
+    const uint64_t ia = T.ibase + (uint64_t)SEG_BITS * T.j0, ra = T.rbase + (uint64_t)SEG_BITS * (r0 - T.ni);
+    const uint64_t ie = T.j0 >= T.ni ? ia : i1 == T.ni ? T.rbase : T.ibase + (uint64_t)SEG_BITS * i1;
+    const uint64_t re = j1 <= r0 ? ra : j1 == T.ns ? T.end : T.rbase + (uint64_t)SEG_BITS * (j1 - T.ni);
+    const uint64_t iw = ie > ia ? ((ie + 63) >> 6) - (ia >> 6) : 0, rw = re > ra ? ((re + 63) >> 6) - (ra >> 6) : 0;
+    const bool words_staged = iw + rw + 6 <= TASK_WORDS;   // a dummy before and look-ahead after each
+    uint64_t *si = sw, *sr = sw + iw + 3;
+    if (words_staged) {
+        for (uint32_t i = threadIdx.x; i < iw; i += BLOCK) si[i + 1] = staged_pair(W[(ia >> 6) + i]);
+        for (uint32_t i = threadIdx.x; i < rw; i += BLOCK) sr[i + 1] = staged_pair(W[(ra >> 6) + i]);
+    }
     __syncthreads();
-    const bool staged = T.count <= DECODE_STAGE;
     uint32_t *out = crow ? ccol + crow[h.pos[T.h]] + (T.out - h.loff[T.h]) : h.list + T.out;
     const uint32_t j = T.j0 + threadIdx.x;
+    auto segment = [&](auto &r, uint32_t *dst) {   // the reader stands at segment j
+        if (j < T.ni) {
+            read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
+                put_run<BLOCK>(&sh, dst, atomicAdd(&sh.cnt, len), l, len);
+            });
+        } else {
+            const uint32_t c = r.gamma();   // claims the segment's slots
+            uint32_t o = atomicAdd(&sh.cnt, c);
+            read_residual_ids(r, T.v, c, [&](uint32_t u) { dst[o++] = u; });
+        }
+    };
+    const uint64_t at = j < T.ni ? T.ibase + (uint64_t)SEG_BITS * j : T.rbase + (uint64_t)SEG_BITS * (j - T.ni);
     auto decode = [&](uint32_t *dst) {
         if (j < j1) {
-            WinReader<true> r{};
-            r.W = W;
-            if (j < T.ni) {
-                r.w = reinterpret_cast<const uint32_t *>(sw);
-                r.lim = 2 * iw;
-                r.base = ib;
-                r.set(T.ibase + (uint64_t)SEG_BITS * j);
-                read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
-                    put_run<BLOCK>(&sh, dst, atomicAdd(&sh.cnt, len), l, len);
-                });
+            if (words_staged) {
+                WinReader<false> r{};
+                r.w = reinterpret_cast<const uint32_t *>(j < T.ni ? si : sr);
+                r.base = (j < T.ni ? ia : ra) >> 6;
+                r.set(at);
+                segment(r, dst);
             } else {
-                r.w = reinterpret_cast<const uint32_t *>(sw + iw);
-                r.lim = 2 * rw;
-                r.base = rb;
-                r.set(T.rbase + (uint64_t)SEG_BITS * (j - T.ni));
-                const uint32_t c = r.gamma();   // claims the segment's slots
-                uint32_t o = atomicAdd(&sh.cnt, c);
-                read_residual_ids(r, T.v, c, [&](uint32_t u) { dst[o++] = u; });
+                BitReader r;
+                r.seek(W, at);
+                segment(r, dst);
             }
         }
         __syncthreads();
         write_long_runs<BLOCK>(&sh, threadIdx.x, dst);
     };
-    if (staged) {   // two instances: LDS stores in one, global stores in the other
+    if (T.count <= DECODE_STAGE) {   // two instances: LDS stores in one, global stores in the other
         decode(stage);
         __syncthreads();
         for (uint32_t x = threadIdx.x; x < T.count; x += BLOCK) out[x] = stage[x];

@@ -406,16 +406,18 @@ __device__ __forceinline__ uint32_t cms_col(const StepArgs &a, uint32_t r, uint3
     return a.cms_logw ? (uint32_t)(h >> (64 - a.cms_logw)) : 0;
 }
 
-// Intervals at least this long are written by the whole group.
-constexpr uint32_t LONG_RUN = 16;
+// Intervals at least this long are written by 16 lanes together, or by the
+// whole group.
+constexpr uint32_t LONG_RUN = 16, HUGE_RUN = 512;
 
 template <int G> struct GroupShared {
     static constexpr int QCAP = G == BLOCK ? 512 : G == 64 ? 64 : G == 32 ? 32 : 16;
+    static constexpr int HCAP = 8;
     uint32_t cnt;                 // ids written to the list so far
-    uint32_t qn;
-    uint32_t qleft[QCAP];
-    uint32_t qlen[QCAP];
-    uint32_t qpos[QCAP];
+    uint32_t qn, hn;
+    uint32_t qleft[QCAP + HCAP];  // long runs, then huge ones from QCAP on
+    uint32_t qlen[QCAP + HCAP];
+    uint32_t qpos[QCAP + HCAP];
 };
 
 // The record of position p staged in `stage` (cap 64-bit words) by its group,
@@ -446,11 +448,26 @@ __device__ __forceinline__ void with_record(const uint64_t *__restrict__ words, 
     }
 }
 
-// Runs of LONG_RUN or more ids queued by the lanes, written by the group.
+// Empties the group's counters (one lane; the caller synchronises).
+template <int G> __device__ __forceinline__ void clear_runs(GroupShared<G> *sh) {
+    sh->cnt = 0;
+    sh->qn = 0;
+    sh->hn = 0;
+}
+
+// Runs of LONG_RUN or more ids queued by the lanes, written by the group: 16
+// lanes per run (a hub of short runs has hundreds of them: one after another
+// by the whole group they took 43 us of a 152 us decode of a copying graph's
+// hubs), the huge ones by all lanes.
 template <int G>
 __device__ __forceinline__ void write_long_runs(const GroupShared<G> *sh, uint32_t gl, uint32_t *list) {
-    const uint32_t nq = sh->qn < (uint32_t)GroupShared<G>::QCAP ? sh->qn : (uint32_t)GroupShared<G>::QCAP;
-    for (uint32_t q = 0; q < nq; q++) {
+    constexpr uint32_t QCAP = GroupShared<G>::QCAP, HCAP = GroupShared<G>::HCAP;
+    const uint32_t nq = sh->qn < QCAP ? sh->qn : QCAP, nh = sh->hn < HCAP ? sh->hn : HCAP;
+    for (uint32_t q = gl / 16; q < nq; q += G / 16) {
+        const uint32_t l = sh->qleft[q], len = sh->qlen[q], o = sh->qpos[q];
+        for (uint32_t x = gl & 15; x < len; x += 16) list[o + x] = l + x;
+    }
+    for (uint32_t q = QCAP; q < QCAP + nh; q++) {
         const uint32_t l = sh->qleft[q], len = sh->qlen[q], o = sh->qpos[q];
         for (uint32_t x = gl; x < len; x += G) list[o + x] = l + x;
     }
@@ -461,8 +478,17 @@ __device__ __forceinline__ void write_long_runs(const GroupShared<G> *sh, uint32
 template <int G>
 __device__ __forceinline__ void put_run(GroupShared<G> *sh, uint32_t *list, uint32_t o, uint32_t l, uint32_t len) {
     if (len >= LONG_RUN) {
-        const uint32_t q = atomicAdd(&sh->qn, 1u);
-        if (q < (uint32_t)GroupShared<G>::QCAP) {
+        constexpr uint32_t QCAP = GroupShared<G>::QCAP, HCAP = GroupShared<G>::HCAP;
+        uint32_t q = QCAP + HCAP;
+        if (len >= HUGE_RUN) {
+            q = atomicAdd(&sh->hn, 1u);
+            q = q < HCAP ? QCAP + q : QCAP + HCAP;
+        }
+        if (q == QCAP + HCAP) {
+            q = atomicAdd(&sh->qn, 1u);
+            q = q < QCAP ? q : QCAP + HCAP;
+        }
+        if (q < QCAP + HCAP) {
             sh->qleft[q] = l;
             sh->qlen[q] = len;
             sh->qpos[q] = o;
@@ -485,10 +511,7 @@ __device__ __forceinline__ void put_run(GroupShared<G> *sh, uint32_t *list, uint
 template <int G>
 __device__ __forceinline__ uint32_t group_decode(const StepArgs &a, uint32_t p, uint32_t v, uint32_t gl,
                                                  GroupShared<G> *sh, uint32_t *list, uint64_t *stage, uint32_t cap) {
-    if (gl == 0) {
-        sh->cnt = 0;
-        sh->qn = 0;
-    }
+    if (gl == 0) clear_runs(sh);
     // segment j of the record (intervals first, then residuals) is at a
     // position known from the metadata: every lane seeks its own segment
     const uint64_t start = a.offs[p];
@@ -954,7 +977,7 @@ __device__ __forceinline__ void group_decode_tile(const DecodeArgs &a, uint32_t 
     const uint64_t start = a.offs[p], o0 = a.crow[p];
     const uint32_t d = (uint32_t)(a.crow[p + 1] - o0);
     const uint4 m = a.meta[p];
-    if (gl == 0) sh->qn = 0;
+    if (gl == 0) clear_runs(sh);
     with_record<G>(a.words, start, a.offs[p + 1], gl, stage, T, [&](auto &&at) {
         uint32_t done = 0, total;
         for (uint32_t j0 = 0; j0 < m.y; j0 += G) {
