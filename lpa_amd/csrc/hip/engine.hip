@@ -242,8 +242,17 @@ struct lpa_engine {
     DevBuf<uint32_t> L[2];
     int cur = 0;
     bool have_labels = false;
+    // changed labels of a step, one count per stream it uses; h_counter:
+    // their host copies (pinned)
+    static constexpr int LANES = 3;
     DevBuf<unsigned long long> counter;
-    unsigned long long *h_counter = nullptr;   // pinned
+    unsigned long long *h_counter = nullptr;
+    bool counts_clean = false;                 // the device counts are 0
+    DevBuf<unsigned long long> err;            // graph validation: 1 + the first malformed record
+    // side streams: the heavy sets of an eager step run there beside the
+    // bins (spread), see spread_step
+    hipStream_t side[LANES - 1] = {};
+    bool spread = false;
 
     // CGLP
     DevBuf<uint64_t> crow;
@@ -287,12 +296,19 @@ struct lpa_engine {
         for (hipEvent_t x : {ev_copied[0], ev_copied[1], ev_free[0], ev_free[1]})
             if (x) (void)hipEventDestroy(x);
         if (copy_stream) (void)hipStreamDestroy(copy_stream);
+        for (hipStream_t x : side)
+            if (x) (void)hipStreamDestroy(x);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
     void sync() { HIPCHK(hipStreamSynchronize(stream)); }
 
-    StepArgs base_args(bool cglp) const {
+    // stream `lane` of a step (0: the engine stream), and the lane of heavy
+    // set j
+    hipStream_t lane_stream(int lane) const { return lane ? side[lane - 1] : stream; }
+    int heavy_lane(size_t j) const { return spread ? 1 + (int)(j % (LANES - 1)) : 0; }
+
+    StepArgs base_args(bool cglp, int lane = 0) const {
         StepArgs a{};
         a.words = words.p;
         a.offs = offs.p;
@@ -312,15 +328,19 @@ struct lpa_engine {
         a.cms_depth = cms_depth;
         a.cms_logw = ceil_log2(cms_width);
         std::memcpy(a.cms_ab, cms_ab, sizeof cms_ab);
-        a.changed = counter.p;
+        a.changed = counter.p + lane;
         a.rec = rec;
         a.xcds = sched_used.xcd_tiles == 1 ? XCDS : 1;
         return a;
     }
 
     HeavyArgs heavy_args(const HeavySet &hs, const StepArgs &a, bool as_csr) const;
-    void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, bool to_csr = false);
-    void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool decode = true);
+    void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, hipStream_t s,
+                             bool to_csr = false);
+    void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipStream_t s, bool decode = true);
+    bool spread_step(int method) const;
+    void begin_step(bool side_streams);
+    uint64_t end_step();
     template <class F> void for_each_batch(F &&fn);
     void step_host_stream();
     void step(bool cglp, hipEvent_t *launch_events);
@@ -387,23 +407,24 @@ HeavyArgs lpa_engine::heavy_args(const HeavySet &hs, const StepArgs &a, bool as_
 
 // Decode tasks [t0, t1) of a heavy set (compressed part) into its lists, or
 // into their rows of the decoded CSR.
-void lpa_engine::launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, bool to_csr) {
+void lpa_engine::launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, hipStream_t s,
+                                     bool to_csr) {
     if (t1 <= t0) return;
     const HeavyArgs h = heavy_args(hs, a, false);
     const uint64_t *row = to_csr ? crow.p : nullptr;
     uint32_t *col = to_csr ? ccol.p : nullptr;
-    if (hs.cms) hipLaunchKernelGGL(k_heavy_decode<1>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0, row, col);
-    else hipLaunchKernelGGL(k_heavy_decode<0>, dim3(t1 - t0), dim3(BLOCK), 0, stream, h, hs.tasks.p + t0, t1 - t0, row, col);
+    if (hs.cms) hipLaunchKernelGGL(k_heavy_decode<1>, dim3(t1 - t0), dim3(BLOCK), 0, s, h, hs.tasks.p + t0, t1 - t0, row, col);
+    else hipLaunchKernelGGL(k_heavy_decode<0>, dim3(t1 - t0), dim3(BLOCK), 0, s, h, hs.tasks.p + t0, t1 - t0, row, col);
 }
 
 // A heavy set's step: decode its records into the lists (unless `decode` is
 // off: a host-resident stream decodes them batch by batch), then count.
-void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool decode) {
+void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipStream_t s, bool decode) {
     if (hs.nh == 0) return;
     HeavyArgs h = heavy_args(hs, a, as_csr);
     const bool one = K == 1;
     const size_t cells = (size_t)cms_depth * cms_width;
-    if (!as_csr && decode) launch_heavy_decode(hs, a, 0, hs.ntasks);
+    if (!as_csr && decode) launch_heavy_decode(hs, a, 0, hs.ntasks, s);
     if (hs.nlocal) {
         const dim3 b(HBLOCK);
         const size_t sk = cms_local_lds(h.kbl, cells);
@@ -414,8 +435,8 @@ void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool
             h.stash = hs.stash.p;
             h.stash_stride = (uint64_t)CMS_LOCAL * (one ? 1 : HEAVY_KB_CMS_LOCAL);
             const dim3 g(std::min(hs.nlocal, hs.stash_blocks));
-            if (one) hipLaunchKernelGGL((k_heavy_local<1, 1, 4>), g, b, sk, stream, h, hs.local.p, hs.nlocal);
-            else hipLaunchKernelGGL((k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>), g, b, sk, stream, h, hs.local.p, hs.nlocal);
+            if (one) hipLaunchKernelGGL((k_heavy_local<1, 1, 4>), g, b, sk, s, h, hs.local.p, hs.nlocal);
+            else hipLaunchKernelGGL((k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>), g, b, sk, s, h, hs.local.p, hs.nlocal);
         } else {
             // tables of up to 2*CHUNK (8192 ids: 4 per lane) or 4*CHUNK slots (8 per lane);
             // with a row stash, resident workgroups take the vertices one by one
@@ -425,15 +446,15 @@ void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool
                 h.stash_stride = (uint64_t)CHUNK * row_stash_k(this);
                 h.wq = hs.wq.p;
                 const dim3 g(hs.rstash_small ? hs.rstash_small : nsmall);
-                if (one) hipLaunchKernelGGL((k_heavy_local<0, 1, 4>), g, b, t1, stream, h, lsmall, nsmall);
-                else if (h.stash) hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>), g, b, t1, stream, h, lsmall, nsmall);
-                else hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_LOCAL, 4>), g, b, t1, stream, h, lsmall, nsmall);
+                if (one) hipLaunchKernelGGL((k_heavy_local<0, 1, 4>), g, b, t1, s, h, lsmall, nsmall);
+                else if (h.stash) hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>), g, b, t1, s, h, lsmall, nsmall);
+                else hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_LOCAL, 4>), g, b, t1, s, h, lsmall, nsmall);
             }
             h.stash = nullptr;
             if (hs.nlocal_big) {
                 const dim3 g(hs.nlocal_big);
-                if (one) hipLaunchKernelGGL((k_heavy_local<0, 1, 8>), g, b, t2, stream, h, lbig, hs.nlocal_big);
-                else hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_MAX, 8>), g, b, t2, stream, h, lbig, hs.nlocal_big);
+                if (one) hipLaunchKernelGGL((k_heavy_local<0, 1, 8>), g, b, t2, s, h, lbig, hs.nlocal_big);
+                else hipLaunchKernelGGL((k_heavy_local<0, HEAVY_KB_MAX, 8>), g, b, t2, s, h, lbig, hs.nlocal_big);
             }
         }
     }
@@ -441,31 +462,77 @@ void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, bool
     for (uint32_t k0 = 0; k0 < K; k0 += hs.kb) {
         h.k0 = k0;
         h.kb = std::min(hs.kb, K - k0);
-        if (hs.cms) hipLaunchKernelGGL(k_heavy_clear<1>, dim3(hs.nchunked), dim3(BLOCK), 0, stream, h, hs.chunked.p, hs.nchunked);
-        else hipLaunchKernelGGL(k_heavy_clear<0>, dim3(hs.nchunked), dim3(BLOCK), 0, stream, h, hs.chunked.p, hs.nchunked);
+        if (hs.cms) hipLaunchKernelGGL(k_heavy_clear<1>, dim3(hs.nchunked), dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
+        else hipLaunchKernelGGL(k_heavy_clear<0>, dim3(hs.nchunked), dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
         const dim3 g(hs.nchunks), b(HBLOCK);
         if (hs.cms) {
             const size_t sk = cms_local_lds(std::min(h.kbs, h.kb), cells);
             if (one) {
-                hipLaunchKernelGGL((k_heavy_chunks<1, 1>), g, b, sk, stream, h);
-                hipLaunchKernelGGL((k_heavy_chunks<2, 1>), g, b, 0, stream, h);
+                hipLaunchKernelGGL((k_heavy_chunks<1, 1>), g, b, sk, s, h);
+                hipLaunchKernelGGL((k_heavy_chunks<2, 1>), g, b, 0, s, h);
             } else {
-                hipLaunchKernelGGL((k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>), g, b, sk, stream, h);
-                hipLaunchKernelGGL((k_heavy_chunks<2, HEAVY_KB_CMS_LOCAL>), g, b, 0, stream, h);
+                hipLaunchKernelGGL((k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>), g, b, sk, s, h);
+                hipLaunchKernelGGL((k_heavy_chunks<2, HEAVY_KB_CMS_LOCAL>), g, b, 0, s, h);
             }
         } else {
             const size_t tb = 2 * CHUNK * sizeof(uint64_t);
-            if (one) hipLaunchKernelGGL((k_heavy_chunks<0, 1>), g, b, tb, stream, h);
-            else hipLaunchKernelGGL((k_heavy_chunks<0, HEAVY_KB_MAX>), g, b, tb, stream, h);
+            if (one) hipLaunchKernelGGL((k_heavy_chunks<0, 1>), g, b, tb, s, h);
+            else hipLaunchKernelGGL((k_heavy_chunks<0, HEAVY_KB_MAX>), g, b, tb, s, h);
         }
         const uint64_t fin = (uint64_t)hs.nchunked * h.kb;
         const dim3 fg((unsigned)((fin + BLOCK - 1) / BLOCK));
-        if (hs.cms) hipLaunchKernelGGL(k_heavy_finish<1>, fg, dim3(BLOCK), 0, stream, h, hs.chunked.p, hs.nchunked);
-        else hipLaunchKernelGGL(k_heavy_finish<0>, fg, dim3(BLOCK), 0, stream, h, hs.chunked.p, hs.nchunked);
+        if (hs.cms) hipLaunchKernelGGL(k_heavy_finish<1>, fg, dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
+        else hipLaunchKernelGGL(k_heavy_finish<0>, fg, dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
     }
 }
 
-// One synchronous step: clear the counter, every bin reads L[cur] and writes
+// Whether an eager step of this method runs its heavy sets on the side
+// streams: their decode and counting wait for nothing that the bins do (a
+// vertex reads L[cur] and writes its own row of L[cur ^ 1]; in the two-kernel
+// method also its own row of the decoded CSR), and each alone leaves most of
+// the device idle.  The host waits for every stream at the end of the step,
+// so that no events are needed: joining streams on the device costs 30 us.
+// Captured and host-streamed steps, and those timed by events on the engine
+// stream, keep to one stream.
+bool lpa_engine::spread_step(int method) const {
+    if (graph_mode || host_stream || (method >= 1 && !have_csr)) return false;
+    bool any = false, any_heavy = false;
+    for (const Bin &b : bins)
+        any = any || (b.kind != LPA_BIN_SKIP && b.kind != LPA_BIN_CMS && b.kind != LPA_BIN_GLOBAL && b.end > b.begin);
+    for (const auto &hs : heavy) any_heavy = any_heavy || hs->nh;
+    return any_heavy && (any || heavy.size() > 1);
+}
+
+void lpa_engine::begin_step(bool side_streams) {
+    spread = side_streams;
+    if (spread)
+        for (hipStream_t &x : side)
+            if (!x) HIPCHK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+    if (!counts_clean) {
+        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)LANES, 0ull);
+        HIPCHK(hipGetLastError());
+        if (spread) sync();
+    }
+    counts_clean = false;
+}
+
+// Waits for the step; returns its changed labels.
+uint64_t lpa_engine::end_step() {
+    const int lanes = spread ? LANES : 1;
+    for (int l = 0; l < lanes; l++)
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, lane_stream(l), counter.p + l, h_counter + l);
+    HIPCHK(hipGetLastError());
+    uint64_t sum = 0;
+    for (int l = 0; l < lanes; l++) {
+        HIPCHK(hipStreamSynchronize(lane_stream(l)));
+        sum += h_counter[l];
+    }
+    counts_clean = true;
+    spread = false;
+    return sum;
+}
+
+// One synchronous step: every bin reads L[cur] and writes
 // L[cur^1].  Vertices without neighbours are never written (both buffers
 // hold their initial label).  launch_events (or null): 2 * (bins + heavy
 // sets) events, recorded around bin i at [2i, 2i+1] and around heavy set j
@@ -475,7 +542,6 @@ void lpa_engine::step(bool cglp, hipEvent_t *launch_events) {
         step_host_stream();
         return;
     }
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)1, 0ull);
     StepArgs a = base_args(cglp);
     if (!launch_events) launch_bins(bins, a, cglp, sched_used.quarter_max, stream);
     for (size_t i = 0; launch_events && i < bins.size(); i++) {
@@ -495,8 +561,9 @@ void lpa_engine::run_heavy(bool cglp, hipEvent_t *launch_events) {
         if (hs.nh == 0) continue;
         hipEvent_t *ev = launch_events ? launch_events + 2 * (bins.size() + j) : nullptr;
         if (ev) HIPCHK(hipEventRecord(ev[0], stream));
-        const StepArgs a = base_args(cglp && !hs.csr_part);
-        launch_heavy(hs, a, hs.csr_part || cglp);
+        const int lane = heavy_lane(j);
+        const StepArgs a = base_args(cglp && !hs.csr_part, lane);
+        launch_heavy(hs, a, hs.csr_part || cglp, lane_stream(lane));
         if (ev) HIPCHK(hipEventRecord(ev[1], stream));
     }
 }
@@ -529,7 +596,6 @@ template <class F> void lpa_engine::for_each_batch(F &&fn) {
 // launch reads L[cur] and writes L[cur ^ 1], so the order of the launches
 // changes nothing.
 void lpa_engine::step_host_stream() {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)1, 0ull);
     const StepArgs a = base_args(false);
     for_each_batch([&](const StreamBatch &sb, const uint64_t *w) {
         StepArgs ab = a;
@@ -542,17 +608,17 @@ void lpa_engine::step_host_stream() {
             if (c.begin < c.end) launch_bin(c, ab, false, sched_used.quarter_max, stream);
         }
         for (size_t j = 0; j < heavy.size(); j++)
-            if (!heavy[j]->csr_part) launch_heavy_decode(*heavy[j], ab, sb.tasks[j].first, sb.tasks[j].second);
+            if (!heavy[j]->csr_part) launch_heavy_decode(*heavy[j], ab, sb.tasks[j].first, sb.tasks[j].second, stream);
     });
     std::vector<Bin> small;
     for (const Bin &b : bins)
         if (b.csr) small.push_back(b);
     launch_bins(small, a, true, sched_used.quarter_max, stream);
-    for (auto &hp : heavy) launch_heavy(*hp, a, hp->csr_part, false);
+    for (auto &hp : heavy) launch_heavy(*hp, a, hp->csr_part, stream, false);
     HIPCHK(hipGetLastError());
 }
 
-// One fused step like step(false, ...), timing every bin launch and every
+// One fused step like step(false, ...), on one stream, timing every bin launch and every
 // heavy set with HIP events (ms; 0 where nothing ran).
 void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &heavy_ms) {
     const size_t nb = bins.size(), nhs = heavy.size();
@@ -562,7 +628,7 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
     std::vector<char> used(nb + nhs, 0);
     try {
         for (auto &x : ev) HIPCHK(hipEventCreate(&x));
-        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)1, 0ull);
+        begin_step(false);
         const StepArgs a = base_args(false);
         for (size_t i = 0; i < nb; i++) {
             const Bin &b = bins[i];
@@ -576,12 +642,12 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
             HeavySet &hs = *heavy[j];
             if (hs.nh == 0) continue;
             HIPCHK(hipEventRecord(ev[2 * (nb + j)], stream));
-            launch_heavy(hs, base_args(false), hs.csr_part);
+            launch_heavy(hs, base_args(false), hs.csr_part, stream);
             HIPCHK(hipEventRecord(ev[2 * (nb + j) + 1], stream));
             used[nb + j] = 1;
         }
         HIPCHK(hipGetLastError());
-        sync();
+        (void)end_step();
         for (size_t i = 0; i < nb + nhs; i++) {
             if (!used[i]) continue;
             float t = 0;
@@ -605,14 +671,14 @@ static void finish_graph(lpa_engine *e) {
     ddeg.alloc(n_c);
     e->feat0.alloc(n_c * NFEAT);
     e->meta0.alloc(n_c);
-    e->counter.alloc(1);
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
+    if (!e->err.p) e->err.alloc(1);
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->err.p, (uint64_t)1, 0ull);
     if (n_c)
         hipLaunchKernelGGL(k_scan_records, dim3((unsigned)((n_c * SCAN_G + 255) / 256)), dim3(256), 0, e->stream, e->words0.p,
-                           e->offs0.p, e->vid0.p, n_c, (uint32_t)e->n, ddeg.p, e->feat0.p, e->meta0.p, e->counter.p);
+                           e->offs0.p, e->vid0.p, n_c, (uint32_t)e->n, ddeg.p, e->feat0.p, e->meta0.p, e->err.p);
     HIPCHK(hipGetLastError());
     unsigned long long bad = 0;
-    HIPCHK(hipMemcpyAsync(&bad, e->counter.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
     e->deg_c.assign(n_c, 0);
     if (n_c) HIPCHK(hipMemcpyAsync(e->deg_c.data(), ddeg.p, n_c * 4, hipMemcpyDeviceToHost, e->stream));
     e->sync();
@@ -674,8 +740,8 @@ int lpa_engine_create(int device, lpa_engine **out) {
             e->lds_max = prop.sharedMemPerBlock;
             HIPCHK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
             e->scratch_dev = device_scratch(device);
-            e->counter.alloc(1);
-            HIPCHK(hipHostMalloc((void **)&e->h_counter, sizeof(unsigned long long), hipHostMallocDefault));
+            e->counter.alloc(lpa_engine::LANES);
+            HIPCHK(hipHostMalloc((void **)&e->h_counter, lpa_engine::LANES * sizeof(unsigned long long), hipHostMallocDefault));
             const int dyn = (int)(e->lds_max - 20480);
             bins_allow_lds(dyn);
             const void *heavy_fns[] = {(const void *)k_heavy_chunks<0, 1>, (const void *)k_heavy_chunks<0, HEAVY_KB_MAX>,
@@ -709,6 +775,8 @@ int lpa_engine_destroy(lpa_engine *e) {
         if (!e) return;
         (void)hipSetDevice(e->device);
         (void)hipStreamSynchronize(e->stream);
+        for (hipStream_t x : e->side)
+            if (x) (void)hipStreamSynchronize(x);
         delete e;
     });
 }
@@ -827,9 +895,9 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         e->vid0.upload(vert.data(), n_c, e->stream);
         len.alloc(n_c);
         e->offs0.alloc(n_c + 1);
-        e->counter.alloc(1);
-        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
-        launch_encode_len(e->stream, drow.p, dcol.p, e->vid0.p, n_c, n, len.p, e->counter.p, enc::LONG_ROW);
+        if (!e->err.p) e->err.alloc(1);
+        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->err.p, (uint64_t)1, 0ull);
+        launch_encode_len(e->stream, drow.p, dcol.p, e->vid0.p, n_c, n, len.p, e->err.p, enc::LONG_ROW);
         // rows longer than LONG_ROW: one workgroup each, with scratch of
         // d + 1 entries per row for every per-entry array (44 bytes each),
         // in groups of rows whose scratch stays within 2^28 entries
@@ -860,7 +928,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
             lsc = enc::LongScratch{dlbase.p, lleft.p, llen.p, lrid.p, lnxt_i.p, lnxt_r.p, lseg_i.p, lseg_r.p,
                                    lP_i.p, lP_r.p, linfo.p};
             hipLaunchKernelGGL(k_encode_long_len, dim3((unsigned)G.pos.size()), dim3(enc::LONG_LANES), 0, e->stream,
-                               drow.p, dcol.p, e->vid0.p, dlpos.p, (uint32_t)n, lsc, len.p, e->counter.p);
+                               drow.p, dcol.p, e->vid0.p, dlpos.p, (uint32_t)n, lsc, len.p, e->err.p);
         };
         if (!lgroups.empty()) {
             uint64_t tot = 0, rows = 0;
@@ -886,7 +954,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
                            e->offs0.p, nb);
         HIPCHK(hipGetLastError());
         unsigned long long bad = 0;
-        HIPCHK(hipMemcpyAsync(&bad, e->counter.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
+        HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
         e->h_offs.assign(n_c + 1, 0);
         HIPCHK(hipMemcpyAsync(e->h_offs.data(), e->offs0.p, (n_c + 1) * 8, hipMemcpyDeviceToHost, e->stream));
         e->sync();
@@ -1649,18 +1717,28 @@ static void enqueue_step(lpa_engine *e, int method) {
     HIPCHK(hipGraphLaunch(ge, e->stream));
 }
 
-static void finish_step(lpa_engine *e, uint64_t *changed) {
-    HIPCHK(hipMemcpyAsync(e->h_counter, e->counter.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, e->stream));
-    e->sync();
+// One step as the iterate entry points run it; nothing of it is in flight on
+// return, whatever happens.
+static void run_step(lpa_engine *e, int method, uint64_t *changed) {
+    uint64_t sum = 0;
+    try {
+        e->begin_step(e->spread_step(method));
+        enqueue_step(e, method);
+        sum = e->end_step();
+    } catch (...) {
+        for (int l = 0; l < lpa_engine::LANES; l++)
+            if (e->lane_stream(l)) (void)hipStreamSynchronize(e->lane_stream(l));
+        e->spread = false;
+        throw;
+    }
     e->cur ^= 1;
-    if (changed) *changed = *e->h_counter;
+    if (changed) *changed = sum;
 }
 
 int lpa_nova_iterate(lpa_engine *e, uint64_t *changed) {
     return guard([&] {
         require_ready(e);
-        enqueue_step(e, 0);
-        finish_step(e, changed);
+        run_step(e, 0, changed);
     });
 }
 
@@ -1690,7 +1768,7 @@ static void decode_range(lpa_engine *e, const uint64_t *words, uint32_t p0, uint
         if (e->heavy[j]->csr_part) continue;
         StepArgs a = e->base_args(false);
         a.words = words;
-        e->launch_heavy_decode(*e->heavy[j], a, tasks[j].first, tasks[j].second, true);
+        e->launch_heavy_decode(*e->heavy[j], a, tasks[j].first, tasks[j].second, e->lane_stream(e->heavy_lane(j)), true);
     }
 }
 
@@ -1767,7 +1845,6 @@ static void cglp_step(lpa_engine *e) {
 // compressed part, which equals its uncompressed adjacency, and the small
 // CSR): CGLP's second kernel, and on its own the uncompressed comparator.
 static void csr_lp(lpa_engine *e) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->counter.p, (uint64_t)1, 0ull);
     std::vector<Bin> part[2];
     for (const Bin &b : e->bins) part[b.csr].push_back(b);
     launch_bins(part[0], e->base_args(true), true, e->sched_used.quarter_max, e->stream);
@@ -1779,16 +1856,14 @@ static void csr_lp(lpa_engine *e) {
 int lpa_cglp_iterate(lpa_engine *e, uint64_t *changed) {
     return guard([&] {
         require_ready(e);
-        enqueue_step(e, 1);
-        finish_step(e, changed);
+        run_step(e, 1, changed);
     });
 }
 
 int lpa_csr_iterate(lpa_engine *e, uint64_t *changed) {
     return guard([&] {
         require_ready(e);
-        enqueue_step(e, 2);
-        finish_step(e, changed);
+        run_step(e, 2, changed);
     });
 }
 
@@ -2284,15 +2359,15 @@ int lpa_time_iterations(lpa_engine *e, int method, int iters, int use_graph, flo
             }
             e->graph_mode = use_graph != 0;
             for (int it = 0; it < iters; it++) {
+                e->begin_step(false);
                 HIPCHK(hipEventRecord(ev[0], e->stream));
                 if (e->graph_mode) enqueue_step(e, method);
                 else if (method == 0) e->step(false, kev.data());
                 else method_step(e, method);
                 HIPCHK(hipEventRecord(ev[1], e->stream));
-                HIPCHK(hipMemcpyAsync(e->h_counter, e->counter.p, 8, hipMemcpyDeviceToHost, e->stream));
-                e->sync();
+                const uint64_t sum = e->end_step();
                 HIPCHK(hipEventElapsedTime(&ms[it], ev[0], ev[1]));
-                if (changed) changed[it] = *e->h_counter;
+                if (changed) changed[it] = sum;
                 e->cur ^= 1;
                 if (method == 0 && !e->graph_mode && !e->host_stream) {
                     for (size_t l = 0; l < nl; l++) {

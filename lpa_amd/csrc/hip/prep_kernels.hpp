@@ -338,6 +338,16 @@ __global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, 
     }
 }
 
+// End of a step's work on a stream: its change count goes to the host's
+// (pinned) word and starts again at 0, in place of a clear before the step and
+// a copy after it.
+__global__ void k_publish(unsigned long long *count, unsigned long long *host) {
+    if (threadIdx.x == 0) {
+        *host = *count;
+        *count = 0;
+    }
+}
+
 __global__ void k_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
