@@ -185,6 +185,7 @@ namespace {
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 uint64_t *g_scratch_ptr[MAX_DEVICES] = {};
+bool g_lds_allowed[MAX_DEVICES] = {};   // kernel attributes set
 
 // The scratch address on `device`, resolved once per device; the device
 // must be current.
@@ -252,6 +253,7 @@ struct lpa_engine {
     // side streams: the heavy sets of an eager step run there beside the
     // bins (spread), see spread_step
     hipStream_t side[LANES - 1] = {};
+    hipEvent_t ev_side[LANES] = {};            // captured steps: fork, and the join of each side stream
     bool spread = false;
 
     // CGLP
@@ -294,6 +296,8 @@ struct lpa_engine {
         drop_graphs();
         if (h_counter) (void)hipHostFree(h_counter);
         for (hipEvent_t x : {ev_copied[0], ev_copied[1], ev_free[0], ev_free[1]})
+            if (x) (void)hipEventDestroy(x);
+        for (hipEvent_t x : ev_side)
             if (x) (void)hipEventDestroy(x);
         if (copy_stream) (void)hipStreamDestroy(copy_stream);
         for (hipStream_t x : side)
@@ -339,6 +343,9 @@ struct lpa_engine {
                              bool to_csr = false);
     void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipStream_t s, bool decode = true);
     bool spread_step(int method) const;
+    void make_side_streams();
+    void fork_capture();
+    void join_capture();
     void begin_step(bool side_streams);
     uint64_t end_step();
     template <class F> void for_each_batch(F &&fn);
@@ -486,16 +493,19 @@ void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipS
     }
 }
 
-// Whether an eager step of this method runs its heavy sets on the side
-// streams: their decode and counting wait for nothing that the bins do (a
-// vertex reads L[cur] and writes its own row of L[cur ^ 1]; in the two-kernel
-// method also its own row of the decoded CSR), and each alone leaves most of
-// the device idle.  The host waits for every stream at the end of the step,
-// so that no events are needed: joining streams on the device costs 30 us.
-// Captured and host-streamed steps, and those timed by events on the engine
-// stream, keep to one stream.
+// Whether a step of this method runs its heavy sets on the side streams:
+// their decode and counting wait for nothing that the bins do (a vertex reads
+// L[cur] and writes its own row of L[cur ^ 1]; in the two-kernel method also
+// its own row of the decoded CSR), and each alone leaves most of the device
+// idle.  After an eager step the host waits for every stream, so that no
+// events are needed: joining streams on the device costs 30 us.  A captured
+// step forks and joins inside the graph, which pays from SPREAD_LABELS label
+// reads up (20 us against a chain of launches).  Host-streamed steps, and
+// those timed by events on the engine stream, keep to one stream.
+constexpr uint64_t SPREAD_LABELS = 4ull << 20;
 bool lpa_engine::spread_step(int method) const {
-    if (graph_mode || host_stream || (method >= 1 && !have_csr)) return false;
+    if (host_stream || (method >= 1 && !have_csr)) return false;
+    if (graph_mode && (m_c + m_s) * K < SPREAD_LABELS) return false;
     bool any = false, any_heavy = false;
     for (const Bin &b : bins)
         any = any || (b.kind != LPA_BIN_SKIP && b.kind != LPA_BIN_CMS && b.kind != LPA_BIN_GLOBAL && b.end > b.begin);
@@ -503,11 +513,28 @@ bool lpa_engine::spread_step(int method) const {
     return any_heavy && (any || heavy.size() > 1);
 }
 
+void lpa_engine::make_side_streams() {
+    for (hipStream_t &x : side)
+        if (!x) HIPCHK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+}
+
+// Brings the side streams into the capture on the engine stream, and back.
+void lpa_engine::fork_capture() {
+    HIPCHK(hipEventRecord(ev_side[0], stream));
+    for (hipStream_t x : side) HIPCHK(hipStreamWaitEvent(x, ev_side[0], 0));
+    spread = true;
+}
+void lpa_engine::join_capture() {
+    spread = false;
+    for (int l = 1; l < LANES; l++) {
+        HIPCHK(hipEventRecord(ev_side[l], side[l - 1]));
+        HIPCHK(hipStreamWaitEvent(stream, ev_side[l], 0));
+    }
+}
+
 void lpa_engine::begin_step(bool side_streams) {
     spread = side_streams;
-    if (spread)
-        for (hipStream_t &x : side)
-            if (!x) HIPCHK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+    if (spread) make_side_streams();
     if (!counts_clean) {
         hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)LANES, 0ull);
         HIPCHK(hipGetLastError());
@@ -518,15 +545,16 @@ void lpa_engine::begin_step(bool side_streams) {
 
 // Waits for the step; returns its changed labels.
 uint64_t lpa_engine::end_step() {
+    // one stream (all counts): eager steps on it add to the first alone,
+    // captured ones may add to each
     const int lanes = spread ? LANES : 1;
     for (int l = 0; l < lanes; l++)
-        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, lane_stream(l), counter.p + l, h_counter + l);
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, lane_stream(l), counter.p + l, h_counter + l,
+                           (uint32_t)(spread ? 1 : LANES));
     HIPCHK(hipGetLastError());
+    for (int l = 0; l < lanes; l++) HIPCHK(hipStreamSynchronize(lane_stream(l)));
     uint64_t sum = 0;
-    for (int l = 0; l < lanes; l++) {
-        HIPCHK(hipStreamSynchronize(lane_stream(l)));
-        sum += h_counter[l];
-    }
+    for (int l = 0; l < LANES; l++) sum += h_counter[l];
     counts_clean = true;
     spread = false;
     return sum;
@@ -716,6 +744,21 @@ static uint32_t block_cap(const lpa_engine *e);
 static void move_stream(lpa_engine *e, DevBuf<uint64_t> &b, bool to_host);
 static void plan_batches(lpa_engine *e);
 
+// Lets the kernels use up to `dyn` bytes of dynamic LDS (once per device).
+static void allow_lds(int device, int dyn) {
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    if (g_lds_allowed[device]) return;
+    bins_allow_lds(dyn);
+    const void *heavy_fns[] = {(const void *)k_heavy_chunks<0, 1>, (const void *)k_heavy_chunks<0, HEAVY_KB_MAX>,
+                               (const void *)k_heavy_chunks<1, 1>, (const void *)k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>,
+                               (const void *)k_heavy_local<0, 1, 4>, (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4>,
+                               (const void *)k_heavy_local<0, 1, 8>, (const void *)k_heavy_local<0, HEAVY_KB_MAX, 8>,
+                               (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>,
+                               (const void *)k_heavy_local<1, 1, 4>, (const void *)k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>};
+    for (const void *f : heavy_fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
+    g_lds_allowed[device] = true;
+}
+
 extern "C" {
 
 const char *lpa_last_error(void) { return g_err.c_str(); }
@@ -742,15 +785,7 @@ int lpa_engine_create(int device, lpa_engine **out) {
             e->scratch_dev = device_scratch(device);
             e->counter.alloc(lpa_engine::LANES);
             HIPCHK(hipHostMalloc((void **)&e->h_counter, lpa_engine::LANES * sizeof(unsigned long long), hipHostMallocDefault));
-            const int dyn = (int)(e->lds_max - 20480);
-            bins_allow_lds(dyn);
-            const void *heavy_fns[] = {(const void *)k_heavy_chunks<0, 1>, (const void *)k_heavy_chunks<0, HEAVY_KB_MAX>,
-                                       (const void *)k_heavy_chunks<1, 1>, (const void *)k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>,
-                                       (const void *)k_heavy_local<0, 1, 4>, (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4>,
-                                       (const void *)k_heavy_local<0, 1, 8>, (const void *)k_heavy_local<0, HEAVY_KB_MAX, 8>,
-                                       (const void *)k_heavy_local<0, HEAVY_KB_LOCAL, 4, true>,
-                                       (const void *)k_heavy_local<1, 1, 4>, (const void *)k_heavy_local<1, HEAVY_KB_CMS_LOCAL, 4>};
-            for (const void *f : heavy_fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
+            allow_lds(device, (int)(e->lds_max - 20480));
             (void)hipGetLastError();
         } catch (...) {
             delete e;
@@ -1698,10 +1733,19 @@ static void enqueue_step(lpa_engine *e, int method) {
     hipGraphExec_t &ge = e->graphs[method][e->cur];
     if (!ge) {
         hipGraph_t g = nullptr;
+        const bool fork = e->spread_step(method);
+        if (fork) {
+            e->make_side_streams();
+            for (hipEvent_t &x : e->ev_side)
+                if (!x) HIPCHK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+        }
         HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         try {
+            if (fork) e->fork_capture();
             method_step(e, method);
+            if (fork) e->join_capture();
         } catch (...) {
+            e->spread = false;
             (void)hipStreamEndCapture(e->stream, &g);
             if (g) (void)hipGraphDestroy(g);
             throw;
@@ -1722,7 +1766,7 @@ static void enqueue_step(lpa_engine *e, int method) {
 static void run_step(lpa_engine *e, int method, uint64_t *changed) {
     uint64_t sum = 0;
     try {
-        e->begin_step(e->spread_step(method));
+        e->begin_step(!e->graph_mode && e->spread_step(method));
         enqueue_step(e, method);
         sum = e->end_step();
     } catch (...) {

@@ -338,13 +338,13 @@ __global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, 
     }
 }
 
-// End of a step's work on a stream: its change count goes to the host's
-// (pinned) word and starts again at 0, in place of a clear before the step and
+// End of a step's work on a stream: its n change counts go to the host's
+// (pinned) words and start again at 0, in place of a clear before the step and
 // a copy after it.
-__global__ void k_publish(unsigned long long *count, unsigned long long *host) {
-    if (threadIdx.x == 0) {
-        *host = *count;
-        *count = 0;
+__global__ void k_publish(unsigned long long *count, unsigned long long *host, uint32_t n) {
+    if (threadIdx.x < n) {
+        host[threadIdx.x] = count[threadIdx.x];
+        count[threadIdx.x] = 0;
     }
 }
 
