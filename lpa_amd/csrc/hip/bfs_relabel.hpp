@@ -25,9 +25,26 @@
 #include <rocprim/device/device_segmented_radix_sort.hpp>
 
 #include "encode_kernels.hpp"   // the exclusive-scan kernels
+#include "host_link.hpp"
 #include "lpa_amd.h"
 
 namespace lpa {
+
+// Working memory of the relabelling, kept between calls (up to KEEP bytes).
+struct BfsWork {
+    static constexpr uint64_t KEEP = 512ull << 20;
+    void *p = nullptr;
+    uint64_t bytes = 0;
+    BfsWork() = default;
+    BfsWork(const BfsWork &) = delete;
+    BfsWork &operator=(const BfsWork &) = delete;
+    ~BfsWork() { release(); }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
 
 namespace {
 
@@ -39,17 +56,6 @@ constexpr int WPB = 4;   // waves per 256-lane workgroup
         hipError_t e_ = (x);                                                                             \
         if (e_ != hipSuccess) throw std::runtime_error(std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-template <class T> struct Buf {
-    T *p = nullptr;
-    Buf() = default;
-    Buf(const Buf &) = delete;
-    Buf &operator=(const Buf &) = delete;
-    explicit Buf(uint64_t n) { BFS_HIPCHK(hipMalloc((void **)&p, std::max<uint64_t>(n, 1) * sizeof(T))); }
-    ~Buf() {
-        if (p) (void)hipFree(p);
-    }
-};
 
 // global wave index and wave count of a launch of 256-lane workgroups
 __device__ __forceinline__ uint64_t wave_id() { return ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; }
@@ -193,16 +199,22 @@ unsigned blocks_for(uint64_t items, uint64_t per_block) {
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((items + per_block - 1) / per_block, 1ull << 20));
 }
 
-// exclusive scan of n values in place (out[n] = total; out has n + 1 entries)
-void scan_in_place(hipStream_t s, uint64_t *a, uint64_t n) {
-    const uint64_t nb = std::max<uint64_t>(1, (n + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK);
-    Buf<uint64_t> sums(nb);
-    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(256), 0, s, a, n, sums.p);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, s, sums.p, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(256), 0, s, a, n, sums.p, a, nb);
+uint64_t scan_blocks(uint64_t n) { return std::max<uint64_t>(1, (n + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK); }
+
+// exclusive scan of n values in place (out[n] = total; out has n + 1
+// entries); sums: scan_blocks(n) words
+void scan_in_place(hipStream_t s, uint64_t *a, uint64_t n, uint64_t *sums) {
+    const uint64_t nb = scan_blocks(n);
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(256), 0, s, a, n, sums);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, s, sums, nb);
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(256), 0, s, a, n, sums, a, nb);
     BFS_HIPCHK(hipGetLastError());
-    BFS_HIPCHK(hipStreamSynchronize(s));   // sums is freed on return
 }
+
+template <class T> struct WorkPtr {
+    T *p;
+    WorkPtr(void *base, uint64_t at) : p(reinterpret_cast<T *>(static_cast<char *>(base) + at)) {}
+};
 
 uint64_t read_u64(hipStream_t s, const uint64_t *p) {
     uint64_t x = 0;
@@ -215,7 +227,7 @@ uint64_t read_u64(hipStream_t s, const uint64_t *p) {
 
 // Host arrays in and out: row[n+1], col[row[n]] (any CSR with ids < n);
 // new_row[n+1], new_col[row[n]], perm[n] (perm[v] = new id of v).
-void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const uint32_t *h_col, uint32_t root,
+void bfs_relabel_device(hipStream_t s, HostLink &link, BfsWork &work, uint64_t n, const uint64_t *h_row, const uint32_t *h_col, uint32_t root,
                         uint64_t *h_new_row, uint32_t *h_new_col, uint32_t *h_perm) {
     if (n == 0) {
         h_new_row[0] = 0;
@@ -223,12 +235,33 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
     }
     if (root >= n) throw std::invalid_argument("root >= n");
     const uint64_t m = h_row[n];
-    Buf<uint64_t> row(n + 1), new_row(n + 1), cnt(n + 1);
-    Buf<uint32_t> col(m), nid(n), claim(n), order(n);
-    BFS_HIPCHK(hipMemcpyAsync(row.p, h_row, (n + 1) * 8, hipMemcpyHostToDevice, s));
-    if (m) BFS_HIPCHK(hipMemcpyAsync(col.p, h_col, m * 4, hipMemcpyHostToDevice, s));
+    // all arrays from one piece of memory (256-byte aligned)
+    uint64_t need = 0;
+    auto place = [&](uint64_t count, uint64_t size) {
+        const uint64_t at = need;
+        need += (std::max<uint64_t>(count, 1) * size + 255) / 256 * 256;
+        return at;
+    };
+    const uint64_t a_row = place(n + 1, 8), a_new = place(n + 1, 8), a_cnt = place(n + 1, 8), a_sums = place(scan_blocks(n), 8),
+                   a_col = place(m, 4), a_uns = place(m, 4), a_nid = place(n, 4), a_claim = place(n, 4),
+                   a_order = place(n, 4), a_rel = place(n + 1, 4), a_bad = place(1, 4);
+    if (work.bytes < need) {
+        work.release();
+        BFS_HIPCHK(hipMalloc(&work.p, need));
+        work.bytes = need;
+    }
+    struct Trim {   // memory too large to keep goes back, also after an error
+        BfsWork &w;
+        ~Trim() {
+            if (w.bytes > BfsWork::KEEP) w.release();
+        }
+    } trim{work};
+    WorkPtr<uint64_t> row{work.p, a_row}, new_row{work.p, a_new}, cnt{work.p, a_cnt}, sums{work.p, a_sums};
+    WorkPtr<uint32_t> col{work.p, a_col}, unsorted{work.p, a_uns}, nid{work.p, a_nid}, claim{work.p, a_claim},
+        order{work.p, a_order}, rel{work.p, a_rel}, bad{work.p, a_bad};
+    link.in(row.p, h_row, (n + 1) * 8, s);
+    link.in(col.p, h_col, m * 4, s);
     {
-        Buf<uint32_t> bad(1);
         hipLaunchKernelGGL(k_bfs_fill, dim3(1), dim3(64), 0, s, bad.p, (uint64_t)1, 0u);
         if (m) hipLaunchKernelGGL(k_bfs_check_ids, dim3(blocks_for(m, 256)), dim3(256), 0, s, col.p, m, n, bad.p);
         BFS_HIPCHK(hipGetLastError());
@@ -248,7 +281,7 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
         hipLaunchKernelGGL(k_bfs_claim, g, b, 0, s, order.p, lo, fsz, row.p, col.p, nid.p, claim.p);
         hipLaunchKernelGGL(k_bfs_count, g, b, 0, s, order.p, lo, fsz, row.p, col.p, nid.p, claim.p, cnt.p);
         BFS_HIPCHK(hipGetLastError());
-        scan_in_place(s, cnt.p, fsz);
+        scan_in_place(s, cnt.p, fsz, sums.p);
         const uint64_t total = read_u64(s, cnt.p + fsz);
         if (total) {
             hipLaunchKernelGGL(k_bfs_place, g, b, 0, s, order.p, lo, fsz, hi, row.p, col.p, nid.p, claim.p, cnt.p);
@@ -262,7 +295,7 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
         // unreached vertices follow in id order (cnt holds n + 1 words)
         hipLaunchKernelGGL(k_bfs_unreached_flag, dim3(blocks_for(n, 256)), dim3(256), 0, s, nid.p, n, cnt.p);
         BFS_HIPCHK(hipGetLastError());
-        scan_in_place(s, cnt.p, n);
+        scan_in_place(s, cnt.p, n, sums.p);
         hipLaunchKernelGGL(k_bfs_unreached_place, dim3(blocks_for(n, 256)), dim3(256), 0, s, order.p, nid.p, n, hi,
                            cnt.p);
         BFS_HIPCHK(hipGetLastError());
@@ -270,17 +303,14 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
     // relabelled CSR: rows in the new order, then every row sorted
     hipLaunchKernelGGL(k_bfs_new_degree, dim3(blocks_for(n, 256)), dim3(256), 0, s, order.p, n, row.p, new_row.p);
     BFS_HIPCHK(hipGetLastError());
-    scan_in_place(s, new_row.p, n);
-    Buf<uint32_t> unsorted(m);
+    scan_in_place(s, new_row.p, n, sums.p);
     hipLaunchKernelGGL(k_bfs_new_rows, dim3(blocks_for(n, WPB)), dim3(256), 0, s, order.p, n, row.p, col.p, nid.p,
                        new_row.p, unsorted.p);
     BFS_HIPCHK(hipGetLastError());
-    std::vector<uint64_t> nr(n + 1);
-    BFS_HIPCHK(hipMemcpyAsync(nr.data(), new_row.p, (n + 1) * 8, hipMemcpyDeviceToHost, s));
-    BFS_HIPCHK(hipStreamSynchronize(s));
+    link.out(h_new_row, new_row.p, (n + 1) * 8, s);
+    const uint64_t *nr = h_new_row;
     // the old col buffer receives the sorted rows; batches of rows below 2^31 keys
     const uint64_t batch_keys = 1ull << 31;
-    Buf<uint32_t> rel(n + 1);
     size_t temp_bytes = 0;
     void *temp = nullptr;
     try {
@@ -288,7 +318,7 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
             uint64_t s1 = s0 + 1;
             // as many rows as fit the batch (a single longer row is still one batch)
             const uint64_t lim = nr[s0] + batch_keys;
-            s1 = (uint64_t)(std::upper_bound(nr.begin() + s0 + 1, nr.end(), lim) - nr.begin()) - 1;
+            s1 = (uint64_t)(std::upper_bound(nr + s0 + 1, nr + n + 1, lim) - nr) - 1;
             if (s1 <= s0) s1 = s0 + 1;
             s1 = std::min<uint64_t>(s1, std::min<uint64_t>(n, s0 + (1ull << 31)));
             const uint64_t keys = nr[s1] - nr[s0];
@@ -318,10 +348,8 @@ void bfs_relabel_device(hipStream_t s, uint64_t n, const uint64_t *h_row, const 
         throw;
     }
     if (temp) BFS_HIPCHK(hipFree(temp));
-    std::copy(nr.begin(), nr.end(), h_new_row);
-    if (m) BFS_HIPCHK(hipMemcpyAsync(h_new_col, col.p, m * 4, hipMemcpyDeviceToHost, s));
-    BFS_HIPCHK(hipMemcpyAsync(h_perm, nid.p, n * 4, hipMemcpyDeviceToHost, s));
-    BFS_HIPCHK(hipStreamSynchronize(s));
+    link.out(h_new_col, col.p, m * 4, s);
+    link.out(h_perm, nid.p, n * 4, s);
 }
 
 }  // namespace lpa

@@ -30,6 +30,7 @@
 #include "encode_long.hpp"
 #include "encode_wave.hpp"
 #include "heavy_kernels.hpp"
+#include "host_link.hpp"
 #include "mlp_kernels.hpp"
 #include "lp_kernels.hpp"
 #include "lpa_amd.h"
@@ -60,6 +61,9 @@ template <class F> int guard(F &&f) {
     } catch (const Fail &e) {
         g_err = e.what();
         return e.code;
+    } catch (const HostLinkError &e) {
+        g_err = e.what();
+        return LPA_ERR_HIP;
     } catch (const std::bad_alloc &) {
         g_err = "out of host memory";
         return LPA_ERR_RANGE;
@@ -71,7 +75,7 @@ template <class F> int guard(F &&f) {
 
 template <class T> struct DevBuf {
     T *p = nullptr;
-    uint64_t n = 0;
+    uint64_t n = 0, cap = 0;
     bool host = false;   // pinned host memory, mapped into the device's address space
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
@@ -80,14 +84,22 @@ template <class T> struct DevBuf {
     void release() {
         if (p) (void)(host ? hipHostFree(p) : hipFree(p));
         p = nullptr;
-        n = 0;
+        n = cap = 0;
         host = false;
     }
+    // cnt elements of any content; memory that is there already is kept when
+    // it fits without much waste (allocating and freeing cost 0.2 to 0.5 ms
+    // each).  Freeing waited for the device, keeping does not: nothing that
+    // is still queued may use the old content.
     void alloc(uint64_t cnt) {
-        release();
         if (cnt == 0) cnt = 1;
+        if (p && !host && cnt <= cap && cap - cnt <= cnt / 4) {
+            n = cnt;
+            return;
+        }
+        release();
         HIPCHK(hipMalloc((void **)&p, cnt * sizeof(T)));
-        n = cnt;
+        n = cap = cnt;
     }
     // pinned host memory that kernels can read in place (same address on
     // the device) and copies can stream from at full link speed
@@ -96,7 +108,7 @@ template <class T> struct DevBuf {
         if (cnt == 0) cnt = 1;
         HIPCHK(hipHostMalloc((void **)&p, cnt * sizeof(T), hipHostMallocDefault));
         host = true;
-        n = cnt;
+        n = cap = cnt;
         void *d = nullptr;
         HIPCHK(hipHostGetDevicePointer(&d, p, 0));
         if (d != (void *)p) throw Fail(LPA_ERR_HIP, "pinned host memory is mapped at another device address");
@@ -104,12 +116,22 @@ template <class T> struct DevBuf {
     void swap(DevBuf &o) {
         std::swap(p, o.p);
         std::swap(n, o.n);
+        std::swap(cap, o.cap);
         std::swap(host, o.host);
     }
     void upload(const T *h, uint64_t cnt, hipStream_t s) {
         alloc(cnt);
         if (cnt) HIPCHK(hipMemcpyAsync(p, h, cnt * sizeof(T), hipMemcpyHostToDevice, s));
     }
+    void upload(const T *h, uint64_t cnt, hipStream_t s, HostLink &link) {
+        alloc(cnt);
+        link.in(p, h, cnt * sizeof(T), s);
+    }
+    // gives memory back that is too large to keep between calls
+    void trim(uint64_t most_bytes = KEEP_BYTES) {
+        if (cap * sizeof(T) > most_bytes) release();
+    }
+    static constexpr uint64_t KEEP_BYTES = 256ull << 20;
 };
 
 // Heavy vertices of one part (compressed or small CSR) and one mode (CMS or
@@ -206,6 +228,14 @@ struct lpa_engine {
     int device = 0;
     hipStream_t stream = nullptr;
     uint64_t *scratch_dev = nullptr;   // this device's copy of `scratch`
+    HostLink link;
+    // working memory of the encoder and of the relabelling, kept between
+    // calls up to DevBuf::KEEP_BYTES each
+    struct Work {
+        DevBuf<uint64_t> row, len, sums;
+        DevBuf<uint32_t> col, deg;
+        BfsWork bfs;
+    } work;
     int num_cu = 0;
     size_t lds_max = 65536;
 
@@ -695,7 +725,7 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
 // records.
 static void finish_graph(lpa_engine *e) {
     const uint64_t n_c = e->n_c;
-    DevBuf<uint32_t> ddeg;
+    DevBuf<uint32_t> &ddeg = e->work.deg;
     ddeg.alloc(n_c);
     e->feat0.alloc(n_c * NFEAT);
     e->meta0.alloc(n_c);
@@ -707,9 +737,9 @@ static void finish_graph(lpa_engine *e) {
     HIPCHK(hipGetLastError());
     unsigned long long bad = 0;
     HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
-    e->deg_c.assign(n_c, 0);
-    if (n_c) HIPCHK(hipMemcpyAsync(e->deg_c.data(), ddeg.p, n_c * 4, hipMemcpyDeviceToHost, e->stream));
-    e->sync();
+    e->deg_c.resize(n_c);
+    e->link.out(e->deg_c.data(), ddeg.p, n_c * 4, e->stream);
+    ddeg.trim();
     if (bad) throw Fail(LPA_ERR_FORMAT, "malformed CGR record at stream position " + std::to_string(bad - 1));
     e->m_c = 0;
     for (uint32_t d : e->deg_c) e->m_c += d;
@@ -872,14 +902,14 @@ int lpa_graph_upload(lpa_engine *e, uint64_t n, uint64_t n_c, const uint32_t *wo
             }
         } else {
             DevBuf<uint32_t> w32;
-            w32.upload(words, nwords, e->stream);
+            w32.upload(words, nwords, e->stream, e->link);
             e->words0.alloc(n64);
             hipLaunchKernelGGL(k_pack64, dim3((unsigned)((n64 + 255) / 256)), dim3(256), 0, e->stream, w32.p, n32,
                                e->words0.p, n64);
             e->sync();
         }
-        e->offs0.upload(offsets, n_c + 1, e->stream);
-        e->vid0.upload(vertices, n_c, e->stream);
+        e->offs0.upload(offsets, n_c + 1, e->stream, e->link);
+        e->vid0.upload(vertices, n_c, e->stream, e->link);
         finish_graph(e);
     });
 }
@@ -899,35 +929,49 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         // stream order (compressor.cpp:157-290): deg >= 128 by id, then
         // small_thresh <= deg < 128 by id; deg < small_thresh -> small CSR
         const uint32_t large = 128;
-        std::vector<uint32_t> vert;
-        vert.reserve(n);
         auto deg = [&](uint64_t v) { return row[v + 1] - row[v]; };
-        for (uint64_t v = 0; v < n; v++) if (deg(v) >= large) vert.push_back((uint32_t)v);
-        for (uint64_t v = 0; v < n; v++) if (deg(v) >= small_thresh && deg(v) < large) vert.push_back((uint32_t)v);
-        const uint64_t n_c = vert.size();
-        for (uint64_t v = 0; v < n; v++) if (deg(v) < small_thresh) vert.push_back((uint32_t)v);
-        const uint64_t n_s = n - n_c;
-        e->h_soffs.assign(1, 0);
-        e->h_snbr.clear();
-        for (uint64_t j = n_c; j < n; j++) {
-            const uint32_t v = vert[j];
-            for (uint64_t k = row[v]; k < row[v + 1]; k++) {
-                if (col[k] >= n) throw Fail(LPA_ERR_FORMAT, "neighbour id >= n");
-                e->h_snbr.push_back(col[k]);
+        uint64_t nl = 0, n_s = 0, m_s = 0;
+        for (uint64_t v = 0; v < n; v++) {
+            const uint64_t d = deg(v);
+            if (d >= small_thresh || d >= large) {
+                nl += d >= large;
+            } else {
+                n_s++;
+                m_s += d;
             }
-            e->h_soffs.push_back(e->h_snbr.size());
+        }
+        // (a row of 128 or more ids is compressed whatever the threshold)
+        const uint64_t n_c = n - n_s;
+        std::vector<uint32_t> &vert = e->h_vertices;
+        vert.resize(n);
+        e->h_soffs.resize(n_s + 1);
+        e->h_soffs[0] = 0;
+        e->h_snbr.resize(m_s);
+        for (uint64_t v = 0, il = 0, im = nl, is = 0, k = 0; v < n; v++) {
+            const uint64_t d = deg(v);
+            if (d >= large) {
+                vert[il++] = (uint32_t)v;
+            } else if (d >= small_thresh) {
+                vert[im++] = (uint32_t)v;
+            } else {
+                vert[n_c + is] = (uint32_t)v;
+                for (uint64_t j = row[v]; j < row[v + 1]; j++) {
+                    if (col[j] >= n) throw Fail(LPA_ERR_FORMAT, "neighbour id >= n");
+                    e->h_snbr[k++] = col[j];
+                }
+                e->h_soffs[++is] = k;
+            }
         }
         e->n = n;
         e->n_c = n_c;
         e->n_s = n_s;
-        e->m_s = e->h_snbr.size();
-        e->h_vertices = vert;
+        e->m_s = m_s;
         // encode on the device
-        DevBuf<uint64_t> drow, len, offs;
-        DevBuf<uint32_t> dcol;
-        drow.upload(row, n + 1, e->stream);
-        dcol.upload(col, m, e->stream);
-        e->vid0.upload(vert.data(), n_c, e->stream);
+        DevBuf<uint64_t> &drow = e->work.row, &len = e->work.len;
+        DevBuf<uint32_t> &dcol = e->work.col;
+        drow.upload(row, n + 1, e->stream, e->link);
+        dcol.upload(col, m, e->stream, e->link);
+        e->vid0.upload(vert.data(), n_c, e->stream, e->link);
         len.alloc(n_c);
         e->offs0.alloc(n_c + 1);
         if (!e->err.p) e->err.alloc(1);
@@ -981,7 +1025,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
             }
         }
         const uint64_t nb = std::max<uint64_t>(1, (n_c + SCAN_PER_BLOCK - 1) / SCAN_PER_BLOCK);
-        DevBuf<uint64_t> sums;
+        DevBuf<uint64_t> &sums = e->work.sums;
         sums.alloc(nb);
         hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(256), 0, e->stream, len.p, n_c, sums.p);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, e->stream, sums.p, nb);
@@ -990,9 +1034,8 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         HIPCHK(hipGetLastError());
         unsigned long long bad = 0;
         HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
-        e->h_offs.assign(n_c + 1, 0);
-        HIPCHK(hipMemcpyAsync(e->h_offs.data(), e->offs0.p, (n_c + 1) * 8, hipMemcpyDeviceToHost, e->stream));
-        e->sync();
+        e->h_offs.resize(n_c + 1);
+        e->link.out(e->h_offs.data(), e->offs0.p, (n_c + 1) * 8, e->stream);
         if (bad) throw Fail(LPA_ERR_FORMAT, "row of vertex " + std::to_string(bad - 1) +
                                                 " is not strictly increasing or has an id >= n");
         e->nbits = e->h_offs[n_c];
@@ -1012,6 +1055,9 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         HIPCHK(hipGetLastError());
         if (e->host_stream) move_stream(e, e->words0, true);
         finish_graph(e);
+        drow.trim();
+        dcol.trim();
+        len.trim();
     });
 }
 
@@ -1078,7 +1124,7 @@ int lpa_csr_bfs_relabel(lpa_engine *e, uint64_t n, const uint64_t *row, const ui
         if (n && root >= n) throw Fail(LPA_ERR_RANGE, "root >= n");
         HIPCHK(hipSetDevice(e->device));
         try {
-            bfs_relabel_device(e->stream, n, row, col, root, new_row, new_col, perm);
+            bfs_relabel_device(e->stream, e->link, e->work.bfs, n, row, col, root, new_row, new_col, perm);
         } catch (const std::invalid_argument &x) {
             throw Fail(LPA_ERR_FORMAT, x.what());
         } catch (const std::runtime_error &x) {
@@ -1095,8 +1141,9 @@ int lpa_graph_stream(lpa_engine *e, uint64_t *n_c, uint64_t *nbits, uint64_t *wo
         HIPCHK(hipSetDevice(e->device));
         *n_c = e->n_c;
         *nbits = e->nbits;
-        if (words && e->nbits)
-            HIPCHK(hipMemcpyAsync(words, e->words0.p, (e->nbits + 63) / 64 * 8, hipMemcpyDefault, e->stream));
+        const uint64_t wbytes = (e->nbits + 63) / 64 * 8;
+        if (words && wbytes && e->words0.host) std::memcpy(words, e->words0.p, wbytes);
+        else if (words) e->link.out(words, e->words0.p, wbytes, e->stream);
         if (offsets) std::memcpy(offsets, e->h_offs.data(), (e->n_c + 1) * 8);
         if (vertices) std::memcpy(vertices, e->h_vertices.data(), e->n * 4);
         e->sync();
@@ -1664,7 +1711,7 @@ int lpa_labels_init(lpa_engine *e, const uint32_t *labels) {
         const uint32_t seed = e->semi ? SEED_BIT : 0u;
         const dim3 g((unsigned)((tot + 1023) / 1024));
         if (labels && tot)
-            HIPCHK(hipMemcpyAsync(e->L[0].p, labels, tot * sizeof(uint32_t), hipMemcpyHostToDevice, e->stream));
+            e->link.in(e->L[0].p, labels, tot * sizeof(uint32_t), e->stream);
         if (tot && labels)
             hipLaunchKernelGGL(k_labels_given, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, tot, seed);
         else if (tot)
@@ -1684,11 +1731,15 @@ int lpa_labels_get(lpa_engine *e, uint32_t *labels) {
         if (!e->have_labels) throw Fail(LPA_ERR_STATE, "no labels");
         HIPCHK(hipSetDevice(e->device));
         const uint64_t tot = e->n * e->K;
-        HIPCHK(hipMemcpyAsync(labels, e->L[e->cur].p, tot * 4, hipMemcpyDeviceToHost, e->stream));
-        e->sync();
-        // only a clamped seed carries the bit
-        if (e->semi)
-            for (uint64_t i = 0; i < tot; i++) labels[i] = clean_host(labels[i]);
+        if (!e->semi) {
+            e->link.out(labels, e->L[e->cur].p, tot * 4, e->stream);
+        } else {   // clamped seeds carry the bit
+            e->link.out(labels, e->L[e->cur].p, tot * 4, e->stream, [](void *d, const void *p, size_t len) {
+                const uint32_t *x = (const uint32_t *)p;
+                uint32_t *y = (uint32_t *)d;
+                for (size_t i = 0; i < len / 4; i++) y[i] = clean_host(x[i]);
+            });
+        }
     });
 }
 
@@ -1957,6 +2008,18 @@ struct lpa_mlp {
     // buffered: a training step reads state[cur] and writes the other one
     DevBuf<float> state[2], part[2], grad;
     DevBuf<double> loss;
+    HostLink link;
+    // inputs and outputs of a call, kept for the next up to DevBuf::KEEP_BYTES each
+    DevBuf<float> x, y, target;
+    DevBuf<uint8_t> mask;
+    DevBuf<uint32_t> idx;
+    void trim() {
+        x.trim();
+        y.trim();
+        target.trim();
+        mask.trim();
+        idx.trim();
+    }
     int cur = 0;
     int t = 0;
     ~lpa_mlp() {
@@ -2178,14 +2241,14 @@ int lpa_mlp_forward(lpa_mlp *m, const float *x, uint64_t n, float *y) {
         if (!m || (n && (!x || !y))) throw Fail(LPA_ERR_ARG, "null argument");
         if (n == 0) return;
         HIPCHK(hipSetDevice(m->device));
-        DevBuf<float> dx, dy;
-        dx.upload(x, n * MLP_IN, m->stream);
+        DevBuf<float> &dx = m->x, &dy = m->y;
+        dx.upload(x, n * MLP_IN, m->stream, m->link);
         dy.alloc(n * MLP_OUT);
         hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream,
                            m->state[m->cur].p, dx.p, dy.p, n);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(y, dy.p, n * MLP_OUT * 4, hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipStreamSynchronize(m->stream));
+        m->link.out(y, dy.p, n * MLP_OUT * 4, m->stream);
+        m->trim();
     });
 }
 
@@ -2194,11 +2257,11 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
     return guard([&] {
         if (!m || !x || !target || !mask || !loss || !grad || n == 0) throw Fail(LPA_ERR_ARG, "bad arguments");
         HIPCHK(hipSetDevice(m->device));
-        DevBuf<float> dx, dt;
-        DevBuf<uint8_t> dm;
-        dx.upload(x, n * MLP_IN, m->stream);
-        dt.upload(target, n * MLP_OUT, m->stream);
-        dm.upload(mask, n * MLP_OUT, m->stream);
+        DevBuf<float> &dx = m->x, &dt = m->target;
+        DevBuf<uint8_t> &dm = m->mask;
+        dx.upload(x, n * MLP_IN, m->stream, m->link);
+        dt.upload(target, n * MLP_OUT, m->stream, m->link);
+        dm.upload(mask, n * MLP_OUT, m->stream, m->link);
         const uint32_t np = mlp_parts(n, MLP_PARTS_MAX);
         launch_mlp_step(m, nullptr, 0, AdamArgs{}, nullptr, dx.p, dt.p, dm.p, nullptr, n, 1.0f / (float)n, m->part[0].p, np);
         hipLaunchKernelGGL(k_mlp_sum, dim3((MLP_STRIDE / 4 + 63) / 64), dim3(64), 0, m->stream, m->part[0].p, np, m->grad.p);
@@ -2206,6 +2269,7 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
         HIPCHK(hipMemcpyAsync(grad, m->grad.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipMemcpyAsync(loss, m->grad.p + MLP_NPARAM, 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));
+        m->trim();
     });
 }
 
@@ -2215,12 +2279,12 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
         if (!m || !x || !target || !mask || n == 0 || epochs <= 0 || batch <= 0) throw Fail(LPA_ERR_ARG, "bad arguments");
         if (n >= (1ull << 32)) throw Fail(LPA_ERR_RANGE, "too many samples");
         HIPCHK(hipSetDevice(m->device));
-        DevBuf<float> dx, dt;
-        DevBuf<uint8_t> dm;
-        DevBuf<uint32_t> didx;
-        dx.upload(x, n * MLP_IN, m->stream);
-        dt.upload(target, n * MLP_OUT, m->stream);
-        dm.upload(mask, n * MLP_OUT, m->stream);
+        DevBuf<float> &dx = m->x, &dt = m->target;
+        DevBuf<uint8_t> &dm = m->mask;
+        DevBuf<uint32_t> &didx = m->idx;
+        dx.upload(x, n * MLP_IN, m->stream, m->link);
+        dt.upload(target, n * MLP_OUT, m->stream, m->link);
+        dm.upload(mask, n * MLP_OUT, m->stream, m->link);
         didx.alloc(n);
         std::vector<uint32_t> idx(n);
         std::iota(idx.begin(), idx.end(), 0u);
@@ -2262,6 +2326,7 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
         HIPCHK(hipStreamSynchronize(m->stream));
         if (loss_per_epoch)
             for (int ep = 0; ep < epochs; ep++) loss_per_epoch[ep] = (float)(l[ep] / (double)nb);
+        m->trim();
     });
 }
 
