@@ -276,6 +276,7 @@ struct lpa_engine {
     // changed labels of a step, one count per stream it uses; h_counter:
     // their host copies (pinned)
     static constexpr int LANES = 3;
+    static constexpr uint64_t COUNTS = (uint64_t)LANES * COUNT_SLOTS * COUNT_STRIDE;
     DevBuf<unsigned long long> counter;
     unsigned long long *h_counter = nullptr;
     bool counts_clean = false;                 // the device counts are 0
@@ -284,6 +285,7 @@ struct lpa_engine {
     // bins (spread), see spread_step
     hipStream_t side[LANES - 1] = {};
     hipEvent_t ev_side[LANES] = {};            // captured steps: fork, and the join of each side stream
+    hipEvent_t ev_lists = nullptr;             // a heavy set's lists are decoded
     bool spread = false;
 
     // CGLP
@@ -329,6 +331,7 @@ struct lpa_engine {
             if (x) (void)hipEventDestroy(x);
         for (hipEvent_t x : ev_side)
             if (x) (void)hipEventDestroy(x);
+        if (ev_lists) (void)hipEventDestroy(ev_lists);
         if (copy_stream) (void)hipStreamDestroy(copy_stream);
         for (hipStream_t x : side)
             if (x) (void)hipStreamDestroy(x);
@@ -341,6 +344,11 @@ struct lpa_engine {
     // set j
     hipStream_t lane_stream(int lane) const { return lane ? side[lane - 1] : stream; }
     int heavy_lane(size_t j) const { return spread ? 1 + (int)(j % (LANES - 1)) : 0; }
+    // the only heavy set has both kinds of vertices: its chunks take the
+    // second side stream
+    bool chunks_beside() const { return heavy.size() == 1 && heavy[0]->nlocal && heavy[0]->nchunked; }
+    // streams that a spread step uses
+    int side_lanes() const { return heavy.size() > 1 || chunks_beside() ? 3 : 2; }
 
     StepArgs base_args(bool cglp, int lane = 0) const {
         StepArgs a{};
@@ -362,7 +370,7 @@ struct lpa_engine {
         a.cms_depth = cms_depth;
         a.cms_logw = ceil_log2(cms_width);
         std::memcpy(a.cms_ab, cms_ab, sizeof cms_ab);
-        a.changed = counter.p + lane;
+        a.changed = counter.p + (uint64_t)lane * COUNT_SLOTS * COUNT_STRIDE;
         a.rec = rec;
         a.xcds = sched_used.xcd_tiles == 1 ? XCDS : 1;
         return a;
@@ -371,7 +379,7 @@ struct lpa_engine {
     HeavyArgs heavy_args(const HeavySet &hs, const StepArgs &a, bool as_csr) const;
     void launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint32_t t0, uint32_t t1, hipStream_t s,
                              bool to_csr = false);
-    void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipStream_t s, bool decode = true);
+    void launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, int lane, bool decode = true);
     bool spread_step(int method) const;
     void make_side_streams();
     void fork_capture();
@@ -456,12 +464,21 @@ void lpa_engine::launch_heavy_decode(const HeavySet &hs, const StepArgs &a, uint
 
 // A heavy set's step: decode its records into the lists (unless `decode` is
 // off: a host-resident stream decodes them batch by batch), then count.
-void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipStream_t s, bool decode) {
+void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, int lane, bool decode) {
     if (hs.nh == 0) return;
+    const hipStream_t s = lane_stream(lane);
     HeavyArgs h = heavy_args(hs, a, as_csr);
     const bool one = K == 1;
     const size_t cells = (size_t)cms_depth * cms_width;
     if (!as_csr && decode) launch_heavy_decode(hs, a, 0, hs.ntasks, s);
+    // the only heavy set: its hubs' chunks run beside its one-workgroup
+    // vertices, on the other side stream, once what is queued so far (the
+    // decode of the lists, or of the CSR's rows) is done
+    const bool beside = lane == 1 && chunks_beside();
+    if (beside) {
+        HIPCHK(hipEventRecord(ev_lists, s));
+        HIPCHK(hipStreamWaitEvent(lane_stream(2), ev_lists, 0));
+    }
     if (hs.nlocal) {
         const dim3 b(HBLOCK);
         const size_t sk = cms_local_lds(h.kbl, cells);
@@ -496,30 +513,32 @@ void lpa_engine::launch_heavy(HeavySet &hs, const StepArgs &a, bool as_csr, hipS
         }
     }
     if (hs.nchunked == 0) return;
+    const hipStream_t sc = beside ? lane_stream(2) : s;
+    if (beside) h.s.changed = base_args(false, 2).changed;
     for (uint32_t k0 = 0; k0 < K; k0 += hs.kb) {
         h.k0 = k0;
         h.kb = std::min(hs.kb, K - k0);
-        if (hs.cms) hipLaunchKernelGGL(k_heavy_clear<1>, dim3(hs.nchunked), dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
-        else hipLaunchKernelGGL(k_heavy_clear<0>, dim3(hs.nchunked), dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
+        if (hs.cms) hipLaunchKernelGGL(k_heavy_clear<1>, dim3(hs.nchunked), dim3(BLOCK), 0, sc, h, hs.chunked.p, hs.nchunked);
+        else hipLaunchKernelGGL(k_heavy_clear<0>, dim3(hs.nchunked), dim3(BLOCK), 0, sc, h, hs.chunked.p, hs.nchunked);
         const dim3 g(hs.nchunks), b(HBLOCK);
         if (hs.cms) {
             const size_t sk = cms_local_lds(std::min(h.kbs, h.kb), cells);
             if (one) {
-                hipLaunchKernelGGL((k_heavy_chunks<1, 1>), g, b, sk, s, h);
-                hipLaunchKernelGGL((k_heavy_chunks<2, 1>), g, b, 0, s, h);
+                hipLaunchKernelGGL((k_heavy_chunks<1, 1>), g, b, sk, sc, h);
+                hipLaunchKernelGGL((k_heavy_chunks<2, 1>), g, b, 0, sc, h);
             } else {
-                hipLaunchKernelGGL((k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>), g, b, sk, s, h);
-                hipLaunchKernelGGL((k_heavy_chunks<2, HEAVY_KB_CMS_LOCAL>), g, b, 0, s, h);
+                hipLaunchKernelGGL((k_heavy_chunks<1, HEAVY_KB_CMS_LOCAL>), g, b, sk, sc, h);
+                hipLaunchKernelGGL((k_heavy_chunks<2, HEAVY_KB_CMS_LOCAL>), g, b, 0, sc, h);
             }
         } else {
             const size_t tb = 2 * CHUNK * sizeof(uint64_t);
-            if (one) hipLaunchKernelGGL((k_heavy_chunks<0, 1>), g, b, tb, s, h);
-            else hipLaunchKernelGGL((k_heavy_chunks<0, HEAVY_KB_MAX>), g, b, tb, s, h);
+            if (one) hipLaunchKernelGGL((k_heavy_chunks<0, 1>), g, b, tb, sc, h);
+            else hipLaunchKernelGGL((k_heavy_chunks<0, HEAVY_KB_MAX>), g, b, tb, sc, h);
         }
         const uint64_t fin = (uint64_t)hs.nchunked * h.kb;
         const dim3 fg((unsigned)((fin + BLOCK - 1) / BLOCK));
-        if (hs.cms) hipLaunchKernelGGL(k_heavy_finish<1>, fg, dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
-        else hipLaunchKernelGGL(k_heavy_finish<0>, fg, dim3(BLOCK), 0, s, h, hs.chunked.p, hs.nchunked);
+        if (hs.cms) hipLaunchKernelGGL(k_heavy_finish<1>, fg, dim3(BLOCK), 0, sc, h, hs.chunked.p, hs.nchunked);
+        else hipLaunchKernelGGL(k_heavy_finish<0>, fg, dim3(BLOCK), 0, sc, h, hs.chunked.p, hs.nchunked);
     }
 }
 
@@ -546,17 +565,19 @@ bool lpa_engine::spread_step(int method) const {
 void lpa_engine::make_side_streams() {
     for (hipStream_t &x : side)
         if (!x) HIPCHK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+    for (hipEvent_t *x : {&ev_side[0], &ev_side[1], &ev_side[2], &ev_lists})
+        if (!*x) HIPCHK(hipEventCreateWithFlags(x, hipEventDisableTiming));
 }
 
 // Brings the side streams into the capture on the engine stream, and back.
 void lpa_engine::fork_capture() {
     HIPCHK(hipEventRecord(ev_side[0], stream));
-    for (hipStream_t x : side) HIPCHK(hipStreamWaitEvent(x, ev_side[0], 0));
+    for (int l = 1; l < side_lanes(); l++) HIPCHK(hipStreamWaitEvent(side[l - 1], ev_side[0], 0));
     spread = true;
 }
 void lpa_engine::join_capture() {
     spread = false;
-    for (int l = 1; l < LANES; l++) {
+    for (int l = 1; l < side_lanes(); l++) {
         HIPCHK(hipEventRecord(ev_side[l], side[l - 1]));
         HIPCHK(hipStreamWaitEvent(stream, ev_side[l], 0));
     }
@@ -564,9 +585,8 @@ void lpa_engine::join_capture() {
 
 void lpa_engine::begin_step(bool side_streams) {
     spread = side_streams;
-    if (spread) make_side_streams();
     if (!counts_clean) {
-        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, counter.p, (uint64_t)LANES, 0ull);
+        hipLaunchKernelGGL(k_fill_u64, dim3((COUNTS + 255) / 256), dim3(256), 0, stream, counter.p, COUNTS, 0ull);
         HIPCHK(hipGetLastError());
         if (spread) sync();
     }
@@ -577,14 +597,14 @@ void lpa_engine::begin_step(bool side_streams) {
 uint64_t lpa_engine::end_step() {
     // one stream (all counts): eager steps on it add to the first alone,
     // captured ones may add to each
-    const int lanes = spread ? LANES : 1;
+    const int lanes = spread ? side_lanes() : 1;
     for (int l = 0; l < lanes; l++)
-        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, lane_stream(l), counter.p + l, h_counter + l,
-                           (uint32_t)(spread ? 1 : LANES));
+        hipLaunchKernelGGL(k_publish, dim3(spread ? 1 : LANES), dim3(64), 0, lane_stream(l),
+                           counter.p + (uint64_t)l * COUNT_SLOTS * COUNT_STRIDE, COUNT_SLOTS, COUNT_STRIDE, h_counter + l);
     HIPCHK(hipGetLastError());
     for (int l = 0; l < lanes; l++) HIPCHK(hipStreamSynchronize(lane_stream(l)));
     uint64_t sum = 0;
-    for (int l = 0; l < LANES; l++) sum += h_counter[l];
+    for (int l = 0; l < (spread ? lanes : LANES); l++) sum += h_counter[l];
     counts_clean = true;
     spread = false;
     return sum;
@@ -621,7 +641,7 @@ void lpa_engine::run_heavy(bool cglp, hipEvent_t *launch_events) {
         if (ev) HIPCHK(hipEventRecord(ev[0], stream));
         const int lane = heavy_lane(j);
         const StepArgs a = base_args(cglp && !hs.csr_part, lane);
-        launch_heavy(hs, a, hs.csr_part || cglp, lane_stream(lane));
+        launch_heavy(hs, a, hs.csr_part || cglp, lane);
         if (ev) HIPCHK(hipEventRecord(ev[1], stream));
     }
 }
@@ -672,7 +692,7 @@ void lpa_engine::step_host_stream() {
     for (const Bin &b : bins)
         if (b.csr) small.push_back(b);
     launch_bins(small, a, true, sched_used.quarter_max, stream);
-    for (auto &hp : heavy) launch_heavy(*hp, a, hp->csr_part, stream, false);
+    for (auto &hp : heavy) launch_heavy(*hp, a, hp->csr_part, 0, false);
     HIPCHK(hipGetLastError());
 }
 
@@ -700,7 +720,7 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
             HeavySet &hs = *heavy[j];
             if (hs.nh == 0) continue;
             HIPCHK(hipEventRecord(ev[2 * (nb + j)], stream));
-            launch_heavy(hs, base_args(false), hs.csr_part, stream);
+            launch_heavy(hs, base_args(false), hs.csr_part, 0);
             HIPCHK(hipEventRecord(ev[2 * (nb + j) + 1], stream));
             used[nb + j] = 1;
         }
@@ -812,8 +832,14 @@ int lpa_engine_create(int device, lpa_engine **out) {
             e->num_cu = prop.multiProcessorCount;
             e->lds_max = prop.sharedMemPerBlock;
             HIPCHK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
+            // the side streams right behind it: the runtime gives a new
+            // stream the least used of its four hardware queues, so an
+            // engine's three get three of them; made at its first step they
+            // shared one where a process has several engines (3.7 ms
+            // instead of 3.0 for the copying graph's run)
+            e->make_side_streams();
             e->scratch_dev = device_scratch(device);
-            e->counter.alloc(lpa_engine::LANES);
+            e->counter.alloc(lpa_engine::COUNTS);
             HIPCHK(hipHostMalloc((void **)&e->h_counter, lpa_engine::LANES * sizeof(unsigned long long), hipHostMallocDefault));
             allow_lds(device, (int)(e->lds_max - 20480));
             (void)hipGetLastError();
@@ -1785,11 +1811,6 @@ static void enqueue_step(lpa_engine *e, int method) {
     if (!ge) {
         hipGraph_t g = nullptr;
         const bool fork = e->spread_step(method);
-        if (fork) {
-            e->make_side_streams();
-            for (hipEvent_t &x : e->ev_side)
-                if (!x) HIPCHK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
-        }
         HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         try {
             if (fork) e->fork_capture();

@@ -203,7 +203,11 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_decode(HeavyArgs h, const Decod
     }
     __syncthreads();
     uint32_t *out = crow ? ccol + crow[h.pos[T.h]] + (T.out - h.loff[T.h]) : h.list + T.out;
-    const uint32_t j = T.j0 + threadIdx.x;
+    // a lane per segment; a task small enough keeps its two kinds of segments
+    // in different waves, where they do not wait for each other
+    const uint32_t nI = i1 > T.j0 ? i1 - T.j0 : 0, nR = j1 > r0 ? j1 - r0 : 0, t64 = threadIdx.x - 64;
+    uint32_t j = T.j0 + threadIdx.x;
+    if (nI <= 64 && nR <= BLOCK - 64) j = threadIdx.x < 64 ? (threadIdx.x < nI ? j : j1) : (t64 < nR ? r0 + t64 : j1);
     auto segment = [&](auto &r, uint32_t *dst) {   // the reader stands at segment j
         if (j < T.ni) {
             read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
@@ -859,7 +863,7 @@ __device__ __forceinline__ void heavy_local_vertex(const HeavyArgs &h, uint32_t 
                 ST ? st + (uint64_t)k0 * d : nullptr, d);   // k0 is a multiple of 4
         }
     }
-    if (threadIdx.x == 0 && nch) atomicAdd(a.changed, (unsigned long long)nch);
+    if (threadIdx.x == 0 && nch) atomicAdd(count_slot(a.changed), (unsigned long long)nch);
     if (a.rec && threadIdx.x == 0) atomicAdd(&a.rec[v], (cycles() - t0) * HBLOCK);
 }
 

@@ -90,6 +90,16 @@ __device__ __forceinline__ uint32_t pick(uint64_t best, uint32_t old) {
     return ~(uint32_t)best;
 }
 
+// A step's count of changed labels is kept in COUNT_SLOTS words, each in a
+// line of its own, that the workgroups share (k_publish adds them up): atomics
+// on one address take about 10 ns each, one after another, and a step that
+// changes labels everywhere has one per workgroup (a 1024 x 1024 lattice:
+// 4096 of them, 40 of its lane kernel's 56 us).
+constexpr uint32_t COUNT_SLOTS = 64, COUNT_STRIDE = 16;
+__device__ __forceinline__ unsigned long long *count_slot(unsigned long long *counter) {
+    return counter + (blockIdx.x % COUNT_SLOTS) * COUNT_STRIDE;
+}
+
 // Adds the block's changed labels to the counter with one atomic: n is the
 // calling lane's count; every thread of the block must call it.
 __device__ __forceinline__ void flush_changes(uint32_t n, unsigned long long *counter) {
@@ -100,12 +110,12 @@ __device__ __forceinline__ void flush_changes(uint32_t n, unsigned long long *co
     for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
     if ((threadIdx.x & 63) == 0 && n) atomicAdd(&total, n);
     __syncthreads();
-    if (threadIdx.x == 0 && total) atomicAdd(counter, (unsigned long long)total);
+    if (threadIdx.x == 0 && total) atomicAdd(count_slot(counter), (unsigned long long)total);
 }
 
 __device__ __forceinline__ void count_changes(bool ch, unsigned long long *counter) {
     uint64_t b = __ballot(ch);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(counter, (unsigned long long)__popcll(b));
+    if ((threadIdx.x & 63) == 0 && b) atomicAdd(count_slot(counter), (unsigned long long)__popcll(b));
 }
 
 // ------------------------------------------------------------ lane kernel

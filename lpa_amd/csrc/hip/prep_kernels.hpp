@@ -338,14 +338,19 @@ __global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, 
     }
 }
 
-// End of a step's work on a stream: its n change counts go to the host's
-// (pinned) words and start again at 0, in place of a clear before the step and
+// End of a step's work on a stream: change count l (slots at count + l *
+// slots * stride), one per workgroup of 64 lanes, is added up for the host's
+// (pinned) word and starts again at 0, in place of a clear before the step and
 // a copy after it.
-__global__ void k_publish(unsigned long long *count, unsigned long long *host, uint32_t n) {
-    if (threadIdx.x < n) {
-        host[threadIdx.x] = count[threadIdx.x];
-        count[threadIdx.x] = 0;
+__global__ void __launch_bounds__(64) k_publish(unsigned long long *count, uint32_t slots, uint32_t stride,
+                                                unsigned long long *host) {
+    unsigned long long *c = count + (uint64_t)blockIdx.x * slots * stride, x = 0;
+    for (uint32_t i = threadIdx.x; i < slots; i += 64) {
+        x += c[i * stride];
+        c[i * stride] = 0;
     }
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    if (threadIdx.x == 0) host[blockIdx.x] = x;
 }
 
 __global__ void k_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v) {
