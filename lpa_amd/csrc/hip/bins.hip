@@ -80,6 +80,7 @@ static const void *bins_fn(uint32_t K) {
 }
 
 void bins_allow_lds(int dyn) {
+    allow_group_lds<8>(dyn);
     allow_group_lds<16>(dyn);
     allow_group_lds<32>(dyn);
     allow_group_lds<64>(dyn);
@@ -88,13 +89,33 @@ void bins_allow_lds(int dyn) {
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
 }
 
-// groups per workgroup of a WAVE bin of a step.  With 8 vectors per staged
-// gather, lists of 65..128 ids take half waves (4 ids per lane) rather than
-// quarter waves (8 per lane): half the staged registers, twice the waves
-// resident.
+// Lanes per vertex of a WAVE bin, as groups per workgroup.  One or two
+// vectors (8 staged ids per lane whatever the group): as few lanes as hold the
+// list, 8 for up to 64 ids to 64 for 512, because a list of d ids is only
+// about d / 20 segments to decode, a lane each.  More vectors: a quarter wave
+// up to quarter_max ids, a wave above, and with 8 vectors per staged gather
+// half waves for 65..128 ids (4 ids per lane) rather than quarter waves (8
+// per lane): half the staged registers, twice the waves resident.
+// (quarter_max below 128 asks for whole waves above it, whatever K.)
+static int decode_groups(uint32_t logT) {
+    const uint32_t cap = 1u << (logT - 1);
+    return cap <= 64 ? 32 : cap <= 128 ? 16 : cap <= 256 ? 8 : 4;
+}
 static int step_groups(uint32_t logT, uint32_t K, uint32_t quarter_max) {
-    const int ng = wave_groups(logT, quarter_max ? quarter_max : 128);
+    if (quarter_max == 0) quarter_max = 128;
+    if (K <= 2 && quarter_max >= 128) return decode_groups(logT);
+    const int ng = wave_groups(logT, quarter_max);
     return ng == 16 && (1u << (logT - 1)) > 64 && K >= 5 ? 8 : ng;
+}
+// staged ids per lane of the launch of a list of cap ids with groups of G lanes
+static uint32_t staged_ids(int kb, uint32_t cap, uint32_t G) {
+    const uint32_t ipl = (cap + G - 1) / G;
+    return kb <= 2 ? 8 : ipl <= 2 ? 2 : ipl <= 4 ? 4 : 8;
+}
+static size_t step_lds(int ng, uint32_t logT, bool csr, uint32_t K) {
+    const uint32_t cap = 1u << (logT - 1), G = BLOCK / ng;
+    const int kb = group_kb(K);
+    return group_list_inside(csr, K, kb, cap, staged_ids(kb, cap, G) * G) ? (size_t)ng * 8ull << logT : group_lds(ng, logT);
 }
 
 void launch_bin(const Bin &b, StepArgs a, bool as_csr, uint32_t quarter_max, hipStream_t s) {
@@ -110,14 +131,15 @@ void launch_bin(const Bin &b, StepArgs a, bool as_csr, uint32_t quarter_max, hip
         break;
     case LPA_BIN_WAVE: {
         const int ng = step_groups(logT, a.K, quarter_max);
-        const size_t lds = group_lds(ng, logT);
+        const size_t lds = step_lds(ng, logT, as_csr, a.K);
         const dim3 grid((count + ng - 1) / ng);
-        if (ng == 16) launch_group<16>(as_csr, grid, lds, s, a, logT, cap);
+        if (ng == 32) launch_group<8>(as_csr, grid, lds, s, a, logT, cap);
+        else if (ng == 16) launch_group<16>(as_csr, grid, lds, s, a, logT, cap);
         else if (ng == 8) launch_group<32>(as_csr, grid, lds, s, a, logT, cap);
         else launch_group<64>(as_csr, grid, lds, s, a, logT, cap);
         break;
     }
-    case LPA_BIN_BLOCK: launch_group<BLOCK>(as_csr, dim3(count), group_lds(1, logT), s, a, logT, cap); break;
+    case LPA_BIN_BLOCK: launch_group<BLOCK>(as_csr, dim3(count), step_lds(1, logT, as_csr, a.K), s, a, logT, cap); break;
     default: break;   // heavy bins run through their own kernels
     }
 }
@@ -144,6 +166,9 @@ struct Merge {
 };
 
 static size_t static_bytes(size_t s) { return (s + 7) / 8 * 8; }
+static uint32_t group_code(int ng) {
+    return ng == 1 ? BC_G256 : ng == 4 ? BC_G64 : ng == 8 ? BC_G32 : ng == 16 ? BC_G16 : BC_G8;
+}
 
 template <int N> static size_t lane_bytes(bool csr) {
     return csr ? sizeof(LaneShared<N, true>) : sizeof(LaneShared<N, false>);
@@ -181,9 +206,11 @@ void launch_bins(const std::vector<Bin> &bins, const StepArgs &a, bool all_csr, 
         } else if (b.kind == LPA_BIN_WAVE || b.kind == LPA_BIN_BLOCK) {
             const int ng = b.kind == LPA_BIN_BLOCK ? 1 : step_groups(logT, a.K, quarter_max);
             wg = (count + ng - 1) / ng;
-            code = ng == 1 ? BC_G256 : ng == 4 ? BC_G64 : ng == 8 ? BC_G32 : BC_G16;
-            bytes = group_lds(ng, logT) + static_bytes(ng == 1 ? sizeof(GroupStatic<BLOCK, 8>) : ng == 4 ? sizeof(GroupStatic<64, 8>)
-                                                       : ng == 8 ? sizeof(GroupStatic<32, 8>) : sizeof(GroupStatic<16, 8>));
+            code = group_code(ng);
+            bytes = step_lds(ng, logT, csr, a.K) +
+                    static_bytes(ng == 1 ? sizeof(GroupStatic<BLOCK, 8>) : ng == 4 ? sizeof(GroupStatic<64, 8>)
+                                 : ng == 8 ? sizeof(GroupStatic<32, 8>) : ng == 16 ? sizeof(GroupStatic<16, 8>)
+                                                                                   : sizeof(GroupStatic<8, 8>));
         } else {
             continue;
         }
@@ -220,11 +247,11 @@ void launch_decode_bins(const std::vector<Bin> &bins, const DecodeArgs &a, hipSt
             default: one.add(b, BC_LANE64, false, 0, wg, sizeof(LaneDecodeShared<64>)); break;
             }
         } else if (b.kind == LPA_BIN_WAVE || b.kind == LPA_BIN_BLOCK) {
-            const int ng = b.kind == LPA_BIN_BLOCK ? 1 : wave_groups(logT);
+            const int ng = b.kind == LPA_BIN_BLOCK ? 1 : decode_groups(logT);
             const size_t st = ng == 1 ? sizeof(GroupDecodeStatic<BLOCK>) : ng == 4 ? sizeof(GroupDecodeStatic<64>)
-                                                                                  : sizeof(GroupDecodeStatic<16>);
-            one.add(b, ng == 1 ? BC_G256 : ng == 4 ? BC_G64 : BC_G16, false, logT, (count + ng - 1) / ng,
-                    group_lds(ng, logT) + static_bytes(st));
+                              : ng == 8 ? sizeof(GroupDecodeStatic<32>) : ng == 16 ? sizeof(GroupDecodeStatic<16>)
+                                                                                   : sizeof(GroupDecodeStatic<8>);
+            one.add(b, group_code(ng), false, logT, (count + ng - 1) / ng, (size_t)ng * 6ull * (1ull << logT) + static_bytes(st));
         } else {
             continue;
         }

@@ -20,7 +20,8 @@ struct Bin {
 };
 
 // LDS bytes of the WAVE / BLOCK kernels' per-group table (2^logT slots) and
-// neighbour list (2^logT / 2 ids), for ng groups per workgroup.
+// neighbour list (2^logT / 2 ids), for ng groups per workgroup (the most that
+// a launch takes).
 inline size_t group_lds(int ng, uint32_t logT) { return (size_t)ng * 10ull * (1ull << logT); }
 // groups per workgroup of a WAVE bin: a quarter wave per vertex up to
 // quarter_max ids, a whole wave above

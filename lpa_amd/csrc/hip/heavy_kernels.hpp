@@ -177,7 +177,7 @@ template <int CMS>
 __global__ void __launch_bounds__(BLOCK) k_heavy_decode(HeavyArgs h, const DecodeTask *__restrict__ tasks,
                                                         uint32_t ntasks, const uint64_t *__restrict__ crow,
                                                         uint32_t *__restrict__ ccol) {
-    __shared__ GroupShared<BLOCK> sh;
+    __shared__ GroupShared<BLOCK, 512> sh;
     __shared__ uint32_t stage[DECODE_STAGE];
     __shared__ uint64_t sw[TASK_WORDS];
     const uint32_t t = blockIdx.x;
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_decode(HeavyArgs h, const Decod
     auto segment = [&](auto &r, uint32_t *dst) {   // the reader stands at segment j
         if (j < T.ni) {
             read_interval_segment(r, T.v, [&](uint32_t l, uint32_t len) {
-                put_run<BLOCK>(&sh, dst, atomicAdd(&sh.cnt, len), l, len);
+                put_run(&sh, dst, atomicAdd(&sh.cnt, len), l, len);
             });
         } else {
             const uint32_t c = r.gamma();   // claims the segment's slots

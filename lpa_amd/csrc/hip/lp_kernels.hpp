@@ -420,9 +420,10 @@ __device__ __forceinline__ uint32_t cms_col(const StepArgs &a, uint32_t r, uint3
 // whole group.
 constexpr uint32_t LONG_RUN = 16, HUGE_RUN = 512;
 
-template <int G> struct GroupShared {
-    static constexpr int QCAP = G == BLOCK ? 512 : G == 64 ? 64 : G == 32 ? 32 : 16;
-    static constexpr int HCAP = 8;
+// Q: runs of LONG_RUN ids that a list of the group can hold, or a bound on
+// those queued (HCAP more for huge ones).
+template <int G, int Q = G == BLOCK ? 128 : G == 64 ? 64 : G / 2> struct GroupShared {
+    static constexpr uint32_t QCAP = Q, HCAP = G >= 64 ? 8 : 0;
     uint32_t cnt;                 // ids written to the list so far
     uint32_t qn, hn;
     uint32_t qleft[QCAP + HCAP];  // long runs, then huge ones from QCAP on
@@ -459,7 +460,7 @@ __device__ __forceinline__ void with_record(const uint64_t *__restrict__ words, 
 }
 
 // Empties the group's counters (one lane; the caller synchronises).
-template <int G> __device__ __forceinline__ void clear_runs(GroupShared<G> *sh) {
+template <class Sh> __device__ __forceinline__ void clear_runs(Sh *sh) {
     sh->cnt = 0;
     sh->qn = 0;
     sh->hn = 0;
@@ -469,13 +470,13 @@ template <int G> __device__ __forceinline__ void clear_runs(GroupShared<G> *sh) 
 // lanes per run (a hub of short runs has hundreds of them: one after another
 // by the whole group they took 43 us of a 152 us decode of a copying graph's
 // hubs), the huge ones by all lanes.
-template <int G>
-__device__ __forceinline__ void write_long_runs(const GroupShared<G> *sh, uint32_t gl, uint32_t *list) {
-    constexpr uint32_t QCAP = GroupShared<G>::QCAP, HCAP = GroupShared<G>::HCAP;
+template <int G, class Sh>
+__device__ __forceinline__ void write_long_runs(const Sh *sh, uint32_t gl, uint32_t *list) {
+    constexpr uint32_t QCAP = Sh::QCAP, HCAP = Sh::HCAP, R = G < 16 ? G : 16;
     const uint32_t nq = sh->qn < QCAP ? sh->qn : QCAP, nh = sh->hn < HCAP ? sh->hn : HCAP;
-    for (uint32_t q = gl / 16; q < nq; q += G / 16) {
+    for (uint32_t q = gl / R; q < nq; q += G / R) {
         const uint32_t l = sh->qleft[q], len = sh->qlen[q], o = sh->qpos[q];
-        for (uint32_t x = gl & 15; x < len; x += 16) list[o + x] = l + x;
+        for (uint32_t x = gl % R; x < len; x += R) list[o + x] = l + x;
     }
     for (uint32_t q = QCAP; q < QCAP + nh; q++) {
         const uint32_t l = sh->qleft[q], len = sh->qlen[q], o = sh->qpos[q];
@@ -485,12 +486,12 @@ __device__ __forceinline__ void write_long_runs(const GroupShared<G> *sh, uint32
 
 // Ids l .. l + len - 1 at list[o ..): queued for the group when the run is
 // long and the queue has room.
-template <int G>
-__device__ __forceinline__ void put_run(GroupShared<G> *sh, uint32_t *list, uint32_t o, uint32_t l, uint32_t len) {
+template <class Sh>
+__device__ __forceinline__ void put_run(Sh *sh, uint32_t *list, uint32_t o, uint32_t l, uint32_t len) {
     if (len >= LONG_RUN) {
-        constexpr uint32_t QCAP = GroupShared<G>::QCAP, HCAP = GroupShared<G>::HCAP;
+        constexpr uint32_t QCAP = Sh::QCAP, HCAP = Sh::HCAP;
         uint32_t q = QCAP + HCAP;
-        if (len >= HUGE_RUN) {
+        if (HCAP && len >= HUGE_RUN) {
             q = atomicAdd(&sh->hn, 1u);
             q = q < HCAP ? QCAP + q : QCAP + HCAP;
         }
@@ -532,7 +533,7 @@ __device__ __forceinline__ uint32_t group_decode(const StepArgs &a, uint32_t p, 
             if (j < ni) {
                 auto r = at(start + m.x + (uint64_t)SEG_BITS * j);
                 read_interval_segment(r, v, [&](uint32_t l, uint32_t len) {
-                    put_run<G>(sh, list, atomicAdd(&sh->cnt, len), l, len);
+                    put_run(sh, list, atomicAdd(&sh->cnt, len), l, len);
                 });
             } else {
                 auto r = at(start + m.z + (uint64_t)SEG_BITS * (j - ni));
@@ -731,6 +732,16 @@ __device__ __forceinline__ void count_staged(const StepArgs &a, const uint32_t *
 // staged in registers, IPL neighbours per lane (the launch picks the
 // smallest IPL with IPL * G >= listcap, so the staged labels, IPL * KB
 // registers, cost no more occupancy than the bin needs).
+// Whether a group's list lies inside its table's memory (upper half; the
+// staged words in the lower): with one batch of vectors whose labels are all
+// staged, the ids are not read again once the table is in use.  (A wave's LDS
+// operations are in order; the workgroup's own-label check, which such a list
+// always takes, has barriers between.)  CSR rows need no list.  A fifth less
+// LDS: 40 -> 32 KB per workgroup, 5 instead of 3 on a CU.
+inline __host__ __device__ bool group_list_inside(bool csr, uint32_t K, uint32_t kb, uint32_t cap, uint32_t staged) {
+    return csr || (K <= kb && cap <= staged);
+}
+
 template <int G, int KB> struct GroupStatic {
     uint64_t red[BLOCK / 64];
     uint32_t xw[G > 64 ? KB * (G / 64) : 1], xs[KB];
@@ -747,8 +758,11 @@ __device__ __forceinline__ void group_tile(const StepArgs &a, uint32_t logT, uin
     auto &xs = st.xs;
     const uint32_t gid = threadIdx.x / G, gl = threadIdx.x % G;
     const uint32_t T = 1u << logT;
-    uint64_t *tab = lds + (uint64_t)gid * (T + (listcap + 1) / 2);
-    uint32_t *list = (uint32_t *)(tab + T);
+    // the list shares the table's memory when it is not read again once the
+    // (only) batch's labels are staged, see group_list_inside
+    const bool inside = group_list_inside(CSR, a.K, KB, listcap, IPL * G);
+    uint64_t *tab = lds + (uint64_t)gid * (inside ? T : T + T / 4);
+    uint32_t *list = (uint32_t *)(inside ? tab + T / 2 : tab + T);
     GroupShared<G> *sh = &st.gsh[gid];
     const uint32_t stride = tiles * NG;
     uint32_t nch = 0;
@@ -766,7 +780,7 @@ __device__ __forceinline__ void group_tile(const StepArgs &a, uint32_t logT, uin
                 d = (uint32_t)(a.row[p + 1] - a.row[p]);
             }
         } else if (live) {
-            d = group_decode<G>(a, p, v, gl, sh, list, tab, T);
+            d = group_decode<G>(a, p, v, gl, sh, list, tab, inside ? T / 2 : T);
         }
         for (uint32_t k0 = 0; k0 < a.K; k0 += KB) {
             const uint32_t kb = a.K - k0 < (uint32_t)KB ? a.K - k0 : (uint32_t)KB;
@@ -834,7 +848,7 @@ __global__ void __launch_bounds__(BLOCK) k_group(StepArgs a, uint32_t logT, uint
 
 // Bins of one step that share a launch (k_bins).
 // BC_LANE64 only decodes to a CSR here.
-enum BinCode : uint32_t { BC_LANE4, BC_LANE8, BC_LANE16, BC_LANE32, BC_LANE64, BC_G16, BC_G32, BC_G64, BC_G256 };
+enum BinCode : uint32_t { BC_LANE4, BC_LANE8, BC_LANE16, BC_LANE32, BC_LANE64, BC_G8, BC_G16, BC_G32, BC_G64, BC_G256 };
 struct BinTable {
     static constexpr uint32_t MAX = 12;
     struct Entry {
@@ -867,9 +881,12 @@ __device__ __forceinline__ void one_bin(const StepArgs &a, const BinTable::Entry
     case BC_LANE8: lane_tile<8, CSR>(a, tile, *reinterpret_cast<LaneShared<8, CSR> *>(lds)); break;
     case BC_LANE16: lane_tile<16, CSR>(a, tile, *reinterpret_cast<LaneShared<16, CSR> *>(lds)); break;
     case BC_LANE32: lane_tile<32, CSR>(a, tile, *reinterpret_cast<LaneShared<32, CSR> *>(lds)); break;
+    case BC_G8:
+        if (KB <= 2) group_bin<8, CSR, KB>(a, e, tile, tiles, lds);
+        break;
     case BC_G16: group_bin<16, CSR, KB>(a, e, tile, tiles, lds); break;
     case BC_G32:
-        if (KB == 8) group_bin<32, CSR, KB>(a, e, tile, tiles, lds);
+        if (KB != 4) group_bin<32, CSR, KB>(a, e, tile, tiles, lds);
         break;
     case BC_G64: group_bin<64, CSR, KB>(a, e, tile, tiles, lds); break;
     default: group_bin<BLOCK, CSR, KB>(a, e, tile, tiles, lds); break;
@@ -978,8 +995,8 @@ __device__ __forceinline__ void group_decode_tile(const DecodeArgs &a, uint32_t 
     constexpr int NG = BLOCK / G;
     uint32_t *xs = st.xs;
     const uint32_t gid = threadIdx.x / G, gl = threadIdx.x % G, T = 1u << logT;
-    uint64_t *stage = lds + (uint64_t)gid * (T + T / 4);
-    uint32_t *list = (uint32_t *)(stage + T);
+    uint64_t *stage = lds + (uint64_t)gid * (T / 2 + T / 4);
+    uint32_t *list = (uint32_t *)(stage + T / 2);
     GroupShared<G> *sh = &st.gsh[gid];
     const uint32_t p = begin + tile * NG + gid;
     if (p >= end) return;   // whole groups; a workgroup of one group is never empty
@@ -988,7 +1005,7 @@ __device__ __forceinline__ void group_decode_tile(const DecodeArgs &a, uint32_t 
     const uint32_t d = (uint32_t)(a.crow[p + 1] - o0);
     const uint4 m = a.meta[p];
     if (gl == 0) clear_runs(sh);
-    with_record<G>(a.words, start, a.offs[p + 1], gl, stage, T, [&](auto &&at) {
+    with_record<G>(a.words, start, a.offs[p + 1], gl, stage, T / 2, [&](auto &&at) {
         uint32_t done = 0, total;
         for (uint32_t j0 = 0; j0 < m.y; j0 += G) {
             const uint32_t j = j0 + gl;
@@ -1002,7 +1019,7 @@ __device__ __forceinline__ void group_decode_tile(const DecodeArgs &a, uint32_t 
             if (c) {
                 auto r = at(start + m.x + (uint64_t)SEG_BITS * j);
                 read_interval_segment(r, v, [&](uint32_t l, uint32_t len) {
-                    put_run<G>(sh, list, o, l, len);
+                    put_run(sh, list, o, l, len);
                     o += len;
                 });
             }
@@ -1034,7 +1051,9 @@ __device__ __forceinline__ void decode_bin(const DecodeArgs &a, const BinTable::
     case BC_LANE16: lane(reinterpret_cast<LaneDecodeShared<16> *>(lds)); break;
     case BC_LANE32: lane(reinterpret_cast<LaneDecodeShared<32> *>(lds)); break;
     case BC_LANE64: lane(reinterpret_cast<LaneDecodeShared<64> *>(lds)); break;
+    case BC_G8: group(reinterpret_cast<GroupDecodeStatic<8> *>(lds)); break;
     case BC_G16: group(reinterpret_cast<GroupDecodeStatic<16> *>(lds)); break;
+    case BC_G32: group(reinterpret_cast<GroupDecodeStatic<32> *>(lds)); break;
     case BC_G64: group(reinterpret_cast<GroupDecodeStatic<64> *>(lds)); break;
     default: group(reinterpret_cast<GroupDecodeStatic<BLOCK> *>(lds)); break;
     }
