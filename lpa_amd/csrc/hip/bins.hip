@@ -146,7 +146,8 @@ void launch_bin(const Bin &b, StepArgs a, bool as_csr, uint32_t quarter_max, hip
 
 // Workgroups up to which a bin shares its launch with other small ones: with
 // the LDS of the largest (up to 50 KB), three to four workgroups fit a CU, so
-// about this many run at once.  20 steps of R-MAT 12 2.71 -> 1.42 ms (a step
+// about this many run at once (4096: 3 to 5 % slower on R-MAT 19 and 20, all in
+// one 9 % slower).  20 steps of R-MAT 12 2.71 -> 1.42 ms (a step
 // of 13 launches -> 4), R-MAT 20 K = 1 10.0 -> 9.0, R-MAT 19 two-kernel 8.3 ->
 // 6.9, R-MAT 17 K = 64 44.7 -> 34.2, copying graphs 6.9 -> 5.5 (K = 1) and 10.6 ->
 // 6.9 ms (K = 5).

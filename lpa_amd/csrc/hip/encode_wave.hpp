@@ -336,12 +336,12 @@ __device__ __forceinline__ void wave_write(WaveRing *R, uint64_t *words, uint64_
 
 }  // namespace enc
 
-// Record lengths of the positions whose rows have LANE_ROW < d <= long_min
-// ids, a wave each; *err as k_encode_len.
+// Record lengths of the positions from `first` on whose rows have LANE_ROW < d
+// <= long_min ids, a wave each; *err as k_encode_len.
 __global__ void __launch_bounds__(64 * enc::ENC_WAVES) k_encode_wave_len(
-    const uint64_t *__restrict__ row, const uint32_t *__restrict__ col, const uint32_t *__restrict__ vid, uint64_t n_c,
-    uint32_t n, uint64_t *__restrict__ len, unsigned long long *__restrict__ err, uint32_t long_min) {
-    const uint64_t p = (uint64_t)blockIdx.x * enc::ENC_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t *__restrict__ row, const uint32_t *__restrict__ col, const uint32_t *__restrict__ vid,
+    uint64_t first, uint64_t n_c, uint32_t n, uint64_t *__restrict__ len, unsigned long long *__restrict__ err, uint32_t long_min) {
+    const uint64_t p = first + (uint64_t)blockIdx.x * enc::ENC_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (p >= n_c) return;
     const uint32_t v = vid[p];
     const uint64_t r0 = row[v], r1 = row[v + 1];
@@ -355,11 +355,11 @@ __global__ void __launch_bounds__(64 * enc::ENC_WAVES) k_encode_wave_len(
 }
 
 __global__ void __launch_bounds__(64 * enc::ENC_WAVES) k_encode_wave_write(
-    const uint64_t *__restrict__ row, const uint32_t *__restrict__ col, const uint32_t *__restrict__ vid, uint64_t n_c,
-    const uint64_t *__restrict__ offs, uint64_t *words, uint32_t long_min) {
+    const uint64_t *__restrict__ row, const uint32_t *__restrict__ col, const uint32_t *__restrict__ vid,
+    uint64_t first, uint64_t n_c, const uint64_t *__restrict__ offs, uint64_t *words, uint32_t long_min) {
     __shared__ enc::WaveRing ring[enc::ENC_WAVES];
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint64_t p = (uint64_t)blockIdx.x * enc::ENC_WAVES + w;
+    const uint64_t p = first + (uint64_t)blockIdx.x * enc::ENC_WAVES + w;
     if (p >= n_c) return;
     const uint32_t v = vid[p];
     const uint64_t r0 = row[v], r1 = row[v + 1];

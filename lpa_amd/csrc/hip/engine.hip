@@ -740,6 +740,14 @@ void lpa_engine::step_bin_times(std::vector<float> &bin_ms, std::vector<float> &
     for (auto &x : ev) (void)hipEventDestroy(x);
 }
 
+// Launches of at most 2^23 workgroups of 256 (HIP refuses 2^32 threads or
+// more) over n items, per_block to a workgroup: fn(first item, grid).
+template <class F> static void in_launches(uint64_t n, uint64_t per_block, F &&fn) {
+    const uint64_t most = (1ull << 23) * per_block;
+    for (uint64_t i = 0; i < n; i += most)
+        fn(i, dim3((unsigned)((std::min(n - i, most) + per_block - 1) / per_block)));
+}
+
 // Validation pass over the device stream (words0, offs0, vid0 and the host
 // copies set): degrees, features, segment metadata; rejects malformed
 // records.
@@ -751,9 +759,10 @@ static void finish_graph(lpa_engine *e) {
     e->meta0.alloc(n_c);
     if (!e->err.p) e->err.alloc(1);
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, e->stream, e->err.p, (uint64_t)1, 0ull);
-    if (n_c)
-        hipLaunchKernelGGL(k_scan_records, dim3((unsigned)((n_c * SCAN_G + 255) / 256)), dim3(256), 0, e->stream, e->words0.p,
-                           e->offs0.p, e->vid0.p, n_c, (uint32_t)e->n, ddeg.p, e->feat0.p, e->meta0.p, e->err.p);
+    in_launches(n_c, 256 / SCAN_G, [&](uint64_t first, dim3 g) {
+        hipLaunchKernelGGL(k_scan_records, g, dim3(256), 0, e->stream, e->words0.p, e->offs0.p, e->vid0.p, first, n_c,
+                           (uint32_t)e->n, ddeg.p, e->feat0.p, e->meta0.p, e->err.p);
+    });
     HIPCHK(hipGetLastError());
     unsigned long long bad = 0;
     HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
@@ -774,16 +783,20 @@ static void launch_encode_len(hipStream_t s, const uint64_t *row, const uint32_t
     if (n_c == 0) return;
     hipLaunchKernelGGL(k_encode_len, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, s, row, col, vid, n_c,
                        (uint32_t)n, len, err, enc::LANE_ROW);
-    hipLaunchKernelGGL(k_encode_wave_len, dim3((unsigned)((n_c + enc::ENC_WAVES - 1) / enc::ENC_WAVES)),
-                       dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, n_c, (uint32_t)n, len, err, long_min);
+    in_launches(n_c, enc::ENC_WAVES, [&](uint64_t first, dim3 g) {
+        hipLaunchKernelGGL(k_encode_wave_len, g, dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, first, n_c,
+                           (uint32_t)n, len, err, long_min);
+    });
 }
 static void launch_encode_write(hipStream_t s, const uint64_t *row, const uint32_t *col, const uint32_t *vid,
                                 uint64_t n_c, const uint64_t *offs, uint64_t *words, uint32_t long_min) {
     if (n_c == 0) return;
     hipLaunchKernelGGL(k_encode_write, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, s, row, col, vid, n_c, offs,
                        words, enc::LANE_ROW);
-    hipLaunchKernelGGL(k_encode_wave_write, dim3((unsigned)((n_c + enc::ENC_WAVES - 1) / enc::ENC_WAVES)),
-                       dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, n_c, offs, words, long_min);
+    in_launches(n_c, enc::ENC_WAVES, [&](uint64_t first, dim3 g) {
+        hipLaunchKernelGGL(k_encode_wave_write, g, dim3(64 * enc::ENC_WAVES), 0, s, row, col, vid, first, n_c, offs,
+                           words, long_min);
+    });
 }
 
 // ------------------------------------------------------------------ C ABI
@@ -1735,13 +1748,14 @@ int lpa_labels_init(lpa_engine *e, const uint32_t *labels) {
                 b.alloc(tot);
             }
         const uint32_t seed = e->semi ? SEED_BIT : 0u;
-        const dim3 g((unsigned)((tot + 1023) / 1024));
         if (labels && tot)
             e->link.in(e->L[0].p, labels, tot * sizeof(uint32_t), e->stream);
-        if (tot && labels)
-            hipLaunchKernelGGL(k_labels_given, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, tot, seed);
-        else if (tot)
-            hipLaunchKernelGGL(k_labels_own, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, tot, e->K, seed);
+        in_launches(tot, 1024, [&](uint64_t first, dim3 g) {
+            if (labels)
+                hipLaunchKernelGGL(k_labels_given, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, first, tot, seed);
+            else
+                hipLaunchKernelGGL(k_labels_own, g, dim3(256), 0, e->stream, e->L[0].p, e->L[1].p, first, tot, e->K, seed);
+        });
         HIPCHK(hipGetLastError());
         e->cur = 0;
         e->sync();

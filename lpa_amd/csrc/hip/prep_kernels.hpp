@@ -141,13 +141,13 @@ constexpr uint32_t SCAN_G = 16;
 constexpr uint64_t SCAN_LONG = 64 * SEG_BITS;
 __global__ void __launch_bounds__(256) k_scan_records(const uint64_t *__restrict__ W,
                                                       const uint64_t *__restrict__ offs,
-                                                      const uint32_t *__restrict__ vid, uint64_t n_c,
-                                                      uint32_t n, uint32_t *__restrict__ deg,
+                                                      const uint32_t *__restrict__ vid, uint64_t start,
+                                                      uint64_t n_c, uint32_t n, uint32_t *__restrict__ deg,
                                                       float *__restrict__ feat, uint4 *__restrict__ meta,
                                                       unsigned long long *__restrict__ err) {
     constexpr uint32_t PER = 256 / SCAN_G;
     __shared__ ScanPart parts[4];
-    const uint64_t first = (uint64_t)blockIdx.x * PER;
+    const uint64_t first = start + (uint64_t)blockIdx.x * PER;
     auto finish = [&](uint64_t p, bool ok, const ScanPart &s, const uint4 &m, uint64_t bits) {
         if (!ok) atomicCAS(err, 0ull, (unsigned long long)p + 1);
         const uint64_t d = ok ? s.d : 0;
@@ -300,9 +300,9 @@ __global__ void __launch_bounds__(256) k_calibration_gather(const uint32_t *__re
 // i / K, or'ed with `seed` (the clamp bit in semi-supervised mode).  Bound by
 // the stores: 134 MB per buffer (4 M vertices, 8 vectors) in 0.06 ms, where
 // filling on the host, uploading twice and allocating anew took 48 ms.
-__global__ void __launch_bounds__(256) k_labels_own(uint32_t *__restrict__ a, uint32_t *__restrict__ b, uint64_t tot,
-                                                    uint32_t K, uint32_t seed) {
-    const uint64_t i0 = 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+__global__ void __launch_bounds__(256) k_labels_own(uint32_t *__restrict__ a, uint32_t *__restrict__ b,
+                                                    uint64_t first, uint64_t tot, uint32_t K, uint32_t seed) {
+    const uint64_t i0 = first + 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
     if (i0 >= tot) return;
     uint32_t v = (uint32_t)(i0 / K), k = (uint32_t)(i0 - (uint64_t)v * K), x[4];
 #pragma unroll
@@ -323,9 +323,9 @@ __global__ void __launch_bounds__(256) k_labels_own(uint32_t *__restrict__ a, ui
 
 // Given start labels (already in a): labelled entries of a get `seed` or'ed
 // in, and b becomes a copy.
-__global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, uint32_t *__restrict__ b, uint64_t tot,
-                                                      uint32_t seed) {
-    const uint64_t i0 = 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+__global__ void __launch_bounds__(256) k_labels_given(uint32_t *__restrict__ a, uint32_t *__restrict__ b,
+                                                      uint64_t first, uint64_t tot, uint32_t seed) {
+    const uint64_t i0 = first + 4 * ((uint64_t)blockIdx.x * 256 + threadIdx.x);
     if (i0 >= tot) return;
     auto mark = [&](uint32_t x) { return x == 0xFFFFFFFFu ? x : x | seed; };
     if (i0 + 4 <= tot) {

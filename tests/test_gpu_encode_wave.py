@@ -73,3 +73,25 @@ def test_bad_rows_are_rejected(d):
         with pytest.raises(L.LpaError):
             e.encode_csr(row, col, 0)
         e.close()
+
+
+def test_more_rows_than_one_launch_holds():
+    """2^26 rows are 2^32 threads at a wave each: several launches, with rows
+    for the wave encoder at both sides of every joint and at the end"""
+    n = (1 << 26) + 70
+    d = np.zeros(n, np.int64)
+    for at in (0, (1 << 25) - 1, 1 << 25, (1 << 26) - 1, 1 << 26, n - 1):
+        d[at] = 40
+    row = np.zeros(n + 1, np.uint64)
+    np.cumsum(d, out=row[1:].view(np.int64))
+    col = np.concatenate([np.arange(40, dtype=np.uint32) * (3 + i) + i for i in range(6)])
+    g = L.Csr.from_arrays(row, col)
+    cgr = g.encode(0, 128)
+    e = L.Engine(0)
+    e.encode_csr(g.row, g.col, 0)
+    words, offs, _, nbits = e.stream()
+    assert nbits == cgr.nbits and np.array_equal(offs, cgr.offsets)
+    host = np.frombuffer(cgr.stream_bytes(), np.uint8)
+    assert np.array_equal(words.astype(">u8").view(np.uint8)[:len(host)], host)
+    deg = e.degrees()
+    assert np.array_equal(deg, d)
