@@ -24,7 +24,8 @@ struct HostLinkError : std::runtime_error {
 
 // One per engine or model, used by one host thread at a time.  The slots (16
 // MiB of pinned memory) cost about 2 ms to make, so the copies go to the
-// runtime until WORTH bytes have been copied; they are freed with the object.
+// runtime until WORTH bytes have been copied, and where the slots cannot be
+// had; they are freed with the object.
 // 134 MB of labels to new host pages: 12.8 -> 3.6 ms; 33 MB of samples in and 13
 // MB of results out: 2.3 -> 1.6 ms.
 class HostLink {
@@ -92,21 +93,29 @@ class HostLink {
 
     bool worth(size_t n) {
         copied_ = copied_ + n < copied_ ? copied_ : copied_ + n;
-        return pinned_ || copied_ >= WORTH;
+        return copied_ >= WORTH && prepare();
     }
 
     static void check(hipError_t e) {
         if (e != hipSuccess) throw HostLinkError(std::string("host copy: ") + hipGetErrorString(e));
     }
-    void prepare() {
-        if (!pinned_) check(hipHostMalloc((void **)&pinned_, SLOTS * CHUNK, hipHostMallocDefault));
+    bool prepare() {
+        if (!pinned_ && hipHostMalloc((void **)&pinned_, SLOTS * CHUNK, hipHostMallocDefault) != hipSuccess) {
+            pinned_ = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
         for (hipEvent_t &x : ev_)
-            if (!x) check(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+            if (!x && hipEventCreateWithFlags(&x, hipEventDisableTiming) != hipSuccess) {
+                x = nullptr;
+                (void)hipGetLastError();
+                return false;
+            }
+        return true;
     }
     // piece(slot, at, len) for every chunk, slot w's chunks in order by thread
     // w (this one is thread 0).
     template <class Piece> void run(size_t n, Piece &&piece) {
-        prepare();
         int device = 0;
         check(hipGetDevice(&device));
         const size_t chunks = (n + CHUNK - 1) / CHUNK;
