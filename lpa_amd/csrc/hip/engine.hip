@@ -2068,7 +2068,7 @@ struct lpa_mlp {
 // kept at 64; a single gradient spreads over the device.
 constexpr uint32_t MLP_PARTS_TRAIN = 64, MLP_PARTS_MAX = 256;
 static uint32_t mlp_parts(uint64_t n, uint32_t most) {
-    const uint64_t per = MLP_WAVES * MLP_TILE;
+    const uint64_t per = MLP_CHUNK;
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + per - 1) / per, most));
 }
 

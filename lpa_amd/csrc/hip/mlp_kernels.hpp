@@ -10,7 +10,7 @@
 //   k_mlp_forward   y = f(x) for n samples, one lane per sample
 //   k_mlp_step      one training batch: the Adam update of the previous batch,
 //                   then the mean-squared error over the measured outputs
-//                   (mask) and its gradient, on the matrix cores
+//                   (mask) and its gradient, the layers on the matrix cores
 //   k_mlp_sum       loss and gradient of a batch from the workgroups' partials
 // Parameter layout (floats): W1[32][8] b1[32] W2[32][32] b2[32] W3[3][32] b3[3].
 #pragma once
@@ -77,14 +77,19 @@ constexpr int MLP_STRIDE = 1444;
 static_assert(MLP_NPARAM + 1 == MLP_STRIDE && MLP_STRIDE % 4 == 0, "the loss follows the gradient");
 constexpr int MLP_WAVES = 4;                  // waves of a k_mlp_step workgroup
 constexpr int MLP_TILE = 16;                  // samples per wave and round (one MFMA tile)
+constexpr int MLP_CHUNK = MLP_WAVES * MLP_TILE;   // samples per workgroup and round
+static_assert(64 * MLP_WAVES == MLP_H * MLP_IN && 64 * MLP_WAVES == 16 * 16, "a lane's sums");
 
 // Adam of one step; c1 = 1/(1-b1^t), c2 = 1/(1-b2^t) are its bias corrections.
+// (Which products are fused is spelled out, so that the same bits come from
+// every place that this is inlined in.)
 struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;
 };
 __device__ __forceinline__ void adam_update(const AdamArgs &k, float g, float &p, float &m1, float &m2) {
-    const float a = k.b1 * m1 + (1.f - k.b1) * g;
-    const float b = k.b2 * m2 + (1.f - k.b2) * g * g;
+#pragma clang fp contract(off)
+    const float a = __builtin_fmaf(1.f - k.b1, g, k.b1 * m1);
+    const float b = __builtin_fmaf(g, (1.f - k.b2) * g, k.b2 * m2);
     m1 = a;
     m2 = b;
     const float ah = a * k.c1;
@@ -92,31 +97,36 @@ __device__ __forceinline__ void adam_update(const AdamArgs &k, float g, float &p
     p -= k.lr * ah / (sqrtf(bh) + k.eps);
 }
 
-// Sum over the partials of the four values at 4 * i4, in a fixed order
-// (four interleaved sums, so that the loads do not wait for each other).
+// Sum over the partials of the four values at 4 * i4: four partials (256
+// samples) together, then those sums one after the other.
 __device__ __forceinline__ f32x4 mlp_sum_partials(const float *__restrict__ part, uint32_t np, int i4) {
-    f32x4 s[4] = {};
+    f32x4 s = {};
     const f32x4 *src = reinterpret_cast<const f32x4 *>(part) + i4;
     uint32_t w = 0;
     for (; w + 8 <= np; w += 8) {
         f32x4 x[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) x[u] = src[(uint64_t)(w + u) * (MLP_STRIDE / 4)];
-#pragma unroll
-        for (int u = 0; u < 8; u++) s[u & 3] += x[u];
+        s += ((x[0] + x[1]) + x[2]) + x[3];
+        s += ((x[4] + x[5]) + x[6]) + x[7];
     }
-    for (; w < np; w++) s[w & 3] += src[(uint64_t)w * (MLP_STRIDE / 4)];
-    return (s[0] + s[1]) + (s[2] + s[3]);
+    while (w < np) {
+        f32x4 x = src[(uint64_t)w++ * (MLP_STRIDE / 4)];
+        for (; w < np && w % 4; w++) x += src[(uint64_t)w * (MLP_STRIDE / 4)];
+        s += x;
+    }
+    return s;
 }
 
 // LDS of k_mlp_step: the weights with rows padded against bank conflicts
-// (W3 to 16 rows, the last 13 zero), and per wave a staging area of the
-// tile's values, one row per feature with its 16 samples (stride 20: rows
-// 16-byte aligned, four samples per read).
+// (W3 to 16 rows, the last 13 zero), and per wave a staging area of its 16
+// samples' values, one row per feature (stride 20: rows 16-byte aligned, four
+// samples per read, and 16 rows side by side meet every bank once).
 struct MlpShared {
     static constexpr int S2 = 36, SROW = 20;
-    static constexpr int DZ2 = 0, H1 = 32, DZ1 = 64, X = 96, DY = 112, H2 = 128, ROWS = 160;
+    static constexpr int DZ2 = 0, H1 = 32, DZ1 = 64, H2 = 96, X = 128, ONE = 136, DY = 137, ROWS = 140;
     float w1[MLP_H * MLP_IN], b1[MLP_H], w2[MLP_H * S2], b2[MLP_H], w3[16 * S2], b3[16];
+    float loss[MLP_WAVES];
     __align__(16) float stage[MLP_WAVES][ROWS * SROW];
     __device__ __forceinline__ void put(int i, float p) {
         if (i < MLP_B1) w1[i] = p;
@@ -127,7 +137,16 @@ struct MlpShared {
         else b3[i - MLP_B3] = p;
     }
 };
-static_assert(MLP_WAVES * MLP_STRIDE <= MLP_WAVES * MlpShared::ROWS * MlpShared::SROW, "partials reuse the staging area");
+
+// Feature in row m of a 16-row accumulator or weight tile (its own inverse).
+__device__ __forceinline__ int mlp_feature(int m) { return 4 * (m & 3) + (m >> 2); }
+
+// One more term of a gradient, its product rounded first.
+__device__ __forceinline__ void mlp_add(float &acc, float a, float b) {
+#pragma clang fp contract(off)
+    const float p = a * b;
+    acc += p;
+}
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -142,13 +161,25 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 // idx[0..n) (or 0..n-1), of which every workgroup leaves its share in
 // part_out.
 //
-// A wave takes 16 samples at a time, and every product runs on the matrix
-// cores in FP32 (16x16x4 tiles): activations are held as [feature][sample]
-// tiles, whose accumulator registers (rows 4g + r of lane group g) are used
-// as the next product's operand as they are, with the weights read in the
-// same order of the inner index.  Only the gradients, which contract over
-// the samples, need the transposed tiles: they pass through LDS.  Biases
-// take a constant-one feature (row 8 of the inputs' tile).
+// A workgroup takes 64 samples at a time, a wave 16 of them, whose way through
+// the layers and back runs on the matrix cores in FP32 (16x16x4 tiles):
+// activations are held as [feature][sample] tiles, whose accumulator registers
+// are used as the next product's operand as they are.
+//
+// Every sum is taken in the order of a lane that walks over the layers sample
+// by sample, bit for bit.  That matters where a pre-activation is a rounding
+// away from 0: another order flips the unit, and Adam turns the lone gradient
+// of a nearly dead unit into a full step (parameters 5e-5 apart after two
+// epochs of 98 batches, 1e-7 otherwise).  An MFMA adds its four products to the
+// accumulator one after the other, lane group 0 first, each as a fused
+// multiply-add, so features are placed such that every product takes its
+// inputs in ascending order: accumulator row 4g + r (register r of lane group
+// g) is feature 4r + g (mlp_feature), and register r of the groups is then the
+// next four inputs.  The gradients, which contract over the samples, go
+// through LDS to the vector units: a rounded product and a sum per sample, in
+// the samples' order (5.6 of the 1,443 sums per lane; a contraction on the
+// matrix cores fuses them and takes 0.75 us less per batch).  64 samples make a
+// partial, four partials are summed before they join the others.
 //
 // Bound by latency: a batch of 2048 samples is 32 workgroups of 4 waves.
 // Training on 200,000 samples, two epochs at batch 2048: 3.4 ms, against 255
@@ -162,12 +193,10 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
     __shared__ MlpShared sh;
     using M = MlpShared;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int f = mlp_feature(c);   // the feature whose weights this lane passes
     for (int i = threadIdx.x; i < 13 * M::S2; i += blockDim.x) sh.w3[MLP_OUT * M::S2 + i] = 0.f;
     if (threadIdx.x >= MLP_OUT && threadIdx.x < 16) sh.b3[threadIdx.x] = 0.f;
     float *S = sh.stage[wave];
-    // rows that no tile writes: the unused input features and outputs
-    for (int i = lane; i < 7 * M::SROW; i += 64) S[(M::X + 9) * M::SROW + i] = 0.f;
-    for (int i = lane; i < 13 * M::SROW; i += 64) S[(M::DY + MLP_OUT) * M::SROW + i] = 0.f;
     for (int i4 = threadIdx.x; i4 < MLP_STRIDE / 4; i4 += blockDim.x) {
         f32x4 p = reinterpret_cast<const f32x4 *>(cur)[i4];
         if (np) {
@@ -199,18 +228,29 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
     if (n == 0) return;   // the last update of a run
     __syncthreads();
 
-    f32x4 gw2[2][2] = {}, gw1[2] = {}, gw3[2] = {}, gb2[2] = {}, gb3 = {};
-    float lsum = 0.f;
-    const uint64_t ntiles = (n + MLP_TILE - 1) / MLP_TILE;
-    for (uint64_t tile = (uint64_t)blockIdx.x * MLP_WAVES + wave; tile < ntiles; tile += (uint64_t)gridDim.x * MLP_WAVES) {
-        const uint64_t q = tile * MLP_TILE + c;
+    // this lane's sums: four weights of the second layer, one of the first,
+    // and one of the third or a bias, as products of two staged rows
+    const int t4 = threadIdx.x >> 4, t8 = threadIdx.x >> 3;
+    int ra = M::X, rb = M::X, out = -1;
+    if (threadIdx.x < 96) {
+        ra = M::DY + (threadIdx.x >> 5), rb = M::H2 + (threadIdx.x & 31), out = MLP_W3 + threadIdx.x;
+    } else if (threadIdx.x < 160) {
+        const int j = threadIdx.x & 31;
+        ra = (threadIdx.x < 128 ? M::DZ1 : M::DZ2) + j, rb = M::ONE, out = (threadIdx.x < 128 ? MLP_B1 : MLP_B2) + j;
+    } else if (threadIdx.x < 160 + MLP_OUT) {
+        ra = M::DY + threadIdx.x - 160, rb = M::ONE, out = MLP_B3 + threadIdx.x - 160;
+    }
+    float total[6] = {}, lsum = 0.f;
+    const uint64_t chunks = (n + MLP_CHUNK - 1) / MLP_CHUNK;
+    for (uint64_t chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
+        const uint64_t q = chunk * MLP_CHUNK + wave * MLP_TILE + c;
         const bool valid = q < n;
         const uint64_t t = valid ? (idx ? (uint64_t)idx[q] : q) : 0;
         float x0 = 0.f, x1 = 0.f, tg[MLP_OUT] = {};
         bool mk[MLP_OUT] = {};
         if (valid) {
-            x0 = x[t * MLP_IN + 2 * g];
-            x1 = x[t * MLP_IN + 2 * g + 1];
+            x0 = x[t * MLP_IN + g];
+            x1 = x[t * MLP_IN + 4 + g];
             if (g == 0) {
 #pragma unroll
                 for (int j = 0; j < MLP_OUT; j++) {
@@ -219,15 +259,15 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
                 }
             }
         }
-        // forward: lane (g, c) holds rows 16 u + 4 g + r of sample c
+        // forward: lane (g, c) holds features 16 u + 4 r + g of sample c
         float h1[2][4], h2[2][4];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             f32x4 z;
 #pragma unroll
-            for (int r = 0; r < 4; r++) z[r] = sh.b1[16 * u + 4 * g + r];
-            z = mfma4(sh.w1[(16 * u + c) * MLP_IN + 2 * g], x0, z);
-            z = mfma4(sh.w1[(16 * u + c) * MLP_IN + 2 * g + 1], x1, z);
+            for (int r = 0; r < 4; r++) z[r] = sh.b1[16 * u + 4 * r + g];
+            z = mfma4(sh.w1[(16 * u + f) * MLP_IN + g], x0, z);
+            z = mfma4(sh.w1[(16 * u + f) * MLP_IN + 4 + g], x1, z);
 #pragma unroll
             for (int r = 0; r < 4; r++) h1[u][r] = z[r] > 0.f ? z[r] : 0.f;
         }
@@ -235,21 +275,21 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
         for (int u = 0; u < 2; u++) {
             f32x4 z;
 #pragma unroll
-            for (int r = 0; r < 4; r++) z[r] = sh.b2[16 * u + 4 * g + r];
+            for (int r = 0; r < 4; r++) z[r] = sh.b2[16 * u + 4 * r + g];
 #pragma unroll
             for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) z = mfma4(sh.w2[(16 * u + c) * M::S2 + 16 * k + 4 * g + r], h1[k][r], z);
+                for (int r = 0; r < 4; r++) z = mfma4(sh.w2[(16 * u + f) * M::S2 + 16 * k + 4 * r + g], h1[k][r], z);
 #pragma unroll
             for (int r = 0; r < 4; r++) h2[u][r] = z[r] > 0.f ? z[r] : 0.f;
         }
         f32x4 y;
 #pragma unroll
-        for (int r = 0; r < 4; r++) y[r] = sh.b3[4 * g + r];
+        for (int r = 0; r < 4; r++) y[r] = sh.b3[4 * g + r];   // outputs in row order: only three
 #pragma unroll
         for (int k = 0; k < 2; k++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) y = mfma4(sh.w3[c * M::S2 + 16 * k + 4 * g + r], h2[k][r], y);
+            for (int r = 0; r < 4; r++) y = mfma4(sh.w3[c * M::S2 + 16 * k + 4 * r + g], h2[k][r], y);
         // errors: outputs 0..2 of sample c are in lane group 0
         float dy[MLP_OUT], l = 0.f;
         bool any = false;
@@ -269,7 +309,7 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
         float dz2[2][4], dz1[2][4];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            const f32x4 z = mfma4(sh.w3[g * M::S2 + 16 * u + c], dyg, f32x4{});
+            const f32x4 z = mfma4(sh.w3[g * M::S2 + 16 * u + f], dyg, f32x4{});
 #pragma unroll
             for (int r = 0; r < 4; r++) dz2[u][r] = h2[u][r] > 0.f ? z[r] : 0.f;
         }
@@ -279,7 +319,7 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
 #pragma unroll
             for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) z = mfma4(sh.w2[(16 * k + 4 * g + r) * M::S2 + 16 * u + c], dz2[k][r], z);
+                for (int r = 0; r < 4; r++) z = mfma4(sh.w2[(16 * k + 4 * r + g) * M::S2 + 16 * u + f], dz2[k][r], z);
 #pragma unroll
             for (int r = 0; r < 4; r++) dz1[u][r] = h1[u][r] > 0.f ? z[r] : 0.f;
         }
@@ -288,79 +328,52 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
         for (int u = 0; u < 2; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int f = (16 * u + 4 * g + r) * M::SROW + c;
-                S[M::DZ2 * M::SROW + f] = live ? dz2[u][r] : 0.f;
-                S[M::DZ1 * M::SROW + f] = live ? dz1[u][r] : 0.f;
-                S[M::H1 * M::SROW + f] = live ? h1[u][r] : 0.f;
-                S[M::H2 * M::SROW + f] = live ? h2[u][r] : 0.f;
+                const int at = (16 * u + 4 * r + g) * M::SROW + c;
+                S[M::DZ2 * M::SROW + at] = live ? dz2[u][r] : 0.f;
+                S[M::DZ1 * M::SROW + at] = live ? dz1[u][r] : 0.f;
+                S[M::H1 * M::SROW + at] = live ? h1[u][r] : 0.f;
+                S[M::H2 * M::SROW + at] = live ? h2[u][r] : 0.f;
             }
-        S[(M::X + 2 * g) * M::SROW + c] = live ? x0 : 0.f;
-        S[(M::X + 2 * g + 1) * M::SROW + c] = live ? x1 : 0.f;
+        S[(M::X + g) * M::SROW + c] = live ? x0 : 0.f;
+        S[(M::X + 4 + g) * M::SROW + c] = live ? x1 : 0.f;
         if (g == 0) {
-            S[(M::X + 8) * M::SROW + c] = live ? 1.f : 0.f;
+            S[M::ONE * M::SROW + c] = live ? 1.f : 0.f;
 #pragma unroll
             for (int j = 0; j < MLP_OUT; j++) S[(M::DY + j) * M::SROW + c] = dy[j];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // gradients: products over the 16 samples, four per lane group
-        auto rows = [&](int base) { return *reinterpret_cast<const f32x4 *>(&S[(base + c) * M::SROW + 4 * g]); };
-        const f32x4 vx = rows(M::X), vy = rows(M::DY);
-        f32x4 a2[2], a1[2], v1[2], v2[2];
+        __syncthreads();
+        float acc[6] = {};
+        for (int w = 0; w < MLP_WAVES; w++)
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            a2[u] = rows(M::DZ2 + 16 * u);
-            a1[u] = rows(M::DZ1 + 16 * u);
-            v1[u] = rows(M::H1 + 16 * u);
-            v2[u] = rows(M::H2 + 16 * u);
-        }
+            for (int s = 0; s < MLP_TILE; s += 4) {
+                auto row = [&](int i) { return *reinterpret_cast<const f32x4 *>(&sh.stage[w][i * M::SROW + s]); };
+                const f32x4 a0 = row(M::DZ2 + t4), a1 = row(M::DZ2 + 16 + t4), a2 = row(M::DZ1 + t8), a3 = row(ra);
+                const f32x4 v0 = row(M::H1 + c), v1 = row(M::H1 + 16 + c), v2 = row(M::X + (lane & 7)), v3 = row(rb);
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-#pragma unroll
-                for (int k = 0; k < 2; k++) gw2[u][k] = mfma4(a2[u][s], v1[k][s], gw2[u][k]);
-                gw1[u] = mfma4(a1[u][s], vx[s], gw1[u]);
-                gb2[u] = mfma4(a2[u][s], vx[s], gb2[u]);
-                gw3[u] = mfma4(vy[s], v2[u][s], gw3[u]);
+                for (int e = 0; e < 4; e++) {
+                    mlp_add(acc[0], a0[e], v0[e]);
+                    mlp_add(acc[1], a0[e], v1[e]);
+                    mlp_add(acc[2], a1[e], v0[e]);
+                    mlp_add(acc[3], a1[e], v1[e]);
+                    mlp_add(acc[4], a2[e], v2[e]);
+                    mlp_add(acc[5], a3[e], v3[e]);
+                }
             }
-            gb3 = mfma4(vy[s], vx[s], gb3);
-        }
-        __builtin_amdgcn_wave_barrier();   // the staging rows are written again next round
+#pragma unroll
+        for (int i = 0; i < 6; i++) total[i] += acc[i];
+        __syncthreads();   // the staging rows are written again next round
     }
-    // the waves' sums, then the workgroup's partial
-    __syncthreads();
-    float *R = &sh.stage[0][0] + wave * MLP_STRIDE;
+    // the workgroup's partial
+    float *R = part_out + (uint64_t)blockIdx.x * MLP_STRIDE;
 #pragma unroll
-    for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int f = 16 * u + 4 * g + r;
-#pragma unroll
-            for (int k = 0; k < 2; k++) R[MLP_W2 + f * MLP_H + 16 * k + c] = gw2[u][k][r];
-            if (c < MLP_IN) R[MLP_W1 + f * MLP_IN + c] = gw1[u][r];
-            if (c == 8) {
-                R[MLP_B1 + f] = gw1[u][r];
-                R[MLP_B2 + f] = gb2[u][r];
-            }
-            if (g == 0 && r < MLP_OUT) R[MLP_W3 + r * MLP_H + 16 * u + c] = gw3[u][r];
-        }
-    if (g == 0 && c == 8) {
-#pragma unroll
-        for (int r = 0; r < MLP_OUT; r++) R[MLP_B3 + r] = gb3[r];
-    }
+    for (int i = 0; i < 4; i++) R[MLP_W2 + (t4 + 16 * (i >> 1)) * MLP_H + c + 16 * (i & 1)] = total[i];
+    R[MLP_W1 + threadIdx.x] = total[4];
+    if (out >= 0) R[out] = total[5];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
-    if (lane == 0) R[MLP_NPARAM] = lsum;
+    if (lane == 0) sh.loss[wave] = lsum;
     __syncthreads();
-    const f32x4 *all = reinterpret_cast<const f32x4 *>(&sh.stage[0][0]);
-    for (int i4 = threadIdx.x; i4 < MLP_STRIDE / 4; i4 += blockDim.x) {
-        f32x4 s = all[i4];
-#pragma unroll
-        for (int w = 1; w < MLP_WAVES; w++) s += all[w * (MLP_STRIDE / 4) + i4];
-        reinterpret_cast<f32x4 *>(part_out)[(uint64_t)blockIdx.x * (MLP_STRIDE / 4) + i4] = s;
-    }
+    if (threadIdx.x == 0) R[MLP_NPARAM] = (sh.loss[0] + sh.loss[1]) + (sh.loss[2] + sh.loss[3]);
 }
 
 // Gradient and loss (MLP_STRIDE floats) of a batch from its partials.
