@@ -148,6 +148,10 @@ __device__ __forceinline__ void mlp_add(float &acc, float a, float b) {
     acc += p;
 }
 
+__device__ __forceinline__ bool mlp_finite(f32x4 x) {
+    return x[0] * 0.f + x[1] * 0.f + x[2] * 0.f + x[3] * 0.f == 0.f;   // an infinity times 0 is NaN
+}
+
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -306,23 +310,60 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
         const float e0 = __shfl(dy[0], c, 64), e1 = __shfl(dy[1], c, 64), e2 = __shfl(dy[2], c, 64);
         const float dyg = g == 0 ? e0 : g == 1 ? e1 : g == 2 ? e2 : 0.f;
         // back through the layers
-        float dz2[2][4], dz1[2][4];
+        f32x4 dz2[2], dz1[2];
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const f32x4 z = mfma4(sh.w3[g * M::S2 + 16 * u + f], dyg, f32x4{});
+        for (int u = 0; u < 2; u++) dz2[u] = mfma4(sh.w3[g * M::S2 + 16 * u + f], dyg, f32x4{});
+        if (__any(!mlp_finite(dz2[0]) || !mlp_finite(dz2[1]))) {   // rare: 0 times a weight that is not finite counts as 0
 #pragma unroll
-            for (int r = 0; r < 4; r++) dz2[u][r] = h2[u][r] > 0.f ? z[r] : 0.f;
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float *w = &sh.w3[16 * u + 4 * r + g];
+                    float z = e0 != 0.f ? e0 * w[0] : 0.f;
+                    if (e1 != 0.f) z = __builtin_fmaf(e1, w[M::S2], z);
+                    if (e2 != 0.f) z = __builtin_fmaf(e2, w[2 * M::S2], z);
+                    dz2[u][r] = z;
+                }
         }
 #pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) dz2[u][r] = h2[u][r] > 0.f ? dz2[u][r] : 0.f;
+#pragma unroll
         for (int u = 0; u < 2; u++) {
-            f32x4 z = {};
+            dz1[u] = f32x4{};
 #pragma unroll
             for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) z = mfma4(sh.w2[(16 * k + 4 * r + g) * M::S2 + 16 * u + f], dz2[k][r], z);
-#pragma unroll
-            for (int r = 0; r < 4; r++) dz1[u][r] = h1[u][r] > 0.f ? z[r] : 0.f;
+                for (int r = 0; r < 4; r++)
+                    dz1[u] = mfma4(sh.w2[(16 * k + 4 * r + g) * M::S2 + 16 * u + f], dz2[k][r], dz1[u]);
         }
+        if (__any(!mlp_finite(dz1[0]) || !mlp_finite(dz1[1]))) {
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    S[(M::DZ2 + 16 * u + 4 * r + g) * M::SROW + c] = dz2[u][r];
+                    dz1[u][r] = 0.f;
+                }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+            for (int j = 0; j < MLP_H; j++) {
+                const float d = S[(M::DZ2 + j) * M::SROW + c];
+                if (d == 0.f) continue;
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) dz1[u][r] = __builtin_fmaf(sh.w2[j * M::S2 + 16 * u + 4 * r + g], d, dz1[u][r]);
+            }
+            __builtin_amdgcn_wave_barrier();   // the rows are written again below
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) dz1[u][r] = h1[u][r] > 0.f ? dz1[u][r] : 0.f;
         // stage [feature][sample]
 #pragma unroll
         for (int u = 0; u < 2; u++)
@@ -342,23 +383,34 @@ __global__ void __launch_bounds__(64 * MLP_WAVES) k_mlp_step(
             for (int j = 0; j < MLP_OUT; j++) S[(M::DY + j) * M::SROW + c] = dy[j];
         }
         __syncthreads();
-        float acc[6] = {};
-        for (int w = 0; w < MLP_WAVES; w++)
+        float acc[6];
+        auto sums = [&](auto add) {
 #pragma unroll
-            for (int s = 0; s < MLP_TILE; s += 4) {
-                auto row = [&](int i) { return *reinterpret_cast<const f32x4 *>(&sh.stage[w][i * M::SROW + s]); };
-                const f32x4 a0 = row(M::DZ2 + t4), a1 = row(M::DZ2 + 16 + t4), a2 = row(M::DZ1 + t8), a3 = row(ra);
-                const f32x4 v0 = row(M::H1 + c), v1 = row(M::H1 + 16 + c), v2 = row(M::X + (lane & 7)), v3 = row(rb);
+            for (int i = 0; i < 6; i++) acc[i] = 0.f;
+            for (int w = 0; w < MLP_WAVES; w++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    mlp_add(acc[0], a0[e], v0[e]);
-                    mlp_add(acc[1], a0[e], v1[e]);
-                    mlp_add(acc[2], a1[e], v0[e]);
-                    mlp_add(acc[3], a1[e], v1[e]);
-                    mlp_add(acc[4], a2[e], v2[e]);
-                    mlp_add(acc[5], a3[e], v3[e]);
+                for (int s = 0; s < MLP_TILE; s += 4) {
+                    auto row = [&](int i) { return *reinterpret_cast<const f32x4 *>(&sh.stage[w][i * M::SROW + s]); };
+                    const f32x4 a0 = row(M::DZ2 + t4), a1 = row(M::DZ2 + 16 + t4), a2 = row(M::DZ1 + t8), a3 = row(ra);
+                    const f32x4 v0 = row(M::H1 + c), v1 = row(M::H1 + 16 + c), v2 = row(M::X + (lane & 7)), v3 = row(rb);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        add(acc[0], a0[e], v0[e]);
+                        add(acc[1], a0[e], v1[e]);
+                        add(acc[2], a1[e], v0[e]);
+                        add(acc[3], a1[e], v1[e]);
+                        add(acc[4], a2[e], v2[e]);
+                        add(acc[5], a3[e], v3[e]);
+                    }
                 }
-            }
+        };
+        sums([](float &s, float a, float b) { mlp_add(s, a, b); });
+        if (!mlp_finite(f32x4{acc[0], acc[1], acc[2], acc[3]}) || !mlp_finite(f32x4{acc[4], acc[5], 0.f, 0.f})) {
+            asm volatile("" ::: "memory");          // the rows are read again, not kept in 512 registers
+            sums([](float &s, float a, float b) {   // rare, as above: the gradient's factor decides
+                if (a != 0.f) mlp_add(s, a, b);
+            });
+        }
 #pragma unroll
         for (int i = 0; i < 6; i++) total[i] += acc[i];
         __syncthreads();   // the staging rows are written again next round
