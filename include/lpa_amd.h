@@ -88,7 +88,11 @@ typedef struct {
     uint32_t wave_max;      /* deg <= wave_max -> WAVE (0: 512) */
     uint32_t block_max;     /* deg <= block_max -> BLOCK, else the heavy-vertex path (0: LDS limit) */
     uint32_t relayout;      /* records are always reordered so each bin is contiguous; keep 1 */
-    uint32_t quarter_max;   /* WAVE vertices up to this degree use 16-lane groups (0: 128) */
+    uint32_t quarter_max;   /* WAVE vertices whose list holds up to this many ids (a power of two, at
+                               least 32) share a wave (0: 128): 16 lanes each for K = 3 and 4; for
+                               K >= 5 16 lanes up to 64 ids, 32 above; for K <= 2 a value of 128 or
+                               more means 8 to 64 lanes by the list's length, a smaller one 16 lanes
+                               up to it and a whole wave above */
     uint32_t bin_order;     /* vertices inside a bin: 1 by vertex id (neighbouring ids run together),
                                2 by degree, descending; 0: the engine's default (2) */
     uint32_t xcd_tiles;     /* 1: the workgroups one XCD runs take consecutive tiles of a bin (each XCD

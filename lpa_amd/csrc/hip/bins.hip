@@ -26,33 +26,26 @@ template <bool CSR> static void launch_lane(int N, StepArgs a, uint32_t count, h
     }
 }
 
-// label vectors staged per row gather by the group kernels: 8 from K = 5
-// (one gather per neighbour and step at K = 8; with one aggregated match
-// round the kernels stay fast enough at the lower occupancy that even label
-// rows held by the 256 MB last-level cache gain from it), else K rounded
-// down to 4 / 2 / 1.
-static int group_kb(uint32_t K) { return K >= 5 ? 8 : K >= 3 ? 4 : K == 2 ? 2 : 1; }
-
 // instance of the group kernel for a batch size and staged ids per lane
-template <int G, bool CSR> static const void *group_fn(int kb, uint32_t ipl) {
+template <int G, bool CSR> static const void *group_fn(int kb, uint32_t ids) {
     switch (kb) {
     case 1: return (const void *)k_group<G, CSR, 1, 8>;
     case 2: return (const void *)k_group<G, CSR, 2, 8>;
     case 4:
-        return ipl <= 2 ? (const void *)k_group<G, CSR, 4, 2>
-             : ipl <= 4 ? (const void *)k_group<G, CSR, 4, 4> : (const void *)k_group<G, CSR, 4, 8>;
+        return ids == 2 ? (const void *)k_group<G, CSR, 4, 2>
+             : ids == 4 ? (const void *)k_group<G, CSR, 4, 4> : (const void *)k_group<G, CSR, 4, 8>;
     default:
-        return ipl <= 2 ? (const void *)k_group<G, CSR, 8, 2>
-             : ipl <= 4 ? (const void *)k_group<G, CSR, 8, 4> : (const void *)k_group<G, CSR, 8, 8>;
+        return ids == 2 ? (const void *)k_group<G, CSR, 8, 2>
+             : ids == 4 ? (const void *)k_group<G, CSR, 8, 4> : (const void *)k_group<G, CSR, 8, 8>;
     }
 }
 
 template <int G>
 static void launch_group(bool as_csr, dim3 grid, size_t lds, hipStream_t s, const StepArgs &a, uint32_t logT,
                          uint32_t cap) {
-    const uint32_t ipl = (cap + G - 1) / G;
     const int kb = group_kb(a.K);
-    const void *fn = as_csr ? group_fn<G, true>(kb, ipl) : group_fn<G, false>(kb, ipl);
+    const uint32_t ids = staged_ids(kb, cap, G);
+    const void *fn = as_csr ? group_fn<G, true>(kb, ids) : group_fn<G, false>(kb, ids);
     StepArgs args = a;
     void *params[] = {&args, &logT, &cap};
     (void)hipLaunchKernel(fn, grid, dim3(BLOCK), params, lds, s);
@@ -60,8 +53,8 @@ static void launch_group(bool as_csr, dim3 grid, size_t lds, hipStream_t s, cons
 
 template <int G> static void allow_group_lds(int dyn) {
     for (int kb : {1, 2, 4, 8})
-        for (uint32_t ipl : {2u, 4u, 8u})
-            for (const void *f : {group_fn<G, false>(kb, ipl), group_fn<G, true>(kb, ipl)})
+        for (uint32_t ids : {2u, 4u, 8u})
+            for (const void *f : {group_fn<G, false>(kb, ids), group_fn<G, true>(kb, ids)})
                 (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
 }
 
@@ -87,35 +80,6 @@ void bins_allow_lds(int dyn) {
     allow_group_lds<BLOCK>(dyn);
     for (const void *f : {bins_fn(1), bins_fn(2), bins_fn(4), bins_fn(8), (const void *)k_decode_bins})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
-}
-
-// Lanes per vertex of a WAVE bin, as groups per workgroup.  One or two
-// vectors (8 staged ids per lane whatever the group): as few lanes as hold the
-// list, 8 for up to 64 ids to 64 for 512, because a list of d ids is only
-// about d / 20 segments to decode, a lane each.  More vectors: a quarter wave
-// up to quarter_max ids, a wave above, and with 8 vectors per staged gather
-// half waves for 65..128 ids (4 ids per lane) rather than quarter waves (8
-// per lane): half the staged registers, twice the waves resident.
-// (quarter_max below 128 asks for whole waves above it, whatever K.)
-static int decode_groups(uint32_t logT) {
-    const uint32_t cap = 1u << (logT - 1);
-    return cap <= 64 ? 32 : cap <= 128 ? 16 : cap <= 256 ? 8 : 4;
-}
-static int step_groups(uint32_t logT, uint32_t K, uint32_t quarter_max) {
-    if (quarter_max == 0) quarter_max = 128;
-    if (K <= 2 && quarter_max >= 128) return decode_groups(logT);
-    const int ng = wave_groups(logT, quarter_max);
-    return ng == 16 && (1u << (logT - 1)) > 64 && K >= 5 ? 8 : ng;
-}
-// staged ids per lane of the launch of a list of cap ids with groups of G lanes
-static uint32_t staged_ids(int kb, uint32_t cap, uint32_t G) {
-    const uint32_t ipl = (cap + G - 1) / G;
-    return kb <= 2 ? 8 : ipl <= 2 ? 2 : ipl <= 4 ? 4 : 8;
-}
-static size_t step_lds(int ng, uint32_t logT, bool csr, uint32_t K) {
-    const uint32_t cap = 1u << (logT - 1), G = BLOCK / ng;
-    const int kb = group_kb(K);
-    return group_list_inside(csr, K, kb, cap, staged_ids(kb, cap, G) * G) ? (size_t)ng * 8ull << logT : group_lds(ng, logT);
 }
 
 void launch_bin(const Bin &b, StepArgs a, bool as_csr, uint32_t quarter_max, hipStream_t s) {
@@ -166,7 +130,6 @@ struct Merge {
     }
 };
 
-static size_t static_bytes(size_t s) { return (s + 7) / 8 * 8; }
 static uint32_t group_code(int ng) {
     return ng == 1 ? BC_G256 : ng == 4 ? BC_G64 : ng == 8 ? BC_G32 : ng == 16 ? BC_G16 : BC_G8;
 }
@@ -194,6 +157,7 @@ void launch_bins(const std::vector<Bin> &bins, const StepArgs &a, bool all_csr, 
         if (count == 0) continue;
         uint32_t code, wg;
         size_t bytes;
+        bool held = true;
         const bool csr = all_csr || b.csr;
         if (b.kind == LPA_BIN_LANE) {
             wg = (count + BLOCK - 1) / BLOCK;
@@ -202,21 +166,19 @@ void launch_bins(const std::vector<Bin> &bins, const StepArgs &a, bool all_csr, 
             case 8: code = BC_LANE8; bytes = lane_bytes<8>(csr); break;
             case 16: code = BC_LANE16; bytes = lane_bytes<16>(csr); break;
             case 32: code = BC_LANE32; bytes = lane_bytes<32>(csr); break;
-            default: code = BC_LANE64; bytes = 0; break;
+            default: code = BC_LANE64; bytes = 0; held = false; break;
             }
         } else if (b.kind == LPA_BIN_WAVE || b.kind == LPA_BIN_BLOCK) {
             const int ng = b.kind == LPA_BIN_BLOCK ? 1 : step_groups(logT, a.K, quarter_max);
             wg = (count + ng - 1) / ng;
             code = group_code(ng);
-            bytes = step_lds(ng, logT, csr, a.K) +
-                    static_bytes(ng == 1 ? sizeof(GroupStatic<BLOCK, 8>) : ng == 4 ? sizeof(GroupStatic<64, 8>)
-                                 : ng == 8 ? sizeof(GroupStatic<32, 8>) : ng == 16 ? sizeof(GroupStatic<16, 8>)
-                                                                                   : sizeof(GroupStatic<8, 8>));
+            bytes = merged_lds(ng, logT, csr, a.K);
+            held = merged(ng, logT, a.K);
         } else {
             continue;
         }
         // the XCD mapping is per launch, and the recorder times whole bins
-        if (wg > MERGE_BLOCKS || code == BC_LANE64 || a.xcds > 1 || a.rec) {
+        if (wg > MERGE_BLOCKS || !held || a.xcds > 1 || a.rec) {
             launch_bin(b, a, csr, quarter_max, s);
             continue;
         }

@@ -738,8 +738,25 @@ __device__ __forceinline__ void count_staged(const StepArgs &a, const uint32_t *
 // operations are in order; the workgroup's own-label check, which such a list
 // always takes, has barriers between.)  CSR rows need no list.  A fifth less
 // LDS: 40 -> 32 KB per workgroup, 5 instead of 3 on a CU.
-inline __host__ __device__ bool group_list_inside(bool csr, uint32_t K, uint32_t kb, uint32_t cap, uint32_t staged) {
+constexpr __host__ __device__ bool group_list_inside(bool csr, uint32_t K, uint32_t kb, uint32_t cap, uint32_t staged) {
     return csr || (K <= kb && cap <= staged);
+}
+// 64-bit words of a group's table of T slots and its list of T / 2 ids.
+constexpr __host__ __device__ uint32_t group_words(bool inside, uint32_t T) { return inside ? T : T + T / 4; }
+
+// Staged ids per lane (IPL) that a list of cap ids takes in groups of G lanes:
+// the smallest that holds it where the number costs registers (batches of
+// several vectors), else 8.  The host sizes the LDS by it and the kernels are
+// chosen by it, so both must ask here.
+constexpr __host__ __device__ uint32_t staged_ids(uint32_t kb, uint32_t cap, uint32_t G) {
+    const uint32_t ipl = (cap + G - 1) / G;
+    return kb <= 2 ? 8 : ipl <= 2 ? 2 : ipl <= 4 ? 4 : 8;
+}
+// Whether k_bins<kb> has the group kernel for G lanes and `ids` staged ids: not
+// those that only unusual schedules ask for (half waves of 129 to 256 ids, when
+// quarter_max is above 128); such bins take a launch of their own.
+constexpr __host__ __device__ bool bins_hold(uint32_t kb, uint32_t G, uint32_t ids) {
+    return kb <= 2 || (G != 8 && (G != 32 || (kb == 8 && ids == 4)));
 }
 
 template <int G, int KB> struct GroupStatic {
@@ -761,7 +778,7 @@ __device__ __forceinline__ void group_tile(const StepArgs &a, uint32_t logT, uin
     // the list shares the table's memory when it is not read again once the
     // (only) batch's labels are staged, see group_list_inside
     const bool inside = group_list_inside(CSR, a.K, KB, listcap, IPL * G);
-    uint64_t *tab = lds + (uint64_t)gid * (inside ? T : T + T / 4);
+    uint64_t *tab = lds + (uint64_t)gid * group_words(inside, T);
     uint32_t *list = (uint32_t *)(inside ? tab + T / 2 : tab + T);
     GroupShared<G> *sh = &st.gsh[gid];
     const uint32_t stride = tiles * NG;
@@ -860,17 +877,19 @@ struct BinTable {
     uint32_t n;
 };
 
-// Staged ids per lane of a merged bin: those of the separate launch when
-// their number changes the registers (several vectors), else 8.
+// A merged bin of G lanes per vertex.
 template <int G, bool CSR, int KB>
 __device__ __forceinline__ void group_bin(const StepArgs &a, const BinTable::Entry &e, uint32_t tile, uint32_t tiles,
                                           uint64_t *lds) {
     auto &st = *reinterpret_cast<GroupStatic<G, KB> *>(lds);
     uint64_t *dyn = lds + (sizeof(GroupStatic<G, KB>) + 7) / 8;
-    const uint32_t cap = 1u << (e.logT - 1), ipl = (cap + G - 1) / G;
-    if (KB >= 4 && G != 32 && ipl <= 2) group_tile<G, CSR, KB, (KB >= 4 ? 2 : 8)>(a, e.logT, cap, tile, tiles, dyn, st);
-    else if (KB >= 4 && (G == 32 || ipl <= 4)) group_tile<G, CSR, KB, (KB >= 4 ? 4 : 8)>(a, e.logT, cap, tile, tiles, dyn, st);
-    else group_tile<G, CSR, KB, 8>(a, e.logT, cap, tile, tiles, dyn, st);
+    const uint32_t cap = 1u << (e.logT - 1), ids = staged_ids(KB, cap, G);
+    if constexpr (KB >= 4 && bins_hold(KB, G, 2))
+        if (ids == 2) group_tile<G, CSR, KB, 2>(a, e.logT, cap, tile, tiles, dyn, st);
+    if constexpr (KB >= 4 && bins_hold(KB, G, 4))
+        if (ids == 4) group_tile<G, CSR, KB, 4>(a, e.logT, cap, tile, tiles, dyn, st);
+    if constexpr (bins_hold(KB, G, 8))
+        if (ids == 8) group_tile<G, CSR, KB, 8>(a, e.logT, cap, tile, tiles, dyn, st);
 }
 
 template <int KB, bool CSR>
@@ -881,13 +900,9 @@ __device__ __forceinline__ void one_bin(const StepArgs &a, const BinTable::Entry
     case BC_LANE8: lane_tile<8, CSR>(a, tile, *reinterpret_cast<LaneShared<8, CSR> *>(lds)); break;
     case BC_LANE16: lane_tile<16, CSR>(a, tile, *reinterpret_cast<LaneShared<16, CSR> *>(lds)); break;
     case BC_LANE32: lane_tile<32, CSR>(a, tile, *reinterpret_cast<LaneShared<32, CSR> *>(lds)); break;
-    case BC_G8:
-        if (KB <= 2) group_bin<8, CSR, KB>(a, e, tile, tiles, lds);
-        break;
+    case BC_G8: group_bin<8, CSR, KB>(a, e, tile, tiles, lds); break;
     case BC_G16: group_bin<16, CSR, KB>(a, e, tile, tiles, lds); break;
-    case BC_G32:
-        if (KB != 4) group_bin<32, CSR, KB>(a, e, tile, tiles, lds);
-        break;
+    case BC_G32: group_bin<32, CSR, KB>(a, e, tile, tiles, lds); break;
     case BC_G64: group_bin<64, CSR, KB>(a, e, tile, tiles, lds); break;
     default: group_bin<BLOCK, CSR, KB>(a, e, tile, tiles, lds); break;
     }
