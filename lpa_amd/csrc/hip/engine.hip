@@ -312,7 +312,9 @@ struct lpa_engine {
     // work recorder (lane-cycles per vertex id), null when off
     unsigned long long *rec = nullptr;
 
-    // captured steps: graphs[method][cur]
+    // captured steps: graphs[method][cur], with the addresses and parameters
+    // of every buffer that a step uses: whoever moves or changes one of them
+    // drops the graphs
     bool graph_mode = false;
     hipGraphExec_t graphs[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
     void drop_graphs() {
@@ -1925,6 +1927,9 @@ int lpa_stream_residence(lpa_engine *e, int where, uint64_t batch_bytes) {
         HIPCHK(hipSetDevice(e->device));
         e->sync();
         if (e->copy_stream) HIPCHK(hipStreamSynchronize(e->copy_stream));
+        // captured steps read the stream where it is (lpa_time_iterations
+        // captures them with graph mode off, too)
+        e->drop_graphs();
         e->host_stream = host;
         e->batch_bytes = batch_bytes ? batch_bytes : DEFAULT_BATCH_BYTES;
         move_stream(e, e->words0, host);
