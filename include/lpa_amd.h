@@ -48,7 +48,8 @@
  * Conventions: every function returns LPA_OK (0) or a negative status and
  * leaves a message for lpa_last_error() (thread-local).  Device memory is
  * owned by the engine handle.  One host thread per engine; all work is
- * queued on the engine's own stream (default priority).
+ * queued on the engine's own streams (default priority).  A model (lpa_mlp)
+ * may be used by several threads and engines; its calls take turns.
  */
 #ifndef LPA_AMD_H
 #define LPA_AMD_H

@@ -2044,6 +2044,7 @@ int lpa_cglp_csr_get(lpa_engine *e, uint64_t *row, uint32_t *col, uint64_t *m) {
 struct lpa_mlp {
     int device = 0;
     hipStream_t stream = nullptr;
+    std::mutex mu;   // held by every call: several threads (engines) may share a model
     // parameters, first and second moments (MLP_STRIDE floats each), double
     // buffered: a training step reads state[cur] and writes the other one
     DevBuf<float> state[2], part[2], grad;
@@ -2260,6 +2261,7 @@ int lpa_mlp_destroy(lpa_mlp *m) {
 int lpa_mlp_get_params(lpa_mlp *m, float *params) {
     return guard([&] {
         if (!m || !params) throw Fail(LPA_ERR_ARG, "null argument");
+        std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
         HIPCHK(hipMemcpy(params, m->state[m->cur].p, MLP_NPARAM * 4, hipMemcpyDeviceToHost));
     });
@@ -2268,6 +2270,7 @@ int lpa_mlp_get_params(lpa_mlp *m, float *params) {
 int lpa_mlp_set_params(lpa_mlp *m, const float *params) {
     return guard([&] {
         if (!m || !params) throw Fail(LPA_ERR_ARG, "null argument");
+        std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
         float h[3 * MLP_STRIDE] = {};   // zero moments
         std::memcpy(h, params, MLP_NPARAM * 4);
@@ -2280,6 +2283,7 @@ int lpa_mlp_forward(lpa_mlp *m, const float *x, uint64_t n, float *y) {
     return guard([&] {
         if (!m || (n && (!x || !y))) throw Fail(LPA_ERR_ARG, "null argument");
         if (n == 0) return;
+        std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
         DevBuf<float> &dx = m->x, &dy = m->y;
         dx.upload(x, n * MLP_IN, m->stream, m->link);
@@ -2296,6 +2300,7 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
                       float *loss, float *grad) {
     return guard([&] {
         if (!m || !x || !target || !mask || !loss || !grad || n == 0) throw Fail(LPA_ERR_ARG, "bad arguments");
+        std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
         DevBuf<float> &dx = m->x, &dt = m->target;
         DevBuf<uint8_t> &dm = m->mask;
@@ -2318,6 +2323,7 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
     return guard([&] {
         if (!m || !x || !target || !mask || n == 0 || epochs <= 0 || batch <= 0) throw Fail(LPA_ERR_ARG, "bad arguments");
         if (n >= (1ull << 32)) throw Fail(LPA_ERR_RANGE, "too many samples");
+        std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
         DevBuf<float> &dx = m->x, &dt = m->target;
         DevBuf<uint8_t> &dm = m->mask;
