@@ -134,6 +134,12 @@ template <class T> struct DevBuf {
     static constexpr uint64_t KEEP_BYTES = 256ull << 20;
 };
 
+// Trims an object's kept buffers when a call ends, also by an error.
+template <class T> struct TrimAtEnd {
+    T &x;
+    ~TrimAtEnd() { x.trim(); }
+};
+
 // Heavy vertices of one part (compressed or small CSR) and one mode (CMS or
 // exact HBM hash), processed by the chunked kernels of heavy_kernels.hpp.
 struct HeavySet {
@@ -235,6 +241,13 @@ struct lpa_engine {
         DevBuf<uint64_t> row, len, sums;
         DevBuf<uint32_t> col, deg;
         BfsWork bfs;
+        void trim() {
+            row.trim();
+            len.trim();
+            sums.trim();
+            col.trim();
+            deg.trim();
+        }
     } work;
     int num_cu = 0;
     size_t lds_max = 65536;
@@ -755,6 +768,7 @@ template <class F> static void in_launches(uint64_t n, uint64_t per_block, F &&f
 // records.
 static void finish_graph(lpa_engine *e) {
     const uint64_t n_c = e->n_c;
+    TrimAtEnd<lpa_engine::Work> trim{e->work};
     DevBuf<uint32_t> &ddeg = e->work.deg;
     ddeg.alloc(n_c);
     e->feat0.alloc(n_c * NFEAT);
@@ -770,7 +784,6 @@ static void finish_graph(lpa_engine *e) {
     HIPCHK(hipMemcpyAsync(&bad, e->err.p, sizeof bad, hipMemcpyDeviceToHost, e->stream));
     e->deg_c.resize(n_c);
     e->link.out(e->deg_c.data(), ddeg.p, n_c * 4, e->stream);
-    ddeg.trim();
     if (bad) throw Fail(LPA_ERR_FORMAT, "malformed CGR record at stream position " + std::to_string(bad - 1));
     e->m_c = 0;
     for (uint32_t d : e->deg_c) e->m_c += d;
@@ -1008,6 +1021,7 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         e->n_s = n_s;
         e->m_s = m_s;
         // encode on the device
+        TrimAtEnd<lpa_engine::Work> trim{e->work};
         DevBuf<uint64_t> &drow = e->work.row, &len = e->work.len;
         DevBuf<uint32_t> &dcol = e->work.col;
         drow.upload(row, n + 1, e->stream, e->link);
@@ -1096,9 +1110,6 @@ int lpa_graph_encode_csr(lpa_engine *e, uint64_t n, const uint64_t *row, const u
         HIPCHK(hipGetLastError());
         if (e->host_stream) move_stream(e, e->words0, true);
         finish_graph(e);
-        drow.trim();
-        dcol.trim();
-        len.trim();
     });
 }
 
@@ -2285,6 +2296,7 @@ int lpa_mlp_forward(lpa_mlp *m, const float *x, uint64_t n, float *y) {
         if (n == 0) return;
         std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
+        TrimAtEnd<lpa_mlp> trim{*m};
         DevBuf<float> &dx = m->x, &dy = m->y;
         dx.upload(x, n * MLP_IN, m->stream, m->link);
         dy.alloc(n * MLP_OUT);
@@ -2292,7 +2304,6 @@ int lpa_mlp_forward(lpa_mlp *m, const float *x, uint64_t n, float *y) {
                            m->state[m->cur].p, dx.p, dy.p, n);
         HIPCHK(hipGetLastError());
         m->link.out(y, dy.p, n * MLP_OUT * 4, m->stream);
-        m->trim();
     });
 }
 
@@ -2302,6 +2313,7 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
         if (!m || !x || !target || !mask || !loss || !grad || n == 0) throw Fail(LPA_ERR_ARG, "bad arguments");
         std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
+        TrimAtEnd<lpa_mlp> trim{*m};
         DevBuf<float> &dx = m->x, &dt = m->target;
         DevBuf<uint8_t> &dm = m->mask;
         dx.upload(x, n * MLP_IN, m->stream, m->link);
@@ -2314,7 +2326,6 @@ int lpa_mlp_loss_grad(lpa_mlp *m, const float *x, const float *target, const uin
         HIPCHK(hipMemcpyAsync(grad, m->grad.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipMemcpyAsync(loss, m->grad.p + MLP_NPARAM, 4, hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));
-        m->trim();
     });
 }
 
@@ -2325,6 +2336,7 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
         if (n >= (1ull << 32)) throw Fail(LPA_ERR_RANGE, "too many samples");
         std::lock_guard<std::mutex> lk(m->mu);
         HIPCHK(hipSetDevice(m->device));
+        TrimAtEnd<lpa_mlp> trim{*m};
         DevBuf<float> &dx = m->x, &dt = m->target;
         DevBuf<uint8_t> &dm = m->mask;
         DevBuf<uint32_t> &didx = m->idx;
@@ -2372,7 +2384,6 @@ int lpa_mlp_train(lpa_mlp *m, const float *x, const float *target, const uint8_t
         HIPCHK(hipStreamSynchronize(m->stream));
         if (loss_per_epoch)
             for (int ep = 0; ep < epochs; ep++) loss_per_epoch[ep] = (float)(l[ep] / (double)nb);
-        m->trim();
     });
 }
 
