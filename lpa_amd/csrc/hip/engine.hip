@@ -1194,7 +1194,7 @@ int lpa_graph_stream(lpa_engine *e, uint64_t *n_c, uint64_t *nbits, uint64_t *wo
         *n_c = e->n_c;
         *nbits = e->nbits;
         const uint64_t wbytes = (e->nbits + 63) / 64 * 8;
-        if (words && wbytes && e->words0.host) std::memcpy(words, e->words0.p, wbytes);
+        if (words && wbytes && e->words0.host) HIPCHK(hipMemcpyAsync(words, e->words0.p, wbytes, hipMemcpyDefault, e->stream));
         else if (words) e->link.out(words, e->words0.p, wbytes, e->stream);
         if (offsets) std::memcpy(offsets, e->h_offs.data(), (e->n_c + 1) * 8);
         if (vertices) std::memcpy(vertices, e->h_vertices.data(), e->n * 4);

@@ -25,7 +25,10 @@ struct HostLinkError : std::runtime_error {
 // One per engine or model, used by one host thread at a time.  The slots (16
 // MiB of pinned memory) cost about 2 ms to make, so the copies go to the
 // runtime until WORTH bytes have been copied, and where the slots cannot be
-// had; they are freed with the object.
+// had; they are freed with the object.  The caller's side may be any memory that
+// hipMemcpy takes: only ordinary pages go through the slots, since pinned
+// memory is copied at the link's rate by the runtime and device memory is not
+// a thread's to touch.
 // 134 MB of labels to new host pages: 12.8 -> 3.6 ms; 33 MB of samples in and 13
 // MB of results out: 2.3 -> 1.6 ms.
 class HostLink {
@@ -48,8 +51,8 @@ class HostLink {
     // Queues the copy on stream s; src stays as it is until the stream has
     // been waited for.
     void in(void *dst, const void *src, size_t n, hipStream_t s) {
-        if (n < MIN_IN || !worth(n)) {
-            if (n) check(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s));
+        if (n < MIN_IN || !ordinary(src) || !worth(n)) {
+            if (n) check(hipMemcpyAsync(dst, src, n, hipMemcpyDefault, s));
             return;
         }
         run(n, [&](int slot, size_t at, size_t len) {
@@ -64,8 +67,8 @@ class HostLink {
     // Copies after the work queued on stream s; done on return.  Every piece
     // goes through put(dst, src, bytes) (a memcpy by default).
     template <class Put> void out(void *dst, const void *src, size_t n, hipStream_t s, Put &&put) {
-        if (n < MIN_OUT || !worth(n)) {
-            if (n) check(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s));
+        if (n < MIN_OUT || !ordinary(dst) || !worth(n)) {
+            if (n) check(hipMemcpyAsync(dst, src, n, hipMemcpyDefault, s));
             check(hipStreamSynchronize(s));
             if (n) put(dst, dst, n);
             return;
@@ -91,6 +94,13 @@ class HostLink {
     hipEvent_t ev_[SLOTS] = {};
     size_t copied_ = 0;
 
+    // pages that the runtime knows nothing of
+    static bool ordinary(const void *p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return true;
+    }
     bool worth(size_t n) {
         copied_ = copied_ + n < copied_ ? copied_ : copied_ + n;
         return copied_ >= WORTH && prepare();
