@@ -26,7 +26,7 @@ QUARTER = [0, 1, 16, 32, 33, 63, 64, 65, 100, 127, 128, 129, 200, 255, 256, 257,
 def test_lds_given_holds_lds_addressed(bc, K):
     out = np.zeros(7, np.uint64)
     merged = 0
-    for block, logts in ((0, range(6, 11)), (1, range(8, 14))):
+    for block, logts in ((0, range(6, 12)), (1, range(8, 14))):
         for q in QUARTER:
             for logt in logts:
                 for csr in (0, 1):
