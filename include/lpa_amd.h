@@ -260,8 +260,10 @@ int lpa_schedule_learned_judged(lpa_engine *e, lpa_mlp *m, int iters, float *lea
                                 int *kept_learned);
 
 /* Runs iters steps (method 0 = NOVA fused, 1 = CGLP, 2 = uncompressed CSR) and reports the
- * HIP-event time of each (ms) and the changed counts; captures the step in
- * a HIP graph when use_graph != 0. */
+ * HIP-event time of each (ms), as the iterate entry points run it, and the
+ * changed counts; captures the step in a HIP graph when use_graph != 0.  Eager
+ * fused steps are run a second time from the same labels, a launch per bin, for
+ * lpa_last_kernel_times. */
 int lpa_time_iterations(lpa_engine *e, int method, int iters, int use_graph,
                         float *ms, uint64_t *changed);
 /* Replays steps from HIP graphs captured once per label-buffer parity
@@ -298,7 +300,8 @@ int lpa_stream_batches(lpa_engine *e, uint64_t *nbatches, uint64_t *stage_bytes)
  * after every candidate, so tuning never changes results. */
 int lpa_autotune(lpa_engine *e, int iters, lpa_sched_params *best, float *best_ms);
 /* Average time (ms) per step of each kernel family in the last eager timed
- * run (HIP events on the engine stream). */
+ * run, each launch by itself on one stream (HIP events): a step that shares
+ * launches and streams takes less than their sum. */
 int lpa_last_kernel_times(lpa_engine *e, float *ms_per_kind /* LPA_NBIN_KINDS */);
 /* Measurement helper, no counterpart in the reference: copies `bytes`
  * (a multiple of 16) between two fresh device buffers `reps` times with a

@@ -2492,7 +2492,8 @@ int lpa_time_iterations(lpa_engine *e, int method, int iters, int use_graph, flo
     return guard([&] {
         require_ready(e);
         if (iters <= 0 || !ms) throw Fail(LPA_ERR_ARG, "bad arguments");
-        hipEvent_t ev[2] = {nullptr, nullptr};
+        // a step's start, and its end on each stream that it uses
+        hipEvent_t ev[1 + lpa_engine::LANES] = {};
         // per launch (bins, then heavy sets): a family's time is the sum of
         // its launches, wherever they fall in the step
         const size_t nb = e->bins.size(), nl = nb + e->heavy.size();
@@ -2525,17 +2526,27 @@ int lpa_time_iterations(lpa_engine *e, int method, int iters, int use_graph, flo
             }
             e->graph_mode = use_graph != 0;
             for (int it = 0; it < iters; it++) {
-                e->begin_step(false);
+                // the step as the iterate entry points run it: small bins
+                // merged, heavy sets on the side streams
+                e->begin_step(!e->graph_mode && e->spread_step(method));
+                const int lanes = e->spread ? e->side_lanes() : 1;
                 HIPCHK(hipEventRecord(ev[0], e->stream));
-                if (e->graph_mode) enqueue_step(e, method);
-                else if (method == 0) e->step(false, kev.data());
-                else method_step(e, method);
-                HIPCHK(hipEventRecord(ev[1], e->stream));
+                enqueue_step(e, method);
+                for (int l = 0; l < lanes; l++) HIPCHK(hipEventRecord(ev[1 + l], e->lane_stream(l)));
                 const uint64_t sum = e->end_step();
-                HIPCHK(hipEventElapsedTime(&ms[it], ev[0], ev[1]));
+                ms[it] = 0;
+                for (int l = 0; l < lanes; l++) {
+                    float t = 0;
+                    HIPCHK(hipEventElapsedTime(&t, ev[0], ev[1 + l]));
+                    ms[it] = std::max(ms[it], t);
+                }
                 if (changed) changed[it] = sum;
-                e->cur ^= 1;
                 if (method == 0 && !e->graph_mode && !e->host_stream) {
+                    // once more from the same labels (to the same result),
+                    // a launch per bin on one stream: the families' times
+                    e->begin_step(false);
+                    e->step(false, kev.data());
+                    (void)e->end_step();
                     for (size_t l = 0; l < nl; l++) {
                         if (kind_of_launch[l] < 0) continue;
                         float t = 0;
@@ -2543,8 +2554,11 @@ int lpa_time_iterations(lpa_engine *e, int method, int iters, int use_graph, flo
                         kind_sum[kind_of_launch[l]] += t;
                     }
                 }
+                e->cur ^= 1;
             }
         } catch (...) {
+            for (int l = 0; l < lpa_engine::LANES; l++) (void)hipStreamSynchronize(e->lane_stream(l));
+            e->spread = false;
             e->graph_mode = had_graph_mode;
             destroy();
             throw;
