@@ -3,15 +3,19 @@
 The benchmark's profiled command (bench.py --headline-only ...) builds the
 graph, lays it out (with --no-learned the degree schedule; otherwise the
 judged learned schedule), the last k_relayout dispatch, and then runs
-warmup + steps iterations.
-Everything dispatched after that last relayout belongs to those iterations,
-except the copy kernel of the calibration (bench.py --copy-calibration:
-k_calibration_copy over 256 MiB), whose FETCH_SIZE / WRITE_SIZE readings
-give the factor between the counters and bytes actually moved.
+warm-up and timed iterations, eager at the end.  A step ends with one
+k_publish per stream that it used.  A timed iteration is two steps: the step as
+it runs, with small bins merged (k_bins) and heavy sets on other streams, and
+the same step with a launch per bin on one stream.  The kernel table is of the
+first kind, times and traffic per family are of the second, whose launches
+belong to one family each.
+The copy kernel of the calibration (bench.py --copy-calibration:
+k_calibration_copy over 256 MiB) gives the factor between FETCH_SIZE /
+WRITE_SIZE readings and bytes actually moved.
 
 Usage:
   python -m lpa_amd.rocprof_summary --trace DIR [--fetch DIR --write DIR]
-      --iters N --steps S [--pmc-iters N --pmc-steps S] --command "..."
+      --steps S [--pmc-steps S] --command "..."
       --workload W --K K --out PREFIX
 writes PREFIX_kernels.txt and PREFIX_traffic.json.
 """
@@ -42,10 +46,12 @@ def family(name):
         return "global" if args and args[0] == "0" else "cms"
     if k == "k_calibration_copy":
         return "copy"
-    if k in ("k_fill_u64",):
-        return "step"
-    if k.startswith("k_decode_csr"):
+    if k == "k_bins":
+        return "bins"
+    if k == "k_decode_bins":
         return "cglp-decode"
+    if k == "k_publish":
+        return "step"
     return "other"
 
 
@@ -54,49 +60,55 @@ def _rows(path):
         return list(csv.DictReader(f))
 
 
-def _headline(rows, iters, steps):
-    """step-kernel rows of the last `steps` of the `iters` iterations that
-    follow the last k_relayout dispatch (every iteration dispatches the same
-    kernel sequence), plus the calibration copies"""
+def _headline(rows, steps):
+    """(rows of the steps as run, rows of the steps launched bin by bin) of the
+    last `steps` timed iterations, and the calibration copies"""
     rows = sorted(rows, key=lambda r: int(r["Dispatch_Id"]))
     last = max((i for i, r in enumerate(rows) if "k_relayout" in r["Kernel_Name"]), default=-1)
     rows = rows[last + 1:]
-    step = [r for r in rows if family(r["Kernel_Name"]) not in ("copy", "other")]
-    if len(step) % iters:
-        raise SystemExit(f"{len(step)} step dispatches do not split into {iters} iterations")
-    per = len(step) // iters
-    keep = step[(iters - steps) * per:]
-    return keep + [r for r in rows if family(r["Kernel_Name"]) == "copy"]
-
-
-def trace_summary(trace_dir, iters, steps):
-    rows = _headline(_rows(os.path.join(trace_dir, "run_kernel_trace.csv")), iters, steps)
-    per = collections.defaultdict(lambda: [0, 0.0])
+    copies = [r for r in rows if family(r["Kernel_Name"]) == "copy"]
+    done, ended = [[]], False
     for r in rows:
-        d = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3   # us
+        f = family(r["Kernel_Name"])
+        if f in ("copy", "other"):
+            continue
+        if ended and f != "step":
+            done.append([])
+        done[-1].append(r)
+        ended = f == "step"
+    if not ended:
+        done.pop()   # cut off within a step
+    if len(done) < 2 * steps:
+        raise SystemExit(f"{len(done)} steps after the last layout: {steps} timed iterations make {2 * steps}")
+    done = done[-2 * steps:]
+    run, alone = sum(done[::2], []), sum(done[1::2], [])
+    if any(family(r["Kernel_Name"]) == "bins" for r in alone):
+        raise SystemExit("merged bins in a step that launches them one by one: the last steps are not timed eager ones")
+    return run, alone, copies
+
+
+def trace_summary(trace_dir, steps):
+    run, alone, _ = _headline(_rows(os.path.join(trace_dir, "run_kernel_trace.csv")), steps)
+    us = lambda r: (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
+    per = collections.defaultdict(lambda: [0, 0.0])
+    for r in run:
         k = r["Kernel_Name"]
         per[k][0] += 1
-        per[k][1] += d
+        per[k][1] += us(r)
     fam = collections.defaultdict(float)
-    for k, (c, t) in per.items():
-        if family(k) != "copy":
-            fam[family(k)] += t / steps / 1e3   # ms per iteration
+    for r in alone:
+        fam[family(r["Kernel_Name"])] += us(r) / steps / 1e3   # ms per iteration
     return per, fam
 
 
-def counter_summary(dirname, counter, iters, steps):
+def counter_summary(dirname, counter, steps):
     rows = [r for r in _rows(os.path.join(dirname, "run_counter_collection.csv")) if r["Counter_Name"] == counter]
-    rows = _headline(rows, iters, steps)
+    _, alone, copies = _headline(rows, steps)
+    value = lambda r: float(r["Counter_Value"]) * 1024.0   # KiB -> bytes
     fam = collections.defaultdict(float)
-    copy = []
-    for r in rows:
-        f = family(r["Kernel_Name"])
-        v = float(r["Counter_Value"]) * 1024.0   # KiB -> bytes
-        if f == "copy":
-            copy.append(v)
-        else:
-            fam[f] += v / steps
-    return fam, copy
+    for r in alone:
+        fam[family(r["Kernel_Name"])] += value(r) / steps
+    return fam, [value(r) for r in copies]
 
 
 def main():
@@ -104,7 +116,7 @@ def main():
     ap.add_argument("--trace", required=True)
     ap.add_argument("--fetch")
     ap.add_argument("--write")
-    ap.add_argument("--iters", type=int, required=True, help="warmup + timed iterations of the trace run")
+    ap.add_argument("--iters", type=int, help="warmup + timed iterations of the trace run (named in the summary)")
     ap.add_argument("--steps", type=int, required=True, help="timed iterations of the trace run (summarised)")
     ap.add_argument("--pmc-iters", type=int, help="warmup + timed iterations of the counter runs")
     ap.add_argument("--pmc-steps", type=int, help="timed iterations of the counter runs")
@@ -113,22 +125,22 @@ def main():
     ap.add_argument("--K", type=int, required=True)
     ap.add_argument("--out", required=True)
     a = ap.parse_args()
-    per, fam = trace_summary(a.trace, a.iters, a.steps)
+    per, fam = trace_summary(a.trace, a.steps)
     lines = [f"rocprofv3 kernel trace, headline phase of {a.workload} K={a.K}: the {a.steps} timed iterations "
-             f"(of {a.iters}) after the last layout build", "commands:"]
+             f"{f'(of {a.iters}) ' if a.iters else ''}after the last layout build", "commands:"]
     lines += [f"  {c.strip()}" for c in a.command.split(";") if c.strip()]
     lines.append("")
     lines.append(f"{'kernel':78s} {'calls':>6s} {'avg_us':>9s} {'us/iter':>9s} family")
     for k, (c, t) in sorted(per.items(), key=lambda x: -x[1][1]):
         lines.append(f"{k[:78]:78s} {c:6d} {t / c:9.1f} {t / a.steps:9.1f} {family(k)}")
     lines.append("")
-    lines.append("per family (ms per iteration): " +
+    lines.append("per family, a launch per bin on one stream (ms per iteration): " +
                  ", ".join(f"{f} {v:.3f}" for f, v in sorted(fam.items(), key=lambda x: -x[1])))
     out = {"workload": a.workload, "K": a.K, "steps": a.steps, "ms_per_iter": dict(fam)}
     if a.fetch and a.write:
-        pi, ps = a.pmc_iters or a.iters, a.pmc_steps or a.steps
-        fetch, cf = counter_summary(a.fetch, "FETCH_SIZE", pi, ps)
-        write, cw = counter_summary(a.write, "WRITE_SIZE", pi, ps)
+        ps = a.pmc_steps or a.steps
+        fetch, cf = counter_summary(a.fetch, "FETCH_SIZE", ps)
+        write, cw = counter_summary(a.write, "WRITE_SIZE", ps)
         ff = COPY_BYTES / (sum(cf) / len(cf)) if cf else 1.0
         fw = COPY_BYTES / (sum(cw) / len(cw)) if cw else 1.0
         lines.append("")
