@@ -16,7 +16,6 @@ struct Bin {
     int param;         // LANE: network size N; WAVE/BLOCK: log2 table slots
     bool csr;          // small-vertex CSR part
     uint32_t begin, end;
-    uint32_t maxdeg;
 };
 
 // LDS bytes of the WAVE / BLOCK kernels' per-group table (2^logT slots) and

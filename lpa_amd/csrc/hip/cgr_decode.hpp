@@ -223,35 +223,6 @@ LPA_HD __forceinline__ void read_residual_segment(R &r, uint32_t v, F &&emit) {
     read_residual_ids(r, v, c, emit);
 }
 
-// Interval segment at bit q; returns the bit just after it.
-template <class F>
-LPA_HD __forceinline__ uint64_t decode_interval_segment(const uint64_t *__restrict__ W, uint64_t q,
-                                                            uint32_t v, F &&emit_run) {
-    BitReader r;
-    r.seek(W, q);
-    read_interval_segment(r, v, emit_run);
-    return r.pos;
-}
-
-// Residual segment at bit q; returns the bit just after it.
-template <class F>
-LPA_HD __forceinline__ uint64_t decode_residual_segment(const uint64_t *__restrict__ W, uint64_t q,
-                                                            uint32_t v, F &&emit) {
-    BitReader r;
-    r.seek(W, q);
-    read_residual_segment(r, v, emit);
-    return r.pos;
-}
-
-// Segment-count header of a block at bit p: returns #segments, *base = first segment.
-LPA_HD __forceinline__ uint32_t block_header(const uint64_t *__restrict__ W, uint64_t p, uint64_t *base) {
-    BitReader r;
-    r.seek(W, p);
-    uint32_t s = r.gamma() + 1;
-    *base = r.pos;
-    return s;
-}
-
 // Serial decode of a whole staged record (the reader stands at its start):
 // emit(u) per neighbour, in encoded order.
 template <class R, class F>

@@ -1584,7 +1584,7 @@ static void build_layout(lpa_engine *e, const std::vector<uint8_t> &kind_c, cons
             uint64_t r = q;
             const uint32_t x = order[q];
             while (r < cnt && kinds[order[r]] == kinds[x] && sub[order[r]] == sub[x]) r++;
-            Bin b{kinds[x], sub[x], csr, (uint32_t)q, (uint32_t)r, deg(x)};
+            Bin b{kinds[x], sub[x], csr, (uint32_t)q, (uint32_t)r};
             e->bins.push_back(b);
             e->bin_counts[b.kind] += r - q;
             q = r;

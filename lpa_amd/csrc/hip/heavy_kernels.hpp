@@ -161,7 +161,8 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_task_count(StepArgs a, DecodeTa
 // One workgroup per task: the words of its segments (one range of interval
 // segments, one of residual segments) are staged in LDS, then each lane
 // decodes its segment, claiming output slots with one LDS atomic per run
-// (runs of LONG_RUN or more ids are written by the whole workgroup) or per
+// (runs of LONG_RUN or more ids are written by 16 lanes together, HUGE_RUN or
+// more by the whole workgroup) or per
 // residual segment; the task's ids are assembled in LDS and stored to the list
 // with coalesced stores, or written in place when they exceed the staging
 // buffer.  With crow the ids go to the heavy vertex's row of the decoded CSR

@@ -516,8 +516,8 @@ __device__ __forceinline__ void put_run(Sh *sh, uint32_t *list, uint32_t o, uint
 // the residual block, which starts where the last interval segment ends.
 // Each run claims its slots with one LDS atomic, each residual segment with
 // one atomic for its whole count; runs of LONG_RUN or more ids are written by
-// all lanes together so a hub whose neighbours form one long run is not
-// written by a single lane.  Returns the degree (valid in every lane of the
+// 16 lanes together and huge ones by all of them, so that a hub whose neighbours
+// form one long run is not written by a single lane.  Returns the degree (valid in every lane of the
 // group).
 template <int G>
 __device__ __forceinline__ uint32_t group_decode(const StepArgs &a, uint32_t p, uint32_t v, uint32_t gl,
