@@ -30,7 +30,8 @@ struct HostLinkError : std::runtime_error {
 // memory is copied at the link's rate by the runtime and device memory is not
 // a thread's to touch.
 // 134 MB of labels to new host pages: 12.8 -> 3.6 ms; 33 MB of samples in and 13
-// MB of results out: 2.3 -> 1.6 ms.
+// MB of results out: 2.3 -> 1.6 ms (from the second such call of a model on; the
+// first takes 2.5 ms either way).
 class HostLink {
   public:
     static constexpr size_t CHUNK = 2u << 20;
